@@ -74,11 +74,11 @@ def _log(rng, lo, hi):
 
 
 def draw(rng):
-    """A case of the listed ones' ranges; rows, tokens, layers or the vocabulary are
+    """A case of the listed ones' ranges; rows, tokens, layers or widths are
     halved until it costs no more than the largest of them."""
     c = _draw(rng)
     while work(c)["flops"] > 4.9e11 or work(c)["bytes"] > 1.1e9:
-        k = next(k for k in ("M", "T", "layers", "vocab") if c.get(k, 1) > 1)
+        k = next(k for k in ("M", "T", "layers", "vocab", "N") if c.get(k, 1) > 1)
         c[k] //= 2
     return c
 
