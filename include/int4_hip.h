@@ -223,6 +223,29 @@ int w4a16_gemm_noalloc(const void* x, int x_dtype, int64_t M, int64_t N, int64_t
                        const int32_t* qweight, const uint16_t* scales, const uint16_t* zeros,
                        int group_size, void* y, int64_t ldy, void* stream);
 
+/*
+ * Attention of one decode step of a Llama-style layer, in one launch: rotary
+ * embedding of q and k (cos, sin: the position's rows [head_dim / 2]; fp32
+ * products rounded separately), the new key and value written to the fp32
+ * caches k_cache [kv_heads, head_dim, max_len] and v_cache [kv_heads, max_len,
+ * head_dim] at position *pos (device memory), and softmax(q K / sqrt(head_dim))
+ * V over positions 0..*pos in fp32, rounded once into out [num_heads *
+ * head_dim].  q [num_heads * head_dim], k and v [num_kv_heads * head_dim] of
+ * dtype bf16 / fp16, dense.  head_dim 64 or 128; num_heads a multiple of
+ * num_kv_heads.  A *pos outside [0, max_len) leaves caches and out untouched.
+ * workspace: as for w4a16_gemm (256-byte aligned, counter area zero),
+ * w4_attention_decode_workspace_bytes long (0: not a supported shape).
+ * No counterpart in the reference, whose model is Hugging Face's
+ * (benchmarks/eval_llama.py:206-211): it is the attention of the harness model
+ * in int4_hip/llama.py.
+ */
+size_t w4_attention_decode_workspace_bytes(int64_t num_heads, int64_t num_kv_heads, int64_t head_dim,
+                                           int64_t max_len);
+int w4_attention_decode(const void* q, const void* k, const void* v, int dtype, int64_t num_heads,
+                        int64_t num_kv_heads, int64_t head_dim, const float* cos, const float* sin,
+                        float* k_cache, float* v_cache, int64_t max_len, const int64_t* pos, void* out,
+                        void* workspace, size_t workspace_bytes, void* stream);
+
 #ifdef __cplusplus
 }
 #endif

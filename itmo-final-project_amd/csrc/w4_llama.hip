@@ -1,0 +1,365 @@
+// Kernels of a Llama-style decoder layer between its W4A16 linears
+// (int4_hip/llama.py): the attention of one decode step.
+//
+// One token's attention is a handful of tiny operations (rotary embedding of
+// q and k, two cache writes, q.K, softmax, p.V), so as separate launches it is
+// bound by launch latency; here it is one launch.
+#include <hip/hip_runtime.h>
+
+#include "w4_common.hpp"
+
+namespace w4 {
+
+constexpr int kAttnThreads = 256;
+constexpr int kAttnWaves = kAttnThreads / 64;
+constexpr int kAttnMaxChunks = 64;  // position chunks per key-value head
+constexpr int kAttnHeads = 4;       // query heads per workgroup
+constexpr float kLog2e = 1.4426950408889634f;
+
+struct AttnDecodeArgs {
+  const uint16_t* q;  // [nh * D]
+  const uint16_t* k;  // [nkv * D]
+  const uint16_t* v;  // [nkv * D]
+  const float* cos;   // [D / 2], the row of the position
+  const float* sin;
+  float* kc;          // [nkv, D, max_len]
+  float* vc;          // [nkv, max_len, D]
+  const int64_t* pos;
+  uint16_t* out;      // [nh * D]
+  unsigned* cnt;      // one arrival counter per key-value head and head slice
+  float* part;        // [nkv, slices, chunks, kAttnHeads * (D + 2)]
+  float qscale;       // softmax scale * log2(e)
+  int g, max_len, chunk, chunks;
+};
+
+// Rotates the pair (x1, x2) = (x[d], x[d + D/2]); products and sums rounded
+// separately, as the torch-op version does.
+__device__ __forceinline__ void rope_pair(float x1, float x2, float c, float s, float* r1, float* r2) {
+#pragma clang fp contract(off)
+  *r1 = x1 * c - x2 * s;
+  *r2 = x2 * c + x1 * s;
+}
+
+__device__ __forceinline__ float wave_max(float v) {
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) v = fmaxf(v, __shfl_xor(v, o, 64));
+  return v;
+}
+__device__ __forceinline__ float wave_sum(float v) {
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
+  return v;
+}
+
+// One workgroup = one key-value head x one chunk of cache positions (a
+// multiple of 64) x up to four of its query heads (eight would need 256
+// registers), fp32 throughout.
+//
+// What bounds it: the latency of one trip to memory (at 576 positions a head's
+// keys and values are 288 KB).  So positions are cut into chunks over
+// workgroups (9 x 8 heads there), each lane issues its D/4 key loads (lane =
+// position, the cache keeps K transposed, so a wave reads 256 contiguous
+// bytes) and its value loads before the first use, and the chunks of a head
+// meet without a second launch: each publishes (max, sum, unnormalised
+// output), and the last to arrive joins them in chunk order (same bits every
+// run).  The chunk that holds the position writes the new key and value to
+// the cache and uses them from LDS.  A decode step of the 1B model (16 layers,
+// position 575, fp16): 1559 us with the torch operations, 848 us with this.
+template <int DT, int D, int GP>
+__global__ __launch_bounds__(kAttnThreads) void attn_decode_kernel(AttnDecodeArgs a) {
+  constexpr int DW = D / kAttnWaves;   // head elements per wave (keys)
+  constexpr int PW = 64 / kAttnWaves;  // positions per wave (values)
+  constexpr int VE = D / 64;           // value elements per lane
+  constexpr int HW = (GP + kAttnWaves - 1) / kAttnWaves;
+  __shared__ __attribute__((aligned(16))) float q_s[GP][D];
+  __shared__ __attribute__((aligned(16))) float k_s[D];
+  __shared__ __attribute__((aligned(16))) float v_s[D];
+  __shared__ __attribute__((aligned(16))) float p_s[GP][64];
+  __shared__ float alpha_s[GP];
+  __shared__ float m_s[GP], l_s[GP];
+  // cross-wave sums: scores [wave][head][position], then outputs [wave][head][d]
+  __shared__ __attribute__((aligned(16))) float red[kAttnWaves][GP][D];
+  __shared__ float w_s[kAttnMaxChunks][GP];
+  __shared__ unsigned arrived;
+
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int c = blockIdx.x, kvh = blockIdx.y, z = blockIdx.z;
+  const int h0 = kvh * a.g + z * kAttnHeads;  // first query head
+  const int g = min(a.g - z * kAttnHeads, GP);
+  const int64_t pos64 = *a.pos;
+  if (pos64 < 0 || pos64 >= a.max_len) return;  // the caller's table lookup refuses such a position
+  const int pos = (int)pos64;
+  const int active = pos / a.chunk + 1;
+  if (c >= active) return;
+  const int c0 = c * a.chunk;
+  const int c1 = min(c0 + a.chunk, pos + 1);
+  const float* __restrict__ kc = a.kc + (int64_t)kvh * D * a.max_len;
+  const float* __restrict__ vc = a.vc + (int64_t)kvh * a.max_len * D;
+
+  for (int i = tid; i < GP * (D / 2); i += kAttnThreads) {
+    const int h = i / (D / 2), d = i % (D / 2);
+    float r1 = 0.f, r2 = 0.f;
+    if (h < g) {
+      const uint16_t* q = a.q + (int64_t)(h0 + h) * D;
+      rope_pair(act_bits_to_float(q[d], DT), act_bits_to_float(q[d + D / 2], DT), a.cos[d], a.sin[d], &r1, &r2);
+    }
+    q_s[h][d] = r1 * a.qscale;
+    q_s[h][d + D / 2] = r2 * a.qscale;
+  }
+  if (c == active - 1) {
+    if (tid < D / 2) {
+      const uint16_t* k = a.k + (int64_t)kvh * D;
+      float r1, r2;
+      rope_pair(act_bits_to_float(k[tid], DT), act_bits_to_float(k[tid + D / 2], DT), a.cos[tid], a.sin[tid], &r1,
+                &r2);
+      k_s[tid] = r1;
+      k_s[tid + D / 2] = r2;
+      if (z == 0) {
+        a.kc[((int64_t)kvh * D + tid) * a.max_len + pos] = r1;
+        a.kc[((int64_t)kvh * D + tid + D / 2) * a.max_len + pos] = r2;
+      }
+    } else if (tid >= 128 && tid < 128 + D) {
+      const float v = act_bits_to_float(a.v[(int64_t)kvh * D + tid - 128], DT);
+      v_s[tid - 128] = v;
+      if (z == 0) a.vc[((int64_t)kvh * a.max_len + pos) * D + tid - 128] = v;
+    }
+  }
+  __syncthreads();
+
+  float m[HW], l[HW];
+#pragma unroll
+  for (int j = 0; j < HW; ++j) m[j] = -__builtin_inff(), l[j] = 0.f;
+  float o[GP][VE];
+#pragma unroll
+  for (int h = 0; h < GP; ++h)
+#pragma unroll
+    for (int e = 0; e < VE; ++e) o[h][e] = 0.f;
+
+  for (int p0 = c0; p0 < c1; p0 += 64) {
+    const int p = p0 + lane, pc = min(p, pos);
+    float kr[DW], vr[PW][VE];
+#pragma unroll
+    for (int i = 0; i < DW; ++i) kr[i] = kc[(int64_t)(wv * DW + i) * a.max_len + pc];
+#pragma unroll
+    for (int i = 0; i < PW; ++i) {
+      const float* vp = vc + (int64_t)min(p0 + wv * PW + i, pos) * D + lane * VE;
+#pragma unroll
+      for (int e = 0; e < VE; ++e) vr[i][e] = vp[e];
+    }
+    float s[GP];
+#pragma unroll
+    for (int h = 0; h < GP; ++h) s[h] = 0.f;
+#pragma unroll
+    for (int i = 0; i < DW; i += 4) {
+      float kk[4];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) kk[e] = p == pos ? k_s[wv * DW + i + e] : kr[i + e];
+#pragma unroll
+      for (int h = 0; h < GP; ++h) {
+        const f32x4 qv = *reinterpret_cast<const f32x4*>(&q_s[h][wv * DW + i]);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) s[h] = __builtin_fmaf(qv[e], kk[e], s[h]);
+      }
+    }
+#pragma unroll
+    for (int h = 0; h < GP; ++h) red[wv][h][lane] = s[h];
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < HW; ++j) {
+      const int h = wv + j * kAttnWaves;
+      if (h < GP) {
+        float t = (red[0][h][lane] + red[1][h][lane]) + (red[2][h][lane] + red[3][h][lane]);
+        if (p > pos) t = -__builtin_inff();
+        const float mn = fmaxf(m[j], wave_max(t));
+        // a chunk of -inf scores has no weight; a NaN score stays NaN
+        const float pe = (mn == -__builtin_inff() && t == t) ? 0.f : __builtin_amdgcn_exp2f(t - mn);
+        const float al = m[j] == mn ? 1.f : __builtin_amdgcn_exp2f(m[j] - mn);
+        l[j] = l[j] * al + wave_sum(pe);
+        m[j] = mn;
+        p_s[h][lane] = pe;
+        if (lane == 0) alpha_s[h] = al;
+      }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int h = 0; h < GP; ++h) {
+      const float al = alpha_s[h];
+#pragma unroll
+      for (int e = 0; e < VE; ++e) o[h][e] *= al;
+#pragma unroll
+      for (int i = 0; i < PW; i += 4) {
+        const f32x4 pv = *reinterpret_cast<const f32x4*>(&p_s[h][wv * PW + i]);
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+#pragma unroll
+          for (int e = 0; e < VE; ++e) {
+            const float vv = p0 + wv * PW + i + u == pos ? v_s[lane * VE + e] : vr[i + u][e];
+            o[h][e] = __builtin_fmaf(pv[u], vv, o[h][e]);
+          }
+      }
+    }
+    // red is next written after every wave has passed the barrier above
+  }
+#pragma unroll
+  for (int j = 0; j < HW; ++j) {
+    const int h = wv + j * kAttnWaves;
+    if (h < GP && lane == 0) m_s[h] = m[j], l_s[h] = l[j];
+  }
+#pragma unroll
+  for (int h = 0; h < GP; ++h)
+#pragma unroll
+    for (int e = 0; e < VE; ++e) red[wv][h][lane * VE + e] = o[h][e];
+  __syncthreads();
+
+  const int n = g * D;
+  constexpr int stride = kAttnHeads * (D + 2);
+  const int64_t slice = (int64_t)kvh * gridDim.z + z;
+  if (active == 1) {
+    for (int i = tid; i < n; i += kAttnThreads) {
+      const int h = i / D, d = i % D;
+      const float t = (red[0][h][d] + red[1][h][d]) + (red[2][h][d] + red[3][h][d]);
+      a.out[(int64_t)h0 * D + i] = float_to_act_bits<DT>(t / l_s[h]);
+    }
+    return;
+  }
+  // publish (device-coherent stores, waited for), then count the arrival
+  float* const mine = a.part + (slice * a.chunks + c) * stride;
+  for (int i = tid; i < n; i += kAttnThreads) {
+    const int h = i / D, d = i % D;
+    const float t = (red[0][h][d] + red[1][h][d]) + (red[2][h][d] + red[3][h][d]);
+    __hip_atomic_store(mine + i, t, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  }
+  if (tid < g) {
+    __hip_atomic_store(mine + n + tid, m_s[tid], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __hip_atomic_store(mine + n + g + tid, l_s[tid], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  }
+  __builtin_amdgcn_s_waitcnt(0);  // the stores have reached the level all XCDs share
+  __syncthreads();
+  if (tid == 0) arrived = __hip_atomic_fetch_add(a.cnt + slice, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  __syncthreads();
+  if (arrived != (unsigned)(active - 1)) return;
+  if (tid == 0) __hip_atomic_store(a.cnt + slice, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  const float* const all = a.part + slice * a.chunks * stride;
+  // lane = chunk (at most 64): its weight relative to the head's maximum
+#pragma unroll
+  for (int j = 0; j < HW; ++j) {
+    const int h = wv + j * kAttnWaves;
+    if (h < g) {
+      float mc = -__builtin_inff(), lc = 0.f;
+      if (lane < active) {
+        mc = __hip_atomic_load(all + lane * stride + n + h, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        lc = __hip_atomic_load(all + lane * stride + n + g + h, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      }
+      const float mx = wave_max(mc);
+      const float w = lane < active ? __builtin_amdgcn_exp2f(mc - mx) : 0.f;
+      const float sum = wave_sum(lane < active ? w * lc : 0.f);
+      if (lane < active) w_s[lane][h] = w;
+      if (lane == 0) l_s[h] = sum;
+    }
+  }
+  __syncthreads();
+  for (int i = tid; i < n; i += kAttnThreads) {
+    const int h = i / D;
+    float t = 0.f;
+    int cc = 0;
+    for (; cc + 8 <= active; cc += 8) {
+      float r[8];
+#pragma unroll
+      for (int u = 0; u < 8; ++u)
+        r[u] = __hip_atomic_load(all + (cc + u) * stride + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+#pragma unroll
+      for (int u = 0; u < 8; ++u) t = __builtin_fmaf(w_s[cc + u][h], r[u], t);
+    }
+    for (; cc < active; ++cc)
+      t = __builtin_fmaf(w_s[cc][h],
+                         __hip_atomic_load(all + cc * stride + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT), t);
+    a.out[(int64_t)h0 * D + i] = float_to_act_bits<DT>(t / l_s[h]);
+  }
+}
+
+}  // namespace w4
+
+using namespace w4host;
+
+namespace {
+
+// Positions per chunk: 64, more for caches past 4096 positions so that a head
+// has at most 64 chunks (its last workgroup reads one lane per chunk).
+int attn_chunk(int64_t max_len) {
+  return 64 * (int)((max_len + 64 * w4::kAttnMaxChunks - 1) / (64 * w4::kAttnMaxChunks));
+}
+
+int64_t attn_slices(int64_t nh, int64_t nkv) { return (nh / nkv + w4::kAttnHeads - 1) / w4::kAttnHeads; }
+
+bool attn_decode_shape_ok(int64_t nh, int64_t nkv, int64_t head_dim, int64_t max_len) {
+  return nkv >= 1 && nh >= nkv && nh % nkv == 0 &&
+         (head_dim == 64 || head_dim == 128) && max_len >= 1 && max_len < (1LL << 24) &&
+         nkv * attn_slices(nh, nkv) <= (int64_t)(W4_WORKSPACE_COUNTER_BYTES / 4);
+}
+
+template <int DT, int D>
+void launch_decode(const w4::AttnDecodeArgs& a, int nkv, hipStream_t st) {
+  const dim3 grid((unsigned)a.chunks, (unsigned)nkv, (unsigned)attn_slices((int64_t)a.g * nkv, nkv));
+  const dim3 block(w4::kAttnThreads);
+  if (a.g == 1) hipLaunchKernelGGL((w4::attn_decode_kernel<DT, D, 1>), grid, block, 0, st, a);
+  else if (a.g == 2) hipLaunchKernelGGL((w4::attn_decode_kernel<DT, D, 2>), grid, block, 0, st, a);
+  else hipLaunchKernelGGL((w4::attn_decode_kernel<DT, D, 4>), grid, block, 0, st, a);
+}
+
+}  // namespace
+
+extern "C" size_t w4_attention_decode_workspace_bytes(int64_t num_heads, int64_t num_kv_heads, int64_t head_dim,
+                                                      int64_t max_len) {
+  if (!attn_decode_shape_ok(num_heads, num_kv_heads, head_dim, max_len)) return 0;
+  const int64_t chunk = attn_chunk(max_len), chunks = (max_len + chunk - 1) / chunk;
+  return W4_WORKSPACE_COUNTER_BYTES + (size_t)(num_kv_heads * attn_slices(num_heads, num_kv_heads) * chunks *
+                                             w4::kAttnHeads * (head_dim + 2)) * 4;
+}
+
+extern "C" int w4_attention_decode(const void* q, const void* k, const void* v, int dtype, int64_t num_heads,
+                                   int64_t num_kv_heads, int64_t head_dim, const float* cos, const float* sin,
+                                   float* k_cache, float* v_cache, int64_t max_len, const int64_t* pos, void* out,
+                                   void* workspace, size_t workspace_bytes, void* stream) {
+  clear_error();
+  if (dtype != W4_DTYPE_BF16 && dtype != W4_DTYPE_FP16)
+    return fail(W4_ERR_INVALID, "w4_attention_decode: dtype must be bf16 or fp16 (got code %d)", dtype);
+  if (!attn_decode_shape_ok(num_heads, num_kv_heads, head_dim, max_len))
+    return fail(W4_ERR_UNSUPPORTED,
+                "w4_attention_decode: %lld query / %lld key-value heads of %lld over %lld positions "
+                "(heads of 64 or 128)",
+                (long long)num_heads, (long long)num_kv_heads, (long long)head_dim, (long long)max_len);
+  if (!q || !k || !v || !cos || !sin || !k_cache || !v_cache || !pos || !out)
+    return fail(W4_ERR_INVALID, "w4_attention_decode: null pointer");
+  const size_t need = w4_attention_decode_workspace_bytes(num_heads, num_kv_heads, head_dim, max_len);
+  if (workspace == nullptr || workspace_bytes < need || ((uintptr_t)workspace % 256) != 0)
+    return fail(W4_ERR_WORKSPACE, "w4_attention_decode: needs a 256-byte aligned workspace of %zu bytes (got %zu)",
+                need, workspace_bytes);
+  w4::AttnDecodeArgs a{};
+  a.q = static_cast<const uint16_t*>(q);
+  a.k = static_cast<const uint16_t*>(k);
+  a.v = static_cast<const uint16_t*>(v);
+  a.cos = cos;
+  a.sin = sin;
+  a.kc = k_cache;
+  a.vc = v_cache;
+  a.pos = pos;
+  a.out = static_cast<uint16_t*>(out);
+  a.cnt = static_cast<unsigned*>(workspace);
+  a.part = reinterpret_cast<float*>(static_cast<char*>(workspace) + W4_WORKSPACE_COUNTER_BYTES);
+  a.qscale = w4::kLog2e / sqrtf((float)head_dim);
+  a.g = (int)(num_heads / num_kv_heads);
+  a.max_len = (int)max_len;
+  a.chunk = attn_chunk(max_len);
+  a.chunks = (int)((max_len + a.chunk - 1) / a.chunk);
+  hipStream_t st = static_cast<hipStream_t>(stream);
+  const int nkv = (int)num_kv_heads;
+  if (dtype == W4_DTYPE_BF16) {
+    if (head_dim == 64) launch_decode<W4_DTYPE_BF16, 64>(a, nkv, st);
+    else launch_decode<W4_DTYPE_BF16, 128>(a, nkv, st);
+  } else {
+    if (head_dim == 64) launch_decode<W4_DTYPE_FP16, 64>(a, nkv, st);
+    else launch_decode<W4_DTYPE_FP16, 128>(a, nkv, st);
+  }
+  return check_launch("w4_attention_decode");
+}

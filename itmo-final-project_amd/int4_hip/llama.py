@@ -35,6 +35,8 @@ import torch
 import torch.nn as nn
 import torch.nn.functional as F
 
+from . import llama_ops
+
 
 @dataclass
 class LlamaConfig:
@@ -117,7 +119,8 @@ class Attention(nn.Module):
 
     def forward(self, x, cos, sin, kc, vc, pos0: int | None, pos_t: torch.Tensor | None, mask_bias):
         """Prefill (pos0 = 0, T tokens) or one decode token (pos_t = device position,
-        mask_bias [positions] = 0 up to pos_t, -inf past it)."""
+        mask_bias [positions] = 0 up to pos_t, -inf past it, or None where
+        the fused decode kernel applies)."""
         T = x.shape[0]
         nq, nk = self.nh * self.d, self.nkv * self.d
         g = self.nh // self.nkv
@@ -141,6 +144,10 @@ class Attention(nn.Module):
             o = torch.bmm(torch.softmax(s, dim=-1), vv)                   # [kv, g*T, D]
             o = o.view(self.nkv, g, T, self.d).permute(2, 0, 1, 3).reshape(T, nq)
         else:
+            if mask_bias is None:  # one fused launch (the caller found it applicable)
+                qo, ko, vo = _grouped(x, mods) if _all_int4(mods) else [m(x) for m in mods]
+                return self.o_proj(llama_ops.attention_decode(qo, ko, vo, cos, sin, kc, vc, pos_t, self.nh, self.nkv,
+                                                              self.d))
             if _all_int4(mods):
                 qkv = torch.empty((1, nq + 2 * nk), dtype=x.dtype, device=x.device)
                 _grouped(x, mods, qkv)
@@ -223,7 +230,10 @@ class LlamaForCausalLM(nn.Module):
 
     def _layers(self, x, cos, sin, pos0, pos_t):
         mask_bias = None
-        if pos_t is not None:
+        c = self.config
+        if pos_t is not None and not llama_ops.attention_decode_ok(x, self.kc, self.vc, cos, sin, pos_t,
+                                                                   c.num_attention_heads, c.num_key_value_heads,
+                                                                   c.head_dim):
             mask_bias = torch.zeros(self.max_len, device=x.device).masked_fill_(self.key_pos > pos_t, float("-inf"))
         for i, layer in enumerate(self.model.layers):
             x = x + layer.self_attn(layer.input_layernorm(x), cos, sin, self.kc[i], self.vc[i], pos0, pos_t,

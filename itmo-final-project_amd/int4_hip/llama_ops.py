@@ -1,0 +1,86 @@
+"""Python side of the fused kernels that a decoder layer of ``llama.py`` runs
+between its linears (csrc/w4_llama.hip).
+
+``fusable`` says whether plain tensors on one GPU are at hand, outside autograd,
+tracing and tensor subclasses: only then may a kernel be launched on raw
+pointers.  Everything else takes the torch operations of ``llama.py``, which
+define the results.
+"""
+from __future__ import annotations
+
+import torch
+import torch.nn as nn
+from torch.utils._python_dispatch import _get_current_dispatch_mode
+
+from . import _lib
+from .gemm import _with_workspace
+
+_XDT = {torch.bfloat16: _lib.DTYPE_BF16, torch.float16: _lib.DTYPE_FP16}
+_PLAIN = (torch.Tensor, nn.Parameter)
+
+
+def fusable(*tensors: torch.Tensor) -> bool:
+    """Plain tensors on one GPU with nothing recording or transforming the call."""
+    if (torch.compiler.is_compiling() or torch.jit.is_tracing() or _get_current_dispatch_mode() is not None
+            or torch.is_autocast_enabled("cuda")):
+        return False
+    dev = tensors[0].device
+    grad = torch.is_grad_enabled()
+    for t in tensors:
+        if type(t) not in _PLAIN or t.device != dev or torch._C._functorch.is_functorch_wrapped_tensor(t):
+            return False
+        if (grad and t.requires_grad) or (torch.autograd.forward_ad._current_level >= 0 and
+                                          torch.autograd.forward_ad.unpack_dual(t).tangent is not None):
+            return False
+    return dev.type == "cuda" and torch._C._len_torch_function_stack() == 0
+
+
+def _on(device: torch.device, call) -> int:
+    """``call(stream)`` on the current stream of ``device``, made current."""
+    if torch._C._cuda_getDevice() == device.index:
+        return call(torch._C._cuda_getCurrentRawStream(device.index))
+    with torch.cuda.device(device):
+        return call(torch._C._cuda_getCurrentRawStream(device.index))
+
+
+def _dense(*tensors: torch.Tensor) -> bool:
+    return all(t.is_contiguous() and t.data_ptr() % 16 == 0 for t in tensors)
+
+
+_ATTN_WS: dict = {}
+
+
+def _attn_ws_bytes(nh: int, nkv: int, d: int, max_len: int) -> int:
+    """Workspace size of one decode step (0: unsupported shape); a pure function, memoised."""
+    key = (nh, nkv, d, max_len)
+    b = _ATTN_WS.get(key)
+    if b is None:
+        b = _ATTN_WS[key] = _lib.load().w4_attention_decode_workspace_bytes(nh, nkv, d, max_len)
+    return b
+
+
+def attention_decode_ok(x, kc, vc, cos, sin, pos, nh: int, nkv: int, d: int) -> bool:
+    """Whether ``attention_decode`` takes a step with activations like ``x``
+    ([1, hidden]) and the caches ``kc`` [.., nkv, d, L], ``vc`` [.., nkv, L, d]."""
+    return (x.shape[0] == 1 and x.dtype in _XDT and kc.dtype == vc.dtype == cos.dtype == sin.dtype == torch.float32
+            and pos.dtype == torch.int64 and pos.numel() == 1 and cos.shape == sin.shape == (1, d // 2)
+            and kc.is_contiguous() and vc.is_contiguous() and cos.is_contiguous() and sin.is_contiguous()
+            and fusable(x, kc, vc, cos, sin, pos) and _attn_ws_bytes(nh, nkv, d, kc.shape[-1]) > 0)
+
+
+def attention_decode(q, k, v, cos, sin, kc, vc, pos, nh: int, nkv: int, d: int) -> torch.Tensor:
+    """Attention output [1, nh * d] of one token: q [nh * d], k, v [nkv * d] values
+    before the rotary embedding; the caches of one layer are updated in place."""
+    dev = q.device
+    max_len = kc.shape[-1]
+    q, k, v = (t.contiguous() for t in (q, k, v))
+    assert q.dtype == k.dtype == v.dtype and q.numel() == nh * d and k.numel() == v.numel() == nkv * d
+    out = torch.empty((1, nh * d), dtype=q.dtype, device=dev)
+    lib = _lib.load()
+    rc = _on(dev, lambda st: _with_workspace(dev, st, _attn_ws_bytes(nh, nkv, d, max_len), lambda ws, nb:
+             lib.w4_attention_decode(q.data_ptr(), k.data_ptr(), v.data_ptr(), _XDT[q.dtype], nh, nkv, d,
+                                     cos.data_ptr(), sin.data_ptr(), kc.data_ptr(), vc.data_ptr(), max_len,
+                                     pos.data_ptr(), out.data_ptr(), ws, nb, st)))
+    if rc:
+        _lib.check(rc, "w4_attention_decode")
+    return out

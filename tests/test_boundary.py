@@ -76,6 +76,21 @@ def test_c_abi_rejects_bad_gemm_arguments(lib):
         assert n == 0 or n > 65536
 
 
+def test_c_abi_rejects_bad_attention_arguments(lib):
+    fake = ctypes.c_void_p(256)
+    size = lib.w4_attention_decode_workspace_bytes
+    assert size(32, 8, 64, 648) > 65536 and size(32, 8, 96, 648) == 0 and size(30, 8, 64, 648) == 0
+    assert size(32, 8, 64, 0) == 0
+
+    def call(dt=0, nh=8, nkv=2, d=64, L=64, ws=fake, nb=1 << 20, q=fake):
+        return lib.w4_attention_decode(q, fake, fake, dt, nh, nkv, d, fake, fake, fake, fake, L, fake, fake, ws, nb,
+                                       None)
+
+    assert call(dt=2) == _lib.ERR_INVALID and call(q=None) == _lib.ERR_INVALID
+    assert call(d=32) == _lib.ERR_UNSUPPORTED and call(nh=7) == _lib.ERR_UNSUPPORTED
+    assert call(nb=size(8, 2, 64, 64) - 1) == _lib.ERR_WORKSPACE and call(ws=None) == _lib.ERR_WORKSPACE
+
+
 def test_workspace_queries_over_regime_boundaries(lib):
     """The size queries run the launch planners on the host only: a sweep over
     the regime boundaries (M around 1 / 4 / 8 / 16 / 64 / 128, K around 4096 and

@@ -1,0 +1,96 @@
+"""GPU: the fused kernels between the linears of a decoder layer
+(int4_hip/llama_ops.py) against 64-bit torch arithmetic on the CPU."""
+import math
+
+import pytest
+import torch
+
+from _synth import randn
+from int4_hip import llama_ops
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+# one rounding to the output dtype (half an ulp: 2^-8 of the value for bf16's 8
+# significant bits, 2^-11 for fp16's 11), plus fp32 arithmetic: sums of up to a
+# few thousand positive terms of relative error 2^-24 each, far below it
+ROUND = {torch.bfloat16: 2.0 ** -8, torch.float16: 2.0 ** -11}
+FP32 = 1e-5
+
+
+def _rope(t, cos, sin):
+    """t [T, heads, D] fp32, products rounded separately as the kernels do."""
+    h = t.shape[-1] // 2
+    a, b, c, s = t[..., :h], t[..., h:], cos[:, None, :], sin[:, None, :]
+    return torch.cat((a * c - b * s, b * c + a * s), -1)
+
+
+def _tables(n, d):
+    ang = torch.arange(n)[:, None] * (1.0 / 500000.0 ** (torch.arange(0, d, 2) / d))[None, :]
+    return ang.cos().float(), ang.sin().float()
+
+
+def _attention(q, kc, vc, pos0):
+    """fp64 attention of q [T, nh, D] at positions pos0.. over kc [nkv, D, L], vc [nkv, L, D]."""
+    T, nh, D = q.shape
+    nkv, L = kc.shape[0], pos0 + T
+    out = torch.empty((T, nh, D), dtype=torch.float64)
+    mask = torch.arange(L)[None, :] > torch.arange(pos0, L)[:, None]
+    for h in range(nh):
+        s = q[:, h].double() @ kc[h * nkv // nh, :, :L].double() / math.sqrt(D)
+        out[:, h] = torch.softmax(s.masked_fill(mask, float("-inf")), -1) @ vc[h * nkv // nh, :L].double()
+    return out.reshape(T, nh * D)
+
+
+def _check_out(got, want, dtype):
+    got = got.double().cpu()
+    scale = want.square().mean().sqrt()
+    err = (got - want).abs() / torch.maximum(want.abs(), scale)
+    assert err.max().item() <= ROUND[dtype] + 10 * FP32, err.max().item()
+
+
+# positions at the edges of a 64-position chunk and of the cache; one, several
+# and many query heads per key-value head (slices of four); caches past 4096
+# positions (chunks of 128); cache lengths that are no multiple of four
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("nh,nkv,d,max_len,pos", [
+    (1, 1, 64, 1, 0), (8, 2, 64, 96, 0), (8, 2, 64, 96, 63), (8, 2, 64, 96, 64), (8, 8, 64, 97, 96),
+    (32, 8, 64, 648, 575), (6, 2, 128, 200, 127), (20, 2, 128, 333, 332), (16, 2, 64, 4099, 4098),
+    (4, 1, 128, 8193, 5000), (2, 1, 64, 130, 129)])
+def test_attention_decode(dtype, nh, nkv, d, max_len, pos):
+    print(f"[attn decode] {dtype} {nh}/{nkv}x{d} L={max_len} pos={pos}", flush=True)
+    q, k, v = (randn((1, n * d), seed=i, dtype=dtype) for i, n in enumerate((nh, nkv, nkv)))
+    kc, vc = randn((nkv, d, max_len), 5, dtype=torch.float32), randn((nkv, max_len, d), 6, dtype=torch.float32)
+    # what lies past the position takes no part, whatever it holds
+    kc[..., pos + 1:] = float("nan")
+    vc[:, pos + 1:] = float("inf")
+    cos, sin = (t[pos:pos + 1] for t in _tables(max_len, d))
+    p = torch.tensor([pos], device=DEV)
+    args = [t.to(DEV) for t in (q, k, v, cos.contiguous(), sin.contiguous(), kc, vc)]
+    assert llama_ops.attention_decode_ok(args[0], *args[5:], *args[3:5], p, nh, nkv, d)
+    got = llama_ops.attention_decode(*args, p, nh, nkv, d)
+    again = llama_ops.attention_decode(*args, p, nh, nkv, d)
+    kc[:, :, pos] = _rope(k.float().view(1, nkv, d), cos, sin)[0]
+    vc[:, pos] = v.float().view(nkv, d)
+    assert torch.equal(args[5].cpu().nan_to_num(7.0), kc.nan_to_num(7.0)) and torch.equal(args[6].cpu(), vc)
+    assert torch.equal(got, again)
+    _check_out(got, _attention(_rope(q.float().view(1, nh, d), cos, sin), kc, vc, pos), dtype)
+
+
+def test_attention_decode_infinities_and_nan():
+    """-inf scores weigh nothing (a whole chunk of them included), an infinite or
+    NaN score makes its head NaN, as torch's softmax does."""
+    d, L, pos = 64, 256, 200
+    cos, sin = torch.ones((1, d // 2)), torch.zeros((1, d // 2))
+    q = torch.ones((1, 4 * d), dtype=torch.bfloat16)
+    k = v = torch.zeros((1, 4 * d), dtype=torch.bfloat16)
+    kc, vc = torch.zeros((4, d, L)), randn((4, L, d), 1, dtype=torch.float32)
+    kc[0, 0, :64] = float("-inf")   # head 0: its first chunk weighs nothing
+    kc[1, 0, 100] = float("inf")    # head 1: inf - inf
+    kc[2, 0, 70] = float("nan")
+    kc[3, 0, :pos] = float("-inf")  # head 3: only the new position weighs
+    args = [t.to(DEV) for t in (q, k, v, cos, sin, kc, vc)]
+    got = llama_ops.attention_decode(*args, torch.tensor([pos], device=DEV), 4, 4, d).view(4, d).cpu()
+    vc[:, pos] = 0
+    torch.testing.assert_close(got[0].float(), vc[0, 64:pos + 1].mean(0), rtol=1e-2, atol=1e-3)
+    assert got[1].isnan().all() and got[2].isnan().all()
+    assert torch.equal(got[3], torch.zeros(d, dtype=torch.bfloat16))
