@@ -246,6 +246,19 @@ int w4_attention_decode(const void* q, const void* k, const void* v, int dtype, 
                         float* k_cache, float* v_cache, int64_t max_len, const int64_t* pos, void* out,
                         void* workspace, size_t workspace_bytes, void* stream);
 
+/*
+ * RMSNorm of `rows` dense rows of n values (bf16 / fp16; n a multiple of 8, at
+ * most 16384; operands 16-byte aligned): y = x / sqrt(mean(x^2) + eps) *
+ * weight, fp32 inside, rounded once.  With `delta` (else NULL, and sum NULL)
+ * the input is x + delta rounded to the dtype, which is written to `sum`.
+ * w4_silu_mul: y = silu(gate) * up over `count` values (a multiple of 8),
+ * fp32 inside, rounded once.
+ * No counterpart in the reference (see w4_attention_decode).
+ */
+int w4_rmsnorm(const void* x, const void* delta, const void* weight, int dtype, int64_t rows, int64_t n,
+               float eps, void* sum, void* y, void* stream);
+int w4_silu_mul(const void* gate, const void* up, int dtype, int64_t count, void* y, void* stream);
+
 #ifdef __cplusplus
 }
 #endif

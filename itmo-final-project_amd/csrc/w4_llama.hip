@@ -1,5 +1,6 @@
 // Kernels of a Llama-style decoder layer between its W4A16 linears
-// (int4_hip/llama.py): the attention of one decode step.
+// (int4_hip/llama.py): the attention of one decode step, RMSNorm (with the
+// residual addition before it) and the gated activation of the MLP.
 //
 // One token's attention is a handful of tiny operations (rotary embedding of
 // q and k, two cache writes, q.K, softmax, p.V), so as separate launches it is
@@ -278,6 +279,103 @@ __global__ __launch_bounds__(kAttnThreads) void attn_decode_kernel(AttnDecodeArg
   }
 }
 
+// Eight consecutive 16-bit values as floats, and back.
+template <int DT>
+__device__ __forceinline__ void unpack8(const u32x4 r, float v[8]) {
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    v[2 * j] = act_bits_to_float((uint16_t)(r[j] & 0xFFFFu), DT);
+    v[2 * j + 1] = act_bits_to_float((uint16_t)(r[j] >> 16), DT);
+  }
+}
+template <int DT>
+__device__ __forceinline__ u32x4 pack8(const float v[8]) {
+  u32x4 r;
+#pragma unroll
+  for (int j = 0; j < 4; ++j)
+    r[j] = (uint32_t)float_to_act_bits<DT>(v[2 * j]) | ((uint32_t)float_to_act_bits<DT>(v[2 * j + 1]) << 16);
+  return r;
+}
+
+constexpr int kNormThreads = 256;
+constexpr int kNormMaxVecs = 8;  // 16-byte vectors per thread: rows of up to 16384
+
+// y = x / sqrt(mean(x^2) + eps) * weight, rows of n values, fp32 inside and one
+// rounding; with a delta the row is first x + delta, rounded to the dtype (the
+// residual stream) and written to sum.  One workgroup per row, the row held in
+// registers (VPT vectors per thread) between the two passes over it.  For one
+// row it is bound by launch and one trip to memory, for many by HBM: fusing
+// the addition saves a launch and a read and write of the row.  With
+// silu_mul_kernel, the 1B model's decode step went from 848 to 728 us.
+template <int DT, int VPT, bool ADD>
+__global__ __launch_bounds__(kNormThreads) void rmsnorm_kernel(const uint16_t* __restrict__ x,
+                                                               const uint16_t* __restrict__ delta,
+                                                               const uint16_t* __restrict__ weight, int n, float eps,
+                                                               uint16_t* __restrict__ sum, uint16_t* __restrict__ y) {
+  __shared__ float part[kNormThreads / 64];
+  const int tid = threadIdx.x, vecs = n / 8;
+  const int64_t row = (int64_t)blockIdx.x * n;
+  u32x4 xr[VPT], dr[VPT], wr[VPT];
+#pragma unroll
+  for (int i = 0; i < VPT; ++i) {
+    const int v = tid + i * kNormThreads;
+    xr[i] = dr[i] = wr[i] = u32x4{0u, 0u, 0u, 0u};
+    if (v < vecs) {
+      xr[i] = *reinterpret_cast<const u32x4*>(x + row + v * 8);
+      if constexpr (ADD) dr[i] = *reinterpret_cast<const u32x4*>(delta + row + v * 8);
+      wr[i] = *reinterpret_cast<const u32x4*>(weight + v * 8);
+    }
+  }
+  float xv[VPT][8], sq = 0.f;
+#pragma unroll
+  for (int i = 0; i < VPT; ++i) {
+    unpack8<DT>(xr[i], xv[i]);
+    if constexpr (ADD) {
+      float dv[8];
+      unpack8<DT>(dr[i], dv);
+#pragma unroll
+      for (int j = 0; j < 8; ++j) xv[i][j] += dv[j];
+      const u32x4 s = pack8<DT>(xv[i]);
+      const int v = tid + i * kNormThreads;
+      if (v < vecs) *reinterpret_cast<u32x4*>(sum + row + v * 8) = s;
+      unpack8<DT>(s, xv[i]);
+    }
+#pragma unroll
+    for (int j = 0; j < 8; ++j) sq = __builtin_fmaf(xv[i][j], xv[i][j], sq);
+  }
+  sq = wave_sum(sq);
+  if ((tid & 63) == 0) part[tid >> 6] = sq;
+  __syncthreads();
+  const float r = 1.0f / sqrtf(((part[0] + part[1]) + (part[2] + part[3])) / (float)n + eps);
+#pragma unroll
+  for (int i = 0; i < VPT; ++i) {
+    const int v = tid + i * kNormThreads;
+    float wv[8], o[8];
+    unpack8<DT>(wr[i], wv);
+#pragma unroll
+    for (int j = 0; j < 8; ++j) o[j] = xv[i][j] * r * wv[j];
+    if (v < vecs) *reinterpret_cast<u32x4*>(y + row + v * 8) = pack8<DT>(o);
+  }
+}
+
+// y = silu(gate) * up, fp32 inside and one rounding (the separate operations
+// round silu(gate) too).  Eight values per thread: HBM-bound once it fills the
+// chip, a launch and a trip to memory below that.  One launch and pass less
+// than silu and multiply: an MLP of 2048 x 2048 x 8192 from 222 to 205 us.
+template <int DT>
+__global__ __launch_bounds__(256) void silu_mul_kernel(const uint16_t* __restrict__ gate,
+                                                       const uint16_t* __restrict__ up, int64_t vecs,
+                                                       uint16_t* __restrict__ y) {
+  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (i >= vecs) return;
+  float g[8], u[8];
+  unpack8<DT>(reinterpret_cast<const u32x4*>(gate)[i], g);
+  unpack8<DT>(reinterpret_cast<const u32x4*>(up)[i], u);
+#pragma unroll
+  for (int j = 0; j < 8; ++j) u[j] *= g[j] / (1.0f + __expf(-g[j]));
+  reinterpret_cast<u32x4*>(y)[i] = pack8<DT>(u);
+}
+
 }  // namespace w4
 
 using namespace w4host;
@@ -362,4 +460,71 @@ extern "C" int w4_attention_decode(const void* q, const void* k, const void* v, 
     else launch_decode<W4_DTYPE_FP16, 128>(a, nkv, st);
   }
   return check_launch("w4_attention_decode");
+}
+
+namespace {
+
+template <int DT, bool ADD>
+void launch_rmsnorm(const uint16_t* x, const uint16_t* delta, const uint16_t* weight, int64_t rows, int n, float eps,
+                    uint16_t* sum, uint16_t* y, hipStream_t st) {
+  const dim3 grid((unsigned)rows), block(w4::kNormThreads);
+  const int vpt = (n / 8 + w4::kNormThreads - 1) / w4::kNormThreads;
+#define W4_NORM(V) \
+  hipLaunchKernelGGL((w4::rmsnorm_kernel<DT, V, ADD>), grid, block, 0, st, x, delta, weight, n, eps, sum, y)
+  if (vpt <= 1) W4_NORM(1);
+  else if (vpt <= 2) W4_NORM(2);
+  else if (vpt <= 4) W4_NORM(4);
+  else W4_NORM(8);
+#undef W4_NORM
+}
+
+}  // namespace
+
+extern "C" int w4_rmsnorm(const void* x, const void* delta, const void* weight, int dtype, int64_t rows, int64_t n,
+                          float eps, void* sum, void* y, void* stream) {
+  clear_error();
+  if (dtype != W4_DTYPE_BF16 && dtype != W4_DTYPE_FP16)
+    return fail(W4_ERR_INVALID, "w4_rmsnorm: dtype must be bf16 or fp16 (got code %d)", dtype);
+  if (rows < 0 || rows >= (1LL << 31) || n < 8 || n % 8 != 0 || n > 8 * w4::kNormThreads * w4::kNormMaxVecs)
+    return fail(W4_ERR_UNSUPPORTED, "w4_rmsnorm: %lld rows of %lld (a multiple of 8, at most %d)", (long long)rows,
+                (long long)n, 8 * w4::kNormThreads * w4::kNormMaxVecs);
+  if (rows == 0) return W4_OK;
+  if (!x || !weight || !y || (delta != nullptr) != (sum != nullptr))
+    return fail(W4_ERR_INVALID, "w4_rmsnorm: null pointer");
+  if ((((uintptr_t)x | (uintptr_t)delta | (uintptr_t)weight | (uintptr_t)sum | (uintptr_t)y) % 16) != 0)
+    return fail(W4_ERR_INVALID, "w4_rmsnorm: operands must be 16-byte aligned");
+  const uint16_t *xp = static_cast<const uint16_t*>(x), *dp = static_cast<const uint16_t*>(delta),
+                 *wp = static_cast<const uint16_t*>(weight);
+  uint16_t *sp = static_cast<uint16_t*>(sum), *yp = static_cast<uint16_t*>(y);
+  hipStream_t st = static_cast<hipStream_t>(stream);
+  if (dtype == W4_DTYPE_BF16) {
+    if (dp) launch_rmsnorm<W4_DTYPE_BF16, true>(xp, dp, wp, rows, (int)n, eps, sp, yp, st);
+    else launch_rmsnorm<W4_DTYPE_BF16, false>(xp, dp, wp, rows, (int)n, eps, sp, yp, st);
+  } else {
+    if (dp) launch_rmsnorm<W4_DTYPE_FP16, true>(xp, dp, wp, rows, (int)n, eps, sp, yp, st);
+    else launch_rmsnorm<W4_DTYPE_FP16, false>(xp, dp, wp, rows, (int)n, eps, sp, yp, st);
+  }
+  return check_launch("w4_rmsnorm");
+}
+
+extern "C" int w4_silu_mul(const void* gate, const void* up, int dtype, int64_t count, void* y, void* stream) {
+  clear_error();
+  if (dtype != W4_DTYPE_BF16 && dtype != W4_DTYPE_FP16)
+    return fail(W4_ERR_INVALID, "w4_silu_mul: dtype must be bf16 or fp16 (got code %d)", dtype);
+  if (count < 0 || count % 8 != 0 || count / 8 >= (1LL << 31) * 256)
+    return fail(W4_ERR_UNSUPPORTED, "w4_silu_mul: %lld values (a multiple of 8)", (long long)count);
+  if (count == 0) return W4_OK;
+  if (!gate || !up || !y) return fail(W4_ERR_INVALID, "w4_silu_mul: null pointer");
+  if ((((uintptr_t)gate | (uintptr_t)up | (uintptr_t)y) % 16) != 0)
+    return fail(W4_ERR_INVALID, "w4_silu_mul: operands must be 16-byte aligned");
+  const int64_t vecs = count / 8;
+  const dim3 grid((unsigned)((vecs + 255) / 256)), block(256);
+  hipStream_t st = static_cast<hipStream_t>(stream);
+  const uint16_t *gp = static_cast<const uint16_t*>(gate), *up16 = static_cast<const uint16_t*>(up);
+  uint16_t* yp = static_cast<uint16_t*>(y);
+  if (dtype == W4_DTYPE_BF16)
+    hipLaunchKernelGGL((w4::silu_mul_kernel<W4_DTYPE_BF16>), grid, block, 0, st, gp, up16, vecs, yp);
+  else
+    hipLaunchKernelGGL((w4::silu_mul_kernel<W4_DTYPE_FP16>), grid, block, 0, st, gp, up16, vecs, yp);
+  return check_launch("w4_silu_mul");
 }

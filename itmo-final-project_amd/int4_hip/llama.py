@@ -64,7 +64,24 @@ class RMSNorm(nn.Module):
     def forward(self, x: torch.Tensor) -> torch.Tensor:
         # one fused kernel; fp32 statistics (the weight is applied before the
         # final rounding, where the Hugging Face layer rounds first)
+        if llama_ops.rms_norm_ok(x, self.weight):
+            return llama_ops.rms_norm(x, self.weight, self.eps)
         return F.rms_norm(x, (x.shape[-1],), self.weight, self.eps)
+
+
+def _add_norm(x: torch.Tensor, delta: torch.Tensor, norm: nn.Module) -> tuple:
+    """(x + delta, norm(x + delta)), in one launch where ``norm`` is a plain RMSNorm
+    that nothing hooks into."""
+    if (type(norm) is RMSNorm and "forward" not in norm.__dict__ and not norm._forward_hooks
+            and not norm._forward_pre_hooks and not nn.modules.module._has_any_global_hook()
+            and llama_ops.rms_norm_ok(x, norm.weight, delta)):
+        return llama_ops.rms_norm(x, norm.weight, norm.eps, delta)
+    x = x + delta
+    return x, norm(x)
+
+
+def _silu_mul(gate: torch.Tensor, up: torch.Tensor) -> torch.Tensor:
+    return llama_ops.silu_mul(gate, up) if llama_ops.silu_mul_ok(gate, up) else F.silu(gate) * up
 
 
 def rope_inv_freq(cfg: LlamaConfig) -> torch.Tensor:
@@ -172,8 +189,8 @@ class MLP(nn.Module):
     def forward(self, x):
         if _all_int4((self.gate_proj, self.up_proj)):
             g, u = _grouped(x, (self.gate_proj, self.up_proj))
-            return self.down_proj(F.silu(g) * u)
-        return self.down_proj(F.silu(self.gate_proj(x)) * self.up_proj(x))
+            return self.down_proj(_silu_mul(g, u))
+        return self.down_proj(_silu_mul(self.gate_proj(x), self.up_proj(x)))
 
 
 class DecoderLayer(nn.Module):
@@ -235,11 +252,15 @@ class LlamaForCausalLM(nn.Module):
                                                                    c.num_attention_heads, c.num_key_value_heads,
                                                                    c.head_dim):
             mask_bias = torch.zeros(self.max_len, device=x.device).masked_fill_(self.key_pos > pos_t, float("-inf"))
-        for i, layer in enumerate(self.model.layers):
-            x = x + layer.self_attn(layer.input_layernorm(x), cos, sin, self.kc[i], self.vc[i], pos0, pos_t,
-                                    mask_bias)
-            x = x + layer.mlp(layer.post_attention_layernorm(x))
-        return self.lm_head(self.model.norm(x))
+        # each residual addition is fused with the norm that follows it
+        layers = self.model.layers
+        norms = [layer.input_layernorm for layer in layers] + [self.model.norm]
+        h = norms[0](x)
+        for i, layer in enumerate(layers):
+            a = layer.self_attn(h, cos, sin, self.kc[i], self.vc[i], pos0, pos_t, mask_bias)
+            x, h = _add_norm(x, a, layer.post_attention_layernorm)
+            x, h = _add_norm(x, layer.mlp(h), norms[i + 1])
+        return self.lm_head(h)
 
     @torch.no_grad()
     def prefill(self, ids: torch.Tensor) -> torch.Tensor:

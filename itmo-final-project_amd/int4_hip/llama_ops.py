@@ -10,7 +10,9 @@ from __future__ import annotations
 
 import torch
 import torch.nn as nn
-from torch.utils._python_dispatch import _get_current_dispatch_mode
+from torch import _C
+from torch.autograd import forward_ad
+from torch.compiler import is_compiling as _is_compiling
 
 from . import _lib
 from .gemm import _with_workspace
@@ -21,26 +23,26 @@ _PLAIN = (torch.Tensor, nn.Parameter)
 
 def fusable(*tensors: torch.Tensor) -> bool:
     """Plain tensors on one GPU with nothing recording or transforming the call."""
-    if (torch.compiler.is_compiling() or torch.jit.is_tracing() or _get_current_dispatch_mode() is not None
-            or torch.is_autocast_enabled("cuda")):
+    if (_is_compiling() or _C._get_tracing_state() is not None or _C._len_torch_dispatch_stack() or
+            _C._len_torch_function_stack() or _C._functorch.peek_interpreter_stack() is not None or
+            torch.is_autocast_enabled("cuda") or forward_ad._current_level >= 0):
         return False
     dev = tensors[0].device
+    if dev.type != "cuda":
+        return False
     grad = torch.is_grad_enabled()
     for t in tensors:
-        if type(t) not in _PLAIN or t.device != dev or torch._C._functorch.is_functorch_wrapped_tensor(t):
+        if type(t) not in _PLAIN or t.device != dev or (grad and t.requires_grad):
             return False
-        if (grad and t.requires_grad) or (torch.autograd.forward_ad._current_level >= 0 and
-                                          torch.autograd.forward_ad.unpack_dual(t).tangent is not None):
-            return False
-    return dev.type == "cuda" and torch._C._len_torch_function_stack() == 0
+    return True
 
 
 def _on(device: torch.device, call) -> int:
     """``call(stream)`` on the current stream of ``device``, made current."""
-    if torch._C._cuda_getDevice() == device.index:
-        return call(torch._C._cuda_getCurrentRawStream(device.index))
+    if _C._cuda_getDevice() == device.index:
+        return call(_C._cuda_getCurrentRawStream(device.index))
     with torch.cuda.device(device):
-        return call(torch._C._cuda_getCurrentRawStream(device.index))
+        return call(_C._cuda_getCurrentRawStream(device.index))
 
 
 def _dense(*tensors: torch.Tensor) -> bool:
@@ -84,3 +86,45 @@ def attention_decode(q, k, v, cos, sin, kc, vc, pos, nh: int, nkv: int, d: int) 
     if rc:
         _lib.check(rc, "w4_attention_decode")
     return out
+
+
+MAX_NORM = 16384  # widest row of w4_rmsnorm
+
+
+def rms_norm_ok(x, weight, delta=None) -> bool:
+    """Whether ``rms_norm`` takes ``x`` [..., n] (and a residual ``delta`` like it)."""
+    n = x.shape[-1] if x.dim() else 0
+    ts = (x, weight) if delta is None else (x, weight, delta)
+    return (x.dtype in _XDT and 0 < n <= MAX_NORM and n % 8 == 0 and weight.shape == (n,)
+            and all(t.dtype == x.dtype for t in ts) and (delta is None or delta.shape == x.shape)
+            and fusable(*ts) and _dense(*ts))
+
+
+def rms_norm(x, weight, eps: float, delta=None):
+    """RMSNorm of ``x``; with ``delta`` the pair (x + delta, its RMSNorm)."""
+    n = x.shape[-1]
+    y = torch.empty_like(x)
+    s = None if delta is None else torch.empty_like(x)
+    lib = _lib.load()
+    rc = _on(x.device, lambda st: lib.w4_rmsnorm(
+        x.data_ptr(), None if delta is None else delta.data_ptr(), weight.data_ptr(), _XDT[x.dtype], x.numel() // n, n,
+        eps, None if s is None else s.data_ptr(), y.data_ptr(), st))
+    if rc:
+        _lib.check(rc, "w4_rmsnorm")
+    return y if delta is None else (s, y)
+
+
+def silu_mul_ok(gate, up) -> bool:
+    return (gate.dtype in _XDT and up.dtype == gate.dtype and up.shape == gate.shape and gate.numel() % 8 == 0
+            and fusable(gate, up) and _dense(gate, up))
+
+
+def silu_mul(gate, up) -> torch.Tensor:
+    """silu(gate) * up in one pass, one rounding."""
+    y = torch.empty_like(gate)
+    lib = _lib.load()
+    rc = _on(gate.device, lambda st: lib.w4_silu_mul(gate.data_ptr(), up.data_ptr(), _XDT[gate.dtype], gate.numel(),
+                                                     y.data_ptr(), st))
+    if rc:
+        _lib.check(rc, "w4_silu_mul")
+    return y

@@ -91,6 +91,23 @@ def test_c_abi_rejects_bad_attention_arguments(lib):
     assert call(nb=size(8, 2, 64, 64) - 1) == _lib.ERR_WORKSPACE and call(ws=None) == _lib.ERR_WORKSPACE
 
 
+def test_c_abi_rejects_bad_norm_and_activation_arguments(lib):
+    fake, odd = ctypes.c_void_p(256), ctypes.c_void_p(264)
+
+    def norm(x=fake, d=None, dt=0, rows=4, n=64, s=None):
+        return lib.w4_rmsnorm(x, d, fake, dt, rows, n, 1e-5, s, fake, None)
+
+    assert norm(dt=2) == _lib.ERR_INVALID and norm(x=None) == _lib.ERR_INVALID and norm(x=odd) == _lib.ERR_INVALID
+    assert norm(d=fake) == _lib.ERR_INVALID and norm(s=fake) == _lib.ERR_INVALID
+    assert norm(n=60) == _lib.ERR_UNSUPPORTED and norm(n=16392) == _lib.ERR_UNSUPPORTED
+    assert norm(rows=0) == _lib.OK
+    assert lib.w4_silu_mul(fake, fake, 2, 8, fake, None) == _lib.ERR_INVALID
+    assert lib.w4_silu_mul(fake, odd, 0, 8, fake, None) == _lib.ERR_INVALID
+    assert lib.w4_silu_mul(fake, None, 0, 8, fake, None) == _lib.ERR_INVALID
+    assert lib.w4_silu_mul(fake, fake, 0, 12, fake, None) == _lib.ERR_UNSUPPORTED
+    assert lib.w4_silu_mul(None, None, 0, 0, None, None) == _lib.OK
+
+
 def test_workspace_queries_over_regime_boundaries(lib):
     """The size queries run the launch planners on the host only: a sweep over
     the regime boundaries (M around 1 / 4 / 8 / 16 / 64 / 128, K around 4096 and

@@ -94,3 +94,51 @@ def test_attention_decode_infinities_and_nan():
     torch.testing.assert_close(got[0].float(), vc[0, 64:pos + 1].mean(0), rtol=1e-2, atol=1e-3)
     assert got[1].isnan().all() and got[2].isnan().all()
     assert torch.equal(got[3], torch.zeros(d, dtype=torch.bfloat16))
+
+
+# rows of one vector up to the widest (16384), widths that leave threads idle
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("rows,n", [(1, 8), (1, 2048), (3, 2056), (7, 4096), (2, 8200), (500, 512), (1, 16384)])
+def test_rms_norm(dtype, rows, n):
+    print(f"[rms norm] {dtype} {rows}x{n}", flush=True)
+    x, d, w = randn((rows, n), 1, dtype=dtype), randn((rows, n), 2, 0.3, dtype=dtype), randn((n,), 3, dtype=dtype)
+
+    def ref(t):
+        t = t.double()
+        return t * torch.rsqrt(t.square().mean(-1, keepdim=True) + 1e-5) * w.double()
+
+    xd, dd, wd = (t.to(DEV) for t in (x, d, w))
+    assert llama_ops.rms_norm_ok(xd, wd) and llama_ops.rms_norm_ok(xd, wd, dd)
+    _check_out(llama_ops.rms_norm(xd, wd, 1e-5), ref(x), dtype)
+    s, y = llama_ops.rms_norm(xd, wd, 1e-5, dd)
+    assert torch.equal(s.cpu(), x + d)
+    _check_out(y, ref(x + d), dtype)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("shape", [(1, 8), (1, 8192), (100, 2056), (2, 3, 264)])
+def test_silu_mul(dtype, shape):
+    g, u = randn(shape, 1, 4.0, dtype=dtype), randn(shape, 2, dtype=dtype)
+    gd, ud = g.to(DEV), u.to(DEV)
+    assert llama_ops.silu_mul_ok(gd, ud)
+    want = torch.nn.functional.silu(g.double()) * u.double()
+    got = llama_ops.silu_mul(gd, ud).cpu().double()
+    # relative to each value; fp16's smallest subnormal 2^-24 below that
+    assert ((got - want).abs() <= (ROUND[dtype] + FP32) * want.abs() + 2.0 ** -25).all()
+
+
+def test_fused_ops_leave_the_general_path_alone():
+    """Autograd, other dtypes, strided and misaligned operands take the torch operations."""
+    x = torch.randn(4, 64, device=DEV, dtype=torch.bfloat16)
+    w = torch.ones(64, device=DEV, dtype=torch.bfloat16)
+    assert llama_ops.rms_norm_ok(x, w) and llama_ops.silu_mul_ok(x, x)
+    g = x.clone().requires_grad_()
+    assert not llama_ops.rms_norm_ok(g, w) and not llama_ops.silu_mul_ok(g, x)
+    with torch.no_grad():
+        assert llama_ops.rms_norm_ok(g, w)
+    for bad in (x.float(), x.t().contiguous().t(), x.cpu(), torch.empty(257, device=DEV, dtype=x.dtype)[1:].view(4, 64)):
+        assert not llama_ops.rms_norm_ok(bad, w) and not llama_ops.silu_mul_ok(bad, bad)
+    assert not llama_ops.rms_norm_ok(x, w.float()) and not llama_ops.rms_norm_ok(x, w, x[:2])
+    with torch.autocast("cuda", dtype=torch.float16):
+        assert not llama_ops.rms_norm_ok(x, w)
+    assert not torch.func.vmap(lambda t: torch.zeros(()) + llama_ops.silu_mul_ok(t, t))(x).any()
