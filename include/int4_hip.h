@@ -247,6 +247,19 @@ int w4_attention_decode(const void* q, const void* k, const void* v, int dtype, 
                         void* workspace, size_t workspace_bytes, void* stream);
 
 /*
+ * Causal attention of `tokens` new tokens at positions pos0.. of a Llama-style
+ * layer (two launches): q [tokens, num_heads * head_dim], k and v [tokens,
+ * num_kv_heads * head_dim] dense, cos and sin [tokens, head_dim / 2]; caches,
+ * arithmetic and head sizes as in w4_attention_decode, positions before pos0
+ * taken from the caches.  pos0 + tokens <= max_len; out [tokens, num_heads *
+ * head_dim].  q, k, v, v_cache and out 16-byte aligned.
+ */
+int w4_attention_prefill(const void* q, const void* k, const void* v, int dtype, int64_t tokens,
+                         int64_t num_heads, int64_t num_kv_heads, int64_t head_dim, const float* cos,
+                         const float* sin, float* k_cache, float* v_cache, int64_t max_len, int64_t pos0,
+                         void* out, void* stream);
+
+/*
  * RMSNorm of `rows` dense rows of n values (bf16 / fp16; n a multiple of 8, at
  * most 16384; operands 16-byte aligned): y = x / sqrt(mean(x^2) + eps) *
  * weight, fp32 inside, rounded once.  With `delta` (else NULL, and sum NULL)

@@ -82,6 +82,8 @@ SIGNATURES = {
     "w4_attention_decode_workspace_bytes": (_c_sz, [_c_i64, _c_i64, _c_i64, _c_i64]),
     "w4_attention_decode": (_c_int, [_c_vp, _c_vp, _c_vp, _c_int, _c_i64, _c_i64, _c_i64, _c_vp, _c_vp, _c_vp, _c_vp,
                                      _c_i64, _c_vp, _c_vp, _c_vp, _c_sz, _c_vp]),
+    "w4_attention_prefill": (_c_int, [_c_vp, _c_vp, _c_vp, _c_int, _c_i64, _c_i64, _c_i64, _c_i64, _c_vp, _c_vp,
+                                      _c_vp, _c_vp, _c_i64, _c_i64, _c_vp, _c_vp]),
     "w4_rmsnorm": (_c_int, [_c_vp, _c_vp, _c_vp, _c_int, _c_i64, _c_i64, ctypes.c_float, _c_vp, _c_vp, _c_vp]),
     "w4_silu_mul": (_c_int, [_c_vp, _c_vp, _c_int, _c_i64, _c_vp, _c_vp]),
 }

@@ -145,6 +145,9 @@ class Attention(nn.Module):
         mods = (self.q_proj, self.k_proj, self.v_proj)
         if pos_t is None:
             qo, ko, vo = _grouped(x, mods) if _all_int4(mods) else [m(x) for m in mods]
+            if llama_ops.attention_prefill_ok(x, kc, vc, cos, sin, pos0, self.nh, self.nkv, self.d):
+                return self.o_proj(llama_ops.attention_prefill(qo, ko, vo, cos, sin, kc, vc, pos0, self.nh, self.nkv,
+                                                               self.d))
             q = apply_rope(qo.view(T, self.nh, self.d), cos, sin)
             k = apply_rope(ko.view(T, self.nkv, self.d), cos, sin)
             v = vo.view(T, self.nkv, self.d)

@@ -88,6 +88,34 @@ def attention_decode(q, k, v, cos, sin, kc, vc, pos, nh: int, nkv: int, d: int) 
     return out
 
 
+def attention_prefill_ok(x, kc, vc, cos, sin, pos0, nh: int, nkv: int, d: int) -> bool:
+    """Whether ``attention_prefill`` takes the tokens of ``x`` [T, hidden] at positions
+    pos0.. of the caches ``kc`` [nkv, d, L], ``vc`` [nkv, L, d]."""
+    T, L = x.shape[0], kc.shape[-1]
+    return (x.dim() == 2 and T >= 1 and d in (64, 128) and nh % nkv == 0 and type(pos0) is int
+            and 0 <= pos0 <= L - T and L < 1 << 24 and T <= 65535 * 16 and nkv <= 65535
+            and x.dtype in _XDT and kc.dtype == vc.dtype == cos.dtype == sin.dtype == torch.float32
+            and kc.shape == (nkv, d, L) and vc.shape == (nkv, L, d) and cos.shape == sin.shape == (T, d // 2)
+            and kc.is_contiguous() and cos.is_contiguous() and sin.is_contiguous()
+            and fusable(x, kc, vc, cos, sin) and _dense(vc))
+
+
+def attention_prefill(q, k, v, cos, sin, kc, vc, pos0: int, nh: int, nkv: int, d: int) -> torch.Tensor:
+    """Causal attention output [T, nh * d] of T tokens: q [T, nh * d], k, v [T, nkv * d]
+    before the rotary embedding; the caches of one layer are updated in place."""
+    T, dev = q.shape[0], q.device
+    q, k, v = (t if _dense(t) else t.clone(memory_format=torch.contiguous_format) for t in (q, k, v))
+    assert q.dtype == k.dtype == v.dtype and q.shape == (T, nh * d) and k.shape == v.shape == (T, nkv * d)
+    out = torch.empty_like(q)
+    lib = _lib.load()
+    rc = _on(dev, lambda st: lib.w4_attention_prefill(
+        q.data_ptr(), k.data_ptr(), v.data_ptr(), _XDT[q.dtype], T, nh, nkv, d, cos.data_ptr(), sin.data_ptr(),
+        kc.data_ptr(), vc.data_ptr(), kc.shape[-1], pos0, out.data_ptr(), st))
+    if rc:
+        _lib.check(rc, "w4_attention_prefill")
+    return out
+
+
 MAX_NORM = 16384  # widest row of w4_rmsnorm
 
 

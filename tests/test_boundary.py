@@ -88,6 +88,14 @@ def test_c_abi_rejects_bad_attention_arguments(lib):
 
     assert call(dt=2) == _lib.ERR_INVALID and call(q=None) == _lib.ERR_INVALID
     assert call(d=32) == _lib.ERR_UNSUPPORTED and call(nh=7) == _lib.ERR_UNSUPPORTED
+    def prefill(dt=0, T=8, nh=8, nkv=2, d=64, L=64, pos0=0, q=fake, out=fake):
+        return lib.w4_attention_prefill(q, fake, fake, dt, T, nh, nkv, d, fake, fake, fake, fake, L, pos0, out, None)
+
+    assert prefill(dt=2) == _lib.ERR_INVALID and prefill(q=None) == _lib.ERR_INVALID
+    assert prefill(out=ctypes.c_void_p(8)) == _lib.ERR_INVALID
+    assert prefill(T=65) == _lib.ERR_INVALID and prefill(pos0=57) == _lib.ERR_INVALID
+    assert prefill(d=96) == _lib.ERR_UNSUPPORTED and prefill(nh=9) == _lib.ERR_UNSUPPORTED
+    assert prefill(T=0) == _lib.OK
     assert call(nb=size(8, 2, 64, 64) - 1) == _lib.ERR_WORKSPACE and call(ws=None) == _lib.ERR_WORKSPACE
 
 

@@ -76,6 +76,55 @@ def test_attention_decode(dtype, nh, nkv, d, max_len, pos):
     _check_out(got, _attention(_rope(q.float().view(1, nh, d), cos, sin), kc, vc, pos), dtype)
 
 
+# tokens at the edges of a 16- / 32-query tile and of the 64-position blocks, a
+# prompt continued at pos0, cache ends inside a block, odd and even heads per
+# key-value head, cache rows that are no multiple of 16 bytes
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("T,pos0,max_len,nh,nkv,d", [
+    (1, 0, 1, 2, 1, 64), (15, 0, 15, 3, 1, 64), (16, 0, 64, 4, 2, 64), (33, 0, 40, 1, 1, 128), (64, 0, 64, 8, 8, 64),
+    (65, 0, 129, 8, 2, 64), (500, 0, 640, 8, 2, 64), (130, 61, 191, 6, 2, 128), (1, 300, 303, 20, 2, 64),
+    (270, 0, 271, 4, 4, 128)])
+def test_attention_prefill(dtype, T, pos0, max_len, nh, nkv, d):
+    print(f"[attn prefill] {dtype} T={T}+{pos0} L={max_len} {nh}/{nkv}x{d}", flush=True)
+    q, k, v = (randn((T, n * d), seed=i, dtype=dtype) for i, n in enumerate((nh, nkv, nkv)))
+    kc, vc = randn((nkv, d, max_len), 5, dtype=torch.float32), randn((nkv, max_len, d), 6, dtype=torch.float32)
+    # what lies past the prompt takes no part, whatever it holds
+    kc[..., pos0 + T:] = float("nan")
+    vc[:, pos0 + T:] = float("inf")
+    cos, sin = (t[pos0:pos0 + T].contiguous() for t in _tables(max_len, d))
+    args = [t.to(DEV) for t in (q, k, v, cos, sin, kc, vc)]
+    assert llama_ops.attention_prefill_ok(args[0], args[5], args[6], args[3], args[4], pos0, nh, nkv, d)
+    got = llama_ops.attention_prefill(*args, pos0, nh, nkv, d)
+    kc[:, :, pos0:pos0 + T] = _rope(k.float().view(T, nkv, d), cos, sin).permute(1, 2, 0)
+    vc[:, pos0:pos0 + T] = v.float().view(T, nkv, d).transpose(0, 1)
+    assert torch.equal(args[5].cpu().nan_to_num(7.0), kc.nan_to_num(7.0)) and torch.equal(args[6].cpu(), vc)
+    assert torch.equal(got, llama_ops.attention_prefill(*args, pos0, nh, nkv, d))
+    _check_out(got, _attention(_rope(q.float().view(T, nh, d), cos, sin), kc, vc, pos0), dtype)
+
+
+def test_attention_prefill_infinities_and_nan():
+    """As torch's softmax: rows that see only -inf scores, an infinite or a NaN score
+    are NaN; -inf scores beside finite ones weigh nothing."""
+    d, T = 64, 200
+    cos, sin = torch.ones((T, d // 2)), torch.zeros((T, d // 2))
+    # scores that overflow: an infinite key would be NaN after the rotation (inf * 0)
+    q = torch.full((T, 4 * d), 64.0, dtype=torch.bfloat16)
+    k = torch.zeros((T, 4, d), dtype=torch.bfloat16)
+    k[:64, 0, 0] = -3e38
+    k[100, 1, 0] = 3e38
+    k[70, 2, 0] = float("nan")
+    v = randn((T, 4, d), 1)
+    kc, vc = torch.zeros((4, d, T), device=DEV), torch.zeros((4, T, d), device=DEV)
+    got = llama_ops.attention_prefill(q.to(DEV), k.view(T, -1).to(DEV), v.view(T, -1).to(DEV), cos.to(DEV),
+                                      sin.to(DEV), kc, vc, 0, 4, 4, d).cpu().view(T, 4, d)
+    nan = got.isnan()
+    assert nan[:64, 0].all() and not nan[64:, 0].any()
+    torch.testing.assert_close(got[199, 0].float(), v[64:, 0].float().mean(0), rtol=1e-2, atol=1e-3)
+    assert not nan[:100, 1].any() and nan[100:, 1].all()
+    assert not nan[:70, 2].any() and nan[70:, 2].all()
+    assert not nan[:, 3].any()
+
+
 def test_attention_decode_infinities_and_nan():
     """-inf scores weigh nothing (a whole chunk of them included), an infinite or
     NaN score makes its head NaN, as torch's softmax does."""
