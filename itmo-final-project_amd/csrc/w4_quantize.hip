@@ -434,36 +434,59 @@ __global__ __launch_bounds__(QWAVES * 64) void quantize_large_group_kernel(
   }
 }
 
-// W_hat[N, K] = round_once((q - z) * s): 64x64-word tiles transposed through
-// LDS so that both the qweight reads and the W_hat row writes are coalesced.
+// W_hat[N, K] = round_once((q - z) * s): tiles of 64 columns x 64 words,
+// transposed through LDS so that both the qweight reads (256-byte rows) and the
+// W_hat row writes (1 KB in bf16 / fp16) are whole lines.
+//
+// What bounds it: HBM, four fifths of the bytes being writes.  Eight waves per
+// tile, every wave's eight word loads and the tile's scales and zeros (staged
+// once, two 16-bit values in one LDS word) in flight before the barrier: with
+// four waves that fetched a scale and a zero per word from memory between the
+// writes, the 8192 x 2048 weight took 14.3 us, this 8.4 us (5.0 TB/s,
+// what a large copy reaches).  16-bit rows are stored non-temporal (9.7 us
+// cached); fp32 lanes store two 16-byte halves 32 bytes apart, where partial
+// lines made that slower (26 against 16.5 us).
 template <int ODT>
-__global__ __launch_bounds__(256) void dequantize_kernel(const int32_t* __restrict__ qw,
+__global__ __launch_bounds__(512) void dequantize_kernel(const int32_t* __restrict__ qw,
                                                          const uint16_t* __restrict__ sc,
                                                          const uint16_t* __restrict__ ze,
                                                          int64_t N, int64_t K8, int gshift,
                                                          void* __restrict__ out) {
 #pragma clang fp contract(off)
   __shared__ uint32_t tile[64][65];
-  const int t = threadIdx.x;
+  __shared__ uint32_t sz[64][65];  // [group of the tile][column]: scale | zero << 16
+  const int lane = threadIdx.x & 63;
+  const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int64_t n0 = (int64_t)blockIdx.x * 64;
   const int64_t k80 = (int64_t)blockIdx.y * 64;
-#pragma unroll 4
-  for (int i = 0; i < 16; ++i) {
-    const int kk = i * 4 + (t >> 6), nn = t & 63;
-    const int64_t k8 = k80 + kk, n = n0 + nn;
-    tile[kk][nn] = (k8 < K8 && n < N) ? (uint32_t)qw[k8 * N + n] : 0u;
+  const int64_t n = n0 + lane;
+  const int rows = (int)(K8 - k80 < 64 ? K8 - k80 : 64);  // words per column of this tile
+  uint32_t w[8];
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {
+    const int kk = i * 8 + wv;
+    w[i] = (kk < rows && n < N) ? (uint32_t)__builtin_nontemporal_load(&qw[(k80 + kk) * N + n]) : 0u;
   }
+  // groups first .. first + groups - 1 (a group size below 512 divides the tile's 512 k)
+  const int64_t first = (k80 * 8) >> gshift;
+  const int groups = (int)(((k80 + rows) * 8 - 1) >> gshift) - (int)first + 1;
+  for (int g = wv; g < groups; g += 8)
+    if (n < N) sz[g][lane] = (uint32_t)sc[(first + g) * N + n] | ((uint32_t)ze[(first + g) * N + n] << 16);
+#pragma unroll
+  for (int i = 0; i < 8; ++i) tile[i * 8 + wv][lane] = w[i];
   __syncthreads();
   const int64_t K = K8 * 8;
-#pragma unroll 2
-  for (int i = 0; i < 16; ++i) {
-    const int nn = i * 4 + (t >> 6), kk = t & 63;
-    const int64_t k8 = k80 + kk, n = n0 + nn;
-    if (k8 >= K8 || n >= N) continue;
-    const uint32_t word = tile[kk][nn];
-    const int64_t g = (k8 * 8) >> gshift;
-    const float s = half_bits_to_float(sc[g * N + n]);
-    const float z = half_bits_to_float(ze[g * N + n]);
+  const int64_t k8 = k80 + lane;
+  const int g = (int)(((k8 * 8) >> gshift) - first);
+  if (lane >= rows) return;
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {
+    const int nn = i * 8 + wv;
+    if (n0 + nn >= N) break;
+    const uint32_t word = tile[lane][nn];
+    const uint32_t c = sz[g][nn];
+    const float s = half_bits_to_float((uint16_t)(c & 0xFFFFu));
+    const float z = half_bits_to_float((uint16_t)(c >> 16));
     float v[8];
 #pragma unroll
     for (int j = 0; j < 8; ++j) {
@@ -474,7 +497,7 @@ __global__ __launch_bounds__(256) void dequantize_kernel(const int32_t* __restri
       asm volatile("" : "+v"(v[j]));
     }
     if constexpr (ODT == W4_DTYPE_FP32) {
-      float* o = reinterpret_cast<float*>(out) + n * K + k8 * 8;
+      float* o = reinterpret_cast<float*>(out) + (n0 + nn) * K + k8 * 8;
       f32x4 a, b;
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
@@ -484,13 +507,13 @@ __global__ __launch_bounds__(256) void dequantize_kernel(const int32_t* __restri
       *reinterpret_cast<f32x4*>(o) = a;
       *reinterpret_cast<f32x4*>(o + 4) = b;
     } else {
-      uint16_t* o = reinterpret_cast<uint16_t*>(out) + n * K + k8 * 8;
+      uint16_t* o = reinterpret_cast<uint16_t*>(out) + (n0 + nn) * K + k8 * 8;
       u32x4 p;
 #pragma unroll
       for (int j = 0; j < 4; ++j)
         p[j] = (uint32_t)float_to_act_bits<ODT>(v[2 * j]) |
                ((uint32_t)float_to_act_bits<ODT>(v[2 * j + 1]) << 16);
-      *reinterpret_cast<u32x4*>(o) = p;
+      __builtin_nontemporal_store(p, reinterpret_cast<u32x4*>(o));
     }
   }
 }
@@ -645,13 +668,13 @@ extern "C" int w4_dequantize(const int32_t* qweight, const uint16_t* scales, con
   hipStream_t st = static_cast<hipStream_t>(stream);
   switch (out_dtype) {
     case W4_DTYPE_BF16:
-      hipLaunchKernelGGL((w4::dequantize_kernel<W4_DTYPE_BF16>), grid, dim3(256), 0, st, qweight, scales, zeros, N, K8, gshift, out);
+      hipLaunchKernelGGL((w4::dequantize_kernel<W4_DTYPE_BF16>), grid, dim3(512), 0, st, qweight, scales, zeros, N, K8, gshift, out);
       break;
     case W4_DTYPE_FP16:
-      hipLaunchKernelGGL((w4::dequantize_kernel<W4_DTYPE_FP16>), grid, dim3(256), 0, st, qweight, scales, zeros, N, K8, gshift, out);
+      hipLaunchKernelGGL((w4::dequantize_kernel<W4_DTYPE_FP16>), grid, dim3(512), 0, st, qweight, scales, zeros, N, K8, gshift, out);
       break;
     case W4_DTYPE_FP32:
-      hipLaunchKernelGGL((w4::dequantize_kernel<W4_DTYPE_FP32>), grid, dim3(256), 0, st, qweight, scales, zeros, N, K8, gshift, out);
+      hipLaunchKernelGGL((w4::dequantize_kernel<W4_DTYPE_FP32>), grid, dim3(512), 0, st, qweight, scales, zeros, N, K8, gshift, out);
       break;
     default:
       return fail(W4_ERR_INVALID, "w4_dequantize: bad out dtype %d", out_dtype);

@@ -234,3 +234,19 @@ def test_quantize_grouped_fallbacks(case):
         for w, g, o in zip(ws, gs, outs):
             q, s, z = int4_hip.quantize_int4(w, g)
             assert torch.equal(o[0], q) and torch.equal(o[1].view(torch.int16), s.view(torch.int16))
+
+
+# tiles cut off in columns and words, groups from one word to more than a tile
+@pytest.mark.parametrize("dt", ["bf16", "fp16", "fp32"])
+@pytest.mark.parametrize("N,K,g", [(1, 8, 8), (63, 520, 8), (65, 512, 16), (64, 528, 16), (130, 1536, 512),
+                                   (7, 4096, 2048), (200, 1024, 32)])
+def test_dequantize_tile_edges(N, K, g, dt):
+    rng = np.random.default_rng(N + K)
+    qw = rng.integers(-2**31, 2**31, (K // 8, N)).astype(np.int32)
+    s = (rng.standard_normal((K // g, N)) * 0.01).astype(np.float16)
+    z = rng.integers(0, 16, (K // g, N)).astype(np.float16)
+    tdt = {**TDT, "fp32": torch.float32}[dt]
+    out = int4_hip.dequantize_int4(*(torch.from_numpy(a).to(DEV) for a in (qw, s, z)), tdt).cpu()
+    ref = int4_hip.dequantize_int4_ref(*(torch.from_numpy(a) for a in (qw, s, z)), tdt)
+    view = torch.int32 if dt == "fp32" else torch.int16
+    assert torch.equal(out.view(view), ref.view(view))
