@@ -30,80 +30,73 @@ __device__ __forceinline__ float dpp_mov(float v) {
   return __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, v), CTRL, 0xF, 0xF, true));
 }
 
+// One DPP step of a maximum and a minimum (values without NaN).  Written in
+// assembly: the compiler puts a quieting v_max_f32 x, x before each, and the
+// NaN-propagating forms have no DPP encoding, so a step took four or six
+// instructions.  s_nop 1: a DPP operand written by the instruction before
+// needs two wait states.
+#define W4_MINMAX_DPP(CTRL)                                                     \
+  asm("s_nop 1\n\t"                                                            \
+      "v_max_f32_dpp %0, %0, %0 " CTRL " row_mask:0xf bank_mask:0xf\n\t"       \
+      "v_min_f32_dpp %1, %1, %1 " CTRL " row_mask:0xf bank_mask:0xf\n\t"       \
+      "s_nop 0"                                                                 \
+      : "+v"(mx), "+v"(mn))
+
 // Maximum and minimum over aligned groups of L lanes (L a power of two up to
 // 64): DPP steps inside rows of 16 lanes (swap neighbours, swap pairs,
 // half-row mirror, row mirror), lane shuffles across rows.
 template <int L>
 __device__ __forceinline__ void group_minmax(float& mx, float& mn) {
-  if constexpr (L >= 2) {
-    mx = fmax_p(mx, dpp_mov<0xB1>(mx));  // quad_perm [1,0,3,2]
-    mn = fmin_p(mn, dpp_mov<0xB1>(mn));
-  }
-  if constexpr (L >= 4) {
-    mx = fmax_p(mx, dpp_mov<0x4E>(mx));  // quad_perm [2,3,0,1]
-    mn = fmin_p(mn, dpp_mov<0x4E>(mn));
-  }
-  if constexpr (L >= 8) {
-    mx = fmax_p(mx, dpp_mov<0x141>(mx));  // row_half_mirror
-    mn = fmin_p(mn, dpp_mov<0x141>(mn));
-  }
-  if constexpr (L >= 16) {
-    mx = fmax_p(mx, dpp_mov<0x140>(mx));  // row_mirror
-    mn = fmin_p(mn, dpp_mov<0x140>(mn));
-  }
+  if constexpr (L >= 2) W4_MINMAX_DPP("quad_perm:[1,0,3,2]");
+  if constexpr (L >= 4) W4_MINMAX_DPP("quad_perm:[2,3,0,1]");
+  if constexpr (L >= 8) W4_MINMAX_DPP("row_half_mirror");
+  if constexpr (L >= 16) W4_MINMAX_DPP("row_mirror");
   if constexpr (L >= 32) {
-    mx = fmax_p(mx, __shfl_xor(mx, 16, 64));
-    mn = fmin_p(mn, __shfl_xor(mn, 16, 64));
+    mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
+    mn = fminf(mn, __shfl_xor(mn, 16, 64));
   }
   if constexpr (L >= 64) {
-    mx = fmax_p(mx, __shfl_xor(mx, 32, 64));
-    mn = fmin_p(mn, __shfl_xor(mn, 32, 64));
+    mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+    mn = fminf(mn, __shfl_xor(mn, 32, 64));
   }
 }
+#undef W4_MINMAX_DPP
 
 struct QStats {
   float scale;  // fp16-representable (or 0/inf/NaN in degenerate groups)
   float zero;
 };
 
-// Fast form of group_stats, bit-identical to it, plus rcp(scale).
+// Fast form of group_stats, plus rcp(scale): bit-identical to it unless *bad.
 //  - scale: for x = wmax - wmin in [2^-90, 2^126], y = x * fl(1/15) followed
 //    by one fma correction with the exact residual fma(-y, 15, x) is the
 //    correctly rounded x / 15 (checked for every float in that range by
-//    tests/div15_exhaustive.c); elsewhere the IEEE division.
+//    tests/div15_exhaustive.c); every x whose scale is a positive finite fp16
+//    lies in that range, so *bad covers the rest (zero, infinite and NaN).
 //  - zero: -wmin / scale <= 22.5 (scale >= x / 15 up to the fp16 rounding,
 //    which for a subnormal scale >= 2^-24 is at most 2^-25), so with
 //    v_rcp_f32 within 1 ulp t0 = fma(-wmin, rcp(scale), 0.5) is within 6e-6
 //    of the reference's fl(fl(-wmin / scale) + 0.5) and the floors agree
-//    unless fract(t0) is within 2^-15 of 0 or 1, where, and for a zero /
-//    infinite / NaN scale, the IEEE division is used.
-__device__ __forceinline__ QStats group_stats_fast(float rmax, float rmin, float* rcp) {
+//    unless fract(t0) is within 2^-15 of 0 or 1, which sets *bad.
+// No branch: the caller redoes the rare bad groups with group_stats.
+__device__ __forceinline__ QStats group_stats_fast(float rmax, float rmin, float* rcp, bool* bad) {
 #pragma clang fp contract(off)
-  const float wmax = max_nan(rmax, 0.0f);
-  const float wmin = min_nan(rmin, 0.0f);
+  const float wmax = __builtin_elementwise_maximum(rmax, 0.0f);
+  const float wmin = __builtin_elementwise_minimum(rmin, 0.0f);
   const float x = wmax - wmin;
-  float scale;
-  if (x >= 0x1p-90f && x <= 0x1p126f) {
-    constexpr float C15 = 1.0f / 15.0f;
-    const float y = x * C15;
-    scale = __builtin_fmaf(__builtin_fmaf(-y, 15.0f, x), C15, y);
-  } else {
-    scale = x / 15.0f;
-  }
-  if (scale == 0.0f) scale = 1.0f;
-  scale = (float)(_Float16)scale;
-  const float r = __builtin_amdgcn_rcpf(scale);
+  constexpr float C15 = 1.0f / 15.0f;
+  const float y = x * C15;
+  QStats st;
+  float q = __builtin_fmaf(__builtin_fmaf(-y, 15.0f, x), C15, y);
+  asm("" : "+v"(q));  // the fp32 quotient is rounded first, then to fp16: no fused fma-and-convert
+  st.scale = (float)(_Float16)q;
+  const float r = __builtin_amdgcn_rcpf(st.scale);
   const float t0 = __builtin_fmaf(-wmin, r, 0.5f);
   const float f0 = __builtin_amdgcn_fractf(t0);
-  float zero;
-  if (scale > 0.0f && scale < __builtin_inff() && f0 >= 0x1p-15f && f0 <= 1.0f - 0x1p-15f)
-    zero = __builtin_amdgcn_fmed3f(floorf(t0), 0.0f, 15.0f);
-  else
-    zero = clamp_nan(floorf(-wmin / scale + 0.5f), 0.0f, 15.0f);
+  st.zero = __builtin_amdgcn_fmed3f(floorf(t0), 0.0f, 15.0f);
   *rcp = r;
-  QStats st;
-  st.scale = scale;
-  st.zero = zero;
+  *bad = !__builtin_amdgcn_classf(st.scale, 0x100) ||  // positive normal
+         !(__builtin_fabsf(f0 - 0.5f) <= 0.5f - 0x1p-15f);
   return st;
 }
 
@@ -138,28 +131,38 @@ __device__ __forceinline__ uint32_t quantize_pack8(const float v[8], QStats st) 
 }
 
 // Fast form of quantize_pack8 for finite weights and a finite nonzero scale
-// (group_stats' scale is then in [2^-24, 65504]).  t = w * rcp(scale) + 0.5 +
-// zero in one fma (zero is an integer in [0, 15]): v_rcp_f32 is within 1 ulp,
-// so while |w/scale| < 32, t lies within 8e-6 of the reference's
-// fl(fl(w/scale) + 0.5) + zero and both floors agree unless t is within 2^-15
-// of an integer; beyond that range both clamp to the same end (0 or 15).
-// q = trunc(med3(t, 0, 15.5)) is clamp(floor(t), 0, 15).  Returns true in
-// *near when some fract(t) is within 2^-15 of 0 or 1: the caller then repacks
-// the word with quantize_pack8.  Otherwise the word is bit-identical to
-// quantize_pack8's.
+// (group_stats' scale is then in [2^-24, 65504]).  m = 128 + t with t = w *
+// rcp(scale) + 0.5 + zero, in one fma: between 128 and 256 a float's low 16
+// bits are the fraction of t in units of 2^-16 and the bits above them its
+// integer part.  v_rcp_f32 is within 1 ulp and the fma rounds by at most half
+// a unit, so while |w / scale| < 32, t lies within one unit of the reference's
+// fl(fl(w / scale) + 0.5) + zero, and both floors agree unless the fraction is
+// within two units of 0 or 1; beyond that range, as for every t below 0.5 or
+// above 15.5, both clamp to the same end (m is clamped to 128.5 .. 143.5,
+// which gives 0 and 15 and a harmless fraction).  Returns true in *near when
+// some fraction is that close: the caller then repacks the word with
+// quantize_pack8.  Otherwise the word is bit-identical to quantize_pack8's.
+// Two elements share each 32-bit operation after the clamp (39 vector
+// instructions a word; a fract, two extremes, a conversion and a shift per
+// element were 49).
 __device__ __forceinline__ uint32_t quantize_pack8_fast(const float v[8], QStats st, float rcp, bool* near) {
-  const float c = 0.5f + st.zero;
-  uint32_t word = 0;
-  float lo = 1.0f, hi = 0.0f;
+  typedef uint16_t u16x2 __attribute__((ext_vector_type(2)));
+  const float c = 128.5f + st.zero;
+  uint32_t m[8];
 #pragma unroll
-  for (int i = 0; i < 8; ++i) {
-    const float t = __builtin_fmaf(v[i], rcp, c);
-    const float f = __builtin_amdgcn_fractf(t);
-    lo = fmin_p(lo, f);
-    hi = fmax_p(hi, f);
-    word |= (uint32_t)__builtin_amdgcn_fmed3f(t, 0.0f, 15.5f) << (4 * i);
+  for (int i = 0; i < 8; ++i)
+    m[i] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_fmed3f(__builtin_fmaf(v[i], rcp, c), 128.5f, 143.5f));
+  // 0x4300 | q of elements i (low half) and i + 4 (high half)
+  constexpr uint32_t kExp = 0x43004300u * 0x1111u;
+  uint32_t word = 0u - kExp;
+  u16x2 lo = u16x2{0xFFFF, 0xFFFF};
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    word += __builtin_amdgcn_perm(m[i + 4], m[i], 0x07060302u) << (4 * i);
+    const u16x2 f = __builtin_bit_cast(u16x2, __builtin_amdgcn_perm(m[i + 4], m[i], 0x05040100u));
+    lo = __builtin_elementwise_min(lo, (u16x2)(f + (uint16_t)2));
   }
-  *near = !(lo >= 0x1p-15f && hi <= 1.0f - 0x1p-15f);
+  *near = lo[0] < 4 || lo[1] < 4;
   return word;
 }
 
@@ -183,25 +186,8 @@ __device__ __forceinline__ uint16_t zero_bits(float z) {
   return (z != z) ? (uint16_t)0xFE00 : __builtin_bit_cast(uint16_t, (_Float16)z);
 }
 
-template <int DT, bool VEC>
-__device__ __forceinline__ void load8(const uint16_t* __restrict__ w, int64_t n, int64_t k,
-                                      int64_t swn, int64_t swk, float v[8]) {
-  if (VEC) {
-    const u32x4 p = *reinterpret_cast<const u32x4*>(w + n * swn + k);
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      v[2 * i] = act_bits_to_float((uint16_t)(p[i] & 0xFFFFu), DT);
-      v[2 * i + 1] = act_bits_to_float((uint16_t)(p[i] >> 16), DT);
-    }
-  } else {
-#pragma unroll
-    for (int i = 0; i < 8; ++i) v[i] = act_bits_to_float(w[n * swn + (k + i) * swk], DT);
-  }
-}
-
 constexpr int QROWS = 64;  // columns n per tile (= lanes, for the stores)
-constexpr int QWAVES = 4;  // waves per workgroup (two-pass kernel)
-constexpr int QSWAVES = 8;  // waves per workgroup (single-pass kernel)
+constexpr int QSWAVES = 8;  // waves per workgroup
 
 // Waves sharing one (group, 64-column) tile: 64 rows split between up to eight
 // waves, each taking whole iterations of 512 / G rows (a lone wave per tile
@@ -210,6 +196,11 @@ constexpr int quantize_waves_per_tile(int G) { return G / 8 < QSWAVES ? G / 8 : 
 
 // Single-pass kernel for G <= 512: lanes_per_row = G/8 lanes each own one
 // packed word of a row; 64/lanes_per_row rows are processed per iteration.
+// Bound by HBM (154 MB for the block of 1B-model weights at G = 128: 34.5 us =
+// 4.5 TB/s, a large copy reaches 5.1; 37.5 us before the statistics lost their
+// branches, the packing its per-element boundary tests, and the tiles' order
+// went along K, so that the workgroups running at one time read whole rows
+// instead of one column of every row: 35.5 us in the old order).
 // One weight of a quantize launch (w4_quantize_grouped puts several in one).
 struct QuantArgs {
   const uint16_t* w;
@@ -218,6 +209,8 @@ struct QuantArgs {
   uint16_t* ze;
   int64_t N, K, swn, swk;
   int64_t tiles_n, tiles_total;
+  int gshift;  // G > 512: log2(G)
+  int wpr;     // statistics pass of G > 512: waves per row
 };
 
 constexpr int kQuantMaxGrouped = 8;
@@ -228,7 +221,10 @@ struct QuantGroupedArgs {
 };
 
 // The tiles of workgroup `blk` of one weight (see quantize_small_group_kernel).
-template <int DT, int G, bool VEC>
+// GIVEN: pack pass of a group size above 512; G is then only the tile's width
+// in k, and the scale and zero point of each row are read from sc and ze, where
+// the statistics pass has put them (both are exact in fp16).
+template <int DT, int G, bool VEC, bool GIVEN = false>
 __device__ __forceinline__ void quantize_small_group_tiles(const QuantArgs& qa, int blk) {
   const uint16_t* __restrict__ w = qa.w;
   int32_t* __restrict__ qw = qa.qw;
@@ -251,8 +247,10 @@ __device__ __forceinline__ void quantize_small_group_tiles(const QuantArgs& qa, 
   // the host keeps tile counts below 2^31, so the tile index math is 32-bit
   const int t = blk * TPB + ts;
   const bool active = t < (int)tiles_total;
-  const int g = active ? t / (int)tiles_n : 0;
-  const int64_t n0 = active ? (int64_t)(t - g * (int)tiles_n) * QROWS : 0;
+  const int groups = (int)((uint32_t)K / (uint32_t)G);
+  const int tn = active ? t / groups : 0;
+  const int g = active ? t - tn * groups : 0;
+  const int64_t n0 = (int64_t)tn * QROWS;
   const int seg = lane % L;
   const int rsub = lane / L;
 
@@ -266,6 +264,16 @@ __device__ __forceinline__ void quantize_small_group_tiles(const QuantArgs& qa, 
   if (active) {
     for (int b0 = 0; b0 < IT; b0 += B) {
       u32x4 raw[B];
+      uint16_t gs[B], gz[B];
+      if constexpr (GIVEN) {
+#pragma unroll
+        for (int i = 0; i < B; ++i) {
+          const int64_t n = n0 + sub * RW + (b0 + i) * RPI + rsub;
+          const int64_t at = (((int64_t)g * G) >> qa.gshift) * N + n;
+          gs[i] = n < N ? sc[at] : (uint16_t)0x3C00;
+          gz[i] = n < N ? ze[at] : (uint16_t)0;
+        }
+      }
 #pragma unroll
       for (int i = 0; i < B; ++i) {
         const int row = sub * RW + (b0 + i) * RPI + rsub;
@@ -286,32 +294,50 @@ __device__ __forceinline__ void quantize_small_group_tiles(const QuantArgs& qa, 
                          e[4] | ((uint32_t)e[5] << 16), e[6] | ((uint32_t)e[7] << 16)};
         }
       }
-      // NaN-propagating extremes: a group without NaN takes the reciprocal
-      // packing, redone exactly for the rare flagged words; a group with a
-      // NaN (NaN extremes) takes the exact path (the sign of a zero extreme
-      // does not reach group_stats' result)
+      // every word takes the reciprocal packing and the rare flagged ones are
+      // redone exactly, a group with a NaN among them: the NaN-propagating
+      // extremes of its lanes give it NaN extremes and so a NaN scale (the
+      // sign of a zero extreme does not reach group_stats' result)
 #pragma unroll
       for (int i = 0; i < B; ++i) {
         const int row = sub * RW + (b0 + i) * RPI + rsub;
         float v[8];
         unpack_row8<DT>(raw[i], v);
-        float mx = fmax_p(v[0], v[1]), mn = fmin_p(v[0], v[1]);
-#pragma unroll
-        for (int j = 2; j < 8; ++j) {
-          mx = fmax_p(mx, v[j]);
-          mn = fmin_p(mn, v[j]);
-        }
-        group_minmax<L>(mx, mn);
         float rcp;
-        const QStats st = group_stats_fast(mx, mn, &rcp);
-        bool near;
+        bool bad, near;
+        QStats st;
+        float mx, mn;
+        if constexpr (GIVEN) {
+          st.scale = half_bits_to_float(gs[i]);
+          st.zero = half_bits_to_float(gz[i]);
+          rcp = __builtin_amdgcn_rcpf(st.scale);
+          bad = !__builtin_amdgcn_classf(st.scale, 0x100) || st.zero != st.zero;  // positive normal
+        } else {
+          mx = fmax_p(v[0], v[1]), mn = fmin_p(v[0], v[1]);
+#pragma unroll
+          for (int j = 2; j < 8; ++j) {
+            mx = fmax_p(mx, v[j]);
+            mn = fmin_p(mn, v[j]);
+          }
+          const uint64_t nan_lanes = __ballot(mx != mx);
+          group_minmax<L>(mx, mn);
+          if (nan_lanes != 0) {  // rare, wave-uniform: a NaN reaches both extremes of its whole group
+            if constexpr (L == 64)
+              mx = mn = __builtin_nanf("");
+            else if ((nan_lanes >> (lane & ~(L - 1))) & ((1ull << L) - 1))
+              mx = mn = __builtin_nanf("");
+          }
+          st = group_stats_fast(mx, mn, &rcp, &bad);
+        }
         uint32_t word = quantize_pack8_fast(v, st, rcp, &near);
-        // a NaN in the group, a word near a rounding boundary, an infinite
-        // scale (infinite weight) or a scale rounded to 0 in fp16: exact path
-        if (!(mx == mx && mn == mn) || near || !(st.scale > 0.0f && st.scale < __builtin_inff()))
+        // a word near a rounding boundary, or a group whose statistics are:
+        // zero, infinite, NaN or underflowing scale, zero point near one
+        if (near || bad) {
+          if constexpr (!GIVEN) st = group_stats(mx, mn);
           word = quantize_pack8(v, st);
+        }
         tile[ts][seg][row] = word;
-        if (seg == 0) {
+        if (!GIVEN && seg == 0) {
           st_s[ts][row] = scale_bits(st.scale);
           st_z[ts][row] = zero_bits(st.zero);
         }
@@ -328,7 +354,7 @@ __device__ __forceinline__ void quantize_small_group_tiles(const QuantArgs& qa, 
       // (3.5 % on the block against cached stores)
       for (int kk = sub; kk < L; kk += WPT)
         __builtin_nontemporal_store((int32_t)tile[ts][kk][lane], &qw[(k8_0 + kk) * N + n]);
-      if (sub == 0) {
+      if (!GIVEN && sub == 0) {
         __builtin_nontemporal_store(st_s[ts][lane], &sc[g * N + n]);
         __builtin_nontemporal_store(st_z[ts][lane], &ze[g * N + n]);
       }
@@ -353,85 +379,100 @@ __global__ __launch_bounds__(QSWAVES * 64) void quantize_small_group_grouped_ker
   quantize_small_group_tiles<DT, G, true>(ga.prob[p], b - ga.wg_start[p]);
 }
 
-// Two-pass kernel for G > 512 (per-channel G = K included): pass 1 reduces
-// min/max over the whole group row by row, pass 2 re-reads 512-wide chunks
-// and packs them.  One wave per (group, 64-column strip).
+// Group sizes above 512 (per-channel G = K included) take two passes, because a
+// group of 64 columns no longer fits a workgroup's registers: the statistics
+// of every (column, group) row, then the packing in tiles of 128 k.  The
+// second read comes mostly from the Infinity Cache.  The one-kernel form they
+// replace (a wave looping over 64 rows, twice) had N / 64 x K / G waves, 32 for
+// a per-channel 2048 x 8192 weight: the block's seven weights per channel took
+// 3122 us, these 51 us.
+constexpr int QPACK = 128;  // k per tile of the packing pass
+
+// Statistics: `wpr` waves (a power of two, chosen so that few rows still spread
+// over the chip) reduce one row of G weights, eight waves per workgroup.
 template <int DT, bool VEC>
-__global__ __launch_bounds__(QWAVES * 64) void quantize_large_group_kernel(
-    const uint16_t* __restrict__ w, int64_t N, int64_t K, int64_t swn, int64_t swk, int G,
-    int32_t* __restrict__ qw, uint16_t* __restrict__ sc, uint16_t* __restrict__ ze,
-    int64_t tiles_n, int64_t tiles_total) {
-  __shared__ uint32_t tile[QWAVES][64][QROWS + 1];
-  __shared__ float st_scale[QWAVES][QROWS];
-  __shared__ float st_zero[QWAVES][QROWS];
-
+__device__ __forceinline__ void quantize_stats_rows(const QuantArgs& qa, int blk) {
+  __shared__ float part[2][QSWAVES];
   const int lane = threadIdx.x & 63;
-  const int wv = threadIdx.x >> 6;
-  const int64_t t = (int64_t)blockIdx.x * QWAVES + wv;
-  const bool active = t < tiles_total;
-  const int64_t g = active ? t / tiles_n : 0;
-  const int64_t n0 = active ? (t % tiles_n) * QROWS : 0;
-  const int nchunks = G / 512;
-
-  if (active) {
-    for (int row = 0; row < QROWS; ++row) {
-      const int64_t n = n0 + row;
-      if (n >= N) break;
-      float mx = 0.0f, mn = 0.0f;
-      bool first = true;
-      for (int c = 0; c < nchunks; ++c) {
-        float v[8];
-        load8<DT, VEC>(w, n, g * G + c * 512 + lane * 8, swn, swk, v);
+  const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int wpr = qa.wpr, rows = QSWAVES / wpr;  // rows per workgroup
+  const int64_t G = 1ll << qa.gshift;
+  // rows of one group are adjacent columns
+  const int64_t per_group = (qa.N + rows - 1) / rows;
+  const int64_t g = blk / per_group;
+  const int64_t n0 = (blk - g * per_group) * rows;
+  const int64_t n = n0 + wv / wpr;
+  float mx = 0.f, mn = 0.f;
+  if (n < qa.N) {
+    const uint16_t* row = qa.w + n * qa.swn;
+    const int64_t step = 512ll * wpr, k0 = g * G + (wv % wpr) * 512 + lane * 8;
+    bool first = true;
+    for (int64_t k = k0; k < (g + 1) * G; k += 4 * step) {
+      u32x4 raw[4];
 #pragma unroll
-        for (int i = 0; i < 8; ++i) {
-          mx = first ? v[i] : max_nan(mx, v[i]);
-          mn = first ? v[i] : min_nan(mn, v[i]);
-          first = false;
+      for (int u = 0; u < 4; ++u) {
+        // past the group: the row's first load again, which changes no extreme
+        const int64_t ku = k + u * step < (g + 1) * G ? k + u * step : k;
+        if constexpr (VEC) {
+          raw[u] = *reinterpret_cast<const u32x4*>(row + ku);
+        } else {
+#pragma unroll
+          for (int j = 0; j < 4; ++j)
+            raw[u][j] = row[(ku + 2 * j) * qa.swk] | ((uint32_t)row[(ku + 2 * j + 1) * qa.swk] << 16);
         }
       }
 #pragma unroll
-      for (int off = 32; off > 0; off >>= 1) {
-        mx = max_nan(mx, __shfl_xor(mx, off, 64));
-        mn = min_nan(mn, __shfl_xor(mn, off, 64));
-      }
-      const QStats st = group_stats(mx, mn);
-      if (lane == 0) {
-        st_scale[wv][row] = st.scale;
-        st_zero[wv][row] = st.zero;
-      }
-    }
-  }
-  __syncthreads();
-  if (active) {
-    const int64_t n = n0 + lane;
-    if (n < N) {
-      sc[g * N + n] = scale_bits(st_scale[wv][lane]);
-      ze[g * N + n] = zero_bits(st_zero[wv][lane]);
-    }
-  }
-  for (int c = 0; c < nchunks; ++c) {
-    if (active) {
-      for (int row = 0; row < QROWS; ++row) {
-        const int64_t n = n0 + row;
-        if (n >= N) break;
+      for (int u = 0; u < 4; ++u) {
         float v[8];
-        load8<DT, VEC>(w, n, g * G + c * 512 + lane * 8, swn, swk, v);
-        QStats st;
-        st.scale = st_scale[wv][row];
-        st.zero = st_zero[wv][row];
-        tile[wv][lane][row] = quantize_pack8(v, st);
+        unpack_row8<DT>(raw[u], v);
+        if (first) mx = mn = v[0];
+        first = false;
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+          mx = fmax_p(mx, v[j]);
+          mn = fmin_p(mn, v[j]);
+        }
       }
     }
-    __syncthreads();
-    if (active) {
-      const int64_t n = n0 + lane;
-      if (n < N) {
-        const int64_t k8_0 = g * (G / 8) + (int64_t)c * 64;
-        for (int kk = 0; kk < 64; ++kk) qw[(k8_0 + kk) * N + n] = (int32_t)tile[wv][kk][lane];
-      }
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) {
+      mx = fmax_p(mx, __shfl_xor(mx, off, 64));
+      mn = fmin_p(mn, __shfl_xor(mn, off, 64));
     }
-    __syncthreads();
   }
+  if (lane == 0) part[0][wv] = mx, part[1][wv] = mn;
+  __syncthreads();
+  const int r = threadIdx.x;
+  if (r < rows && n0 + r < qa.N) {
+    float a = part[0][r * wpr], b = part[1][r * wpr];
+    for (int w = 1; w < wpr; ++w) {
+      a = fmax_p(a, part[0][r * wpr + w]);
+      b = fmin_p(b, part[1][r * wpr + w]);
+    }
+    const QStats st = group_stats(a, b);
+    qa.sc[g * qa.N + n0 + r] = scale_bits(st.scale);
+    qa.ze[g * qa.N + n0 + r] = zero_bits(st.zero);
+  }
+}
+
+template <int DT, bool VEC>
+__global__ __launch_bounds__(QSWAVES * 64) void quantize_stats_kernel(QuantGroupedArgs ga) {
+  const int b = blockIdx.x;
+  int p = 0;
+#pragma unroll
+  for (int i = 1; i < kQuantMaxGrouped; ++i)
+    if (i < ga.count && b >= ga.wg_start[i]) p = i;
+  quantize_stats_rows<DT, VEC>(ga.prob[p], b - ga.wg_start[p]);
+}
+
+template <int DT, bool VEC>
+__global__ __launch_bounds__(QSWAVES * 64) void quantize_pack_kernel(QuantGroupedArgs ga) {
+  const int b = blockIdx.x;
+  int p = 0;
+#pragma unroll
+  for (int i = 1; i < kQuantMaxGrouped; ++i)
+    if (i < ga.count && b >= ga.wg_start[i]) p = i;
+  quantize_small_group_tiles<DT, QPACK, VEC, true>(ga.prob[p], b - ga.wg_start[p]);
 }
 
 // W_hat[N, K] = round_once((q - z) * s): tiles of 64 columns x 64 words,
@@ -522,16 +563,50 @@ __global__ __launch_bounds__(512) void dequantize_kernel(const int32_t* __restri
 
 using namespace w4host;
 
+// Both passes of `count` weights with group sizes above 512 (gshift set).
+template <int DT, bool VEC>
+static void launch_large(w4::QuantGroupedArgs ga, int count, hipStream_t st) {
+  // waves per row: eight, four, ... while there are fewer rows than give every
+  // CU (256) two workgroups, and at least 512 weights (a load per lane) each
+  int64_t rows = 0;
+  for (int i = 0; i < count; ++i) rows += ga.prob[i].N * (ga.prob[i].K >> ga.prob[i].gshift);
+  int wpr = 1;
+  while (wpr < w4::QSWAVES && rows * wpr * 2 <= 512 * w4::QSWAVES) wpr *= 2;
+  int64_t wgs = 0, packs = 0;
+  w4::QuantGroupedArgs gp = ga;
+  for (int i = 0; i < count; ++i) {
+    w4::QuantArgs& a = ga.prob[i];
+    a.wpr = wpr;
+    while (a.wpr > 1 && 512ll * a.wpr > (1ll << a.gshift)) a.wpr /= 2;
+    const int64_t per_wg = w4::QSWAVES / a.wpr;
+    ga.wg_start[i] = (int)wgs;
+    wgs += (a.N + per_wg - 1) / per_wg * (a.K >> a.gshift);
+    gp.wg_start[i] = (int)packs;
+    const int64_t tpb = w4::QSWAVES / w4::quantize_waves_per_tile(w4::QPACK);
+    packs += (a.tiles_total + tpb - 1) / tpb;
+  }
+  for (int i = count; i <= w4::kQuantMaxGrouped; ++i) ga.wg_start[i] = (int)wgs, gp.wg_start[i] = (int)packs;
+  ga.count = gp.count = count;
+  const dim3 block(w4::QSWAVES * 64);
+  hipLaunchKernelGGL((w4::quantize_stats_kernel<DT, VEC>), dim3((unsigned)wgs), block, 0, st, ga);
+  hipLaunchKernelGGL((w4::quantize_pack_kernel<DT, VEC>), dim3((unsigned)packs), block, 0, st, gp);
+}
+
 template <int DT, bool VEC>
 static void launch_quantize(const uint16_t* w, int64_t N, int64_t K, int64_t swn, int64_t swk,
                             int G, int32_t* qw, uint16_t* sc, uint16_t* ze, hipStream_t st) {
   const int64_t tiles_n = (N + w4::QROWS - 1) / w4::QROWS;
+  if (G > 512) {
+    w4::QuantGroupedArgs ga{};
+    ga.prob[0] = w4::QuantArgs{w, qw, sc, ze, N, K, swn, swk, tiles_n, tiles_n * (K / w4::QPACK), ilog2(G), 1};
+    launch_large<DT, VEC>(ga, 1, st);
+    return;
+  }
   const int64_t tiles_total = tiles_n * (K / G);
-  const bool small = G <= 512;
-  const int64_t tpb = small ? w4::QSWAVES / w4::quantize_waves_per_tile(G) : w4::QWAVES;
+  const int64_t tpb = w4::QSWAVES / w4::quantize_waves_per_tile(G);
   const dim3 grid((unsigned)((tiles_total + tpb - 1) / tpb));
-  const dim3 block((small ? w4::QSWAVES : w4::QWAVES) * 64);
-  const w4::QuantArgs qa{w, qw, sc, ze, N, K, swn, swk, tiles_n, tiles_total};
+  const dim3 block(w4::QSWAVES * 64);
+  const w4::QuantArgs qa{w, qw, sc, ze, N, K, swn, swk, tiles_n, tiles_total, 0, 1};
 #define W4_QS(GG)                                                                                  \
   case GG:                                                                                         \
     hipLaunchKernelGGL((w4::quantize_small_group_kernel<DT, GG, VEC>), grid, block, 0, st, qa); \
@@ -548,8 +623,6 @@ static void launch_quantize(const uint16_t* w, int64_t N, int64_t K, int64_t swn
       break;
   }
 #undef W4_QS
-  hipLaunchKernelGGL((w4::quantize_large_group_kernel<DT, VEC>), grid, block, 0, st, w, N, K, swn,
-                     swk, G, qw, sc, ze, tiles_n, tiles_total);
 }
 
 extern "C" int w4_quantize(const void* w, int w_dtype, int64_t N, int64_t K, int64_t stride_wn,
@@ -567,7 +640,8 @@ extern "C" int w4_quantize(const void* w, int w_dtype, int64_t N, int64_t K, int
   if (G > (int64_t)1 << 30) return fail(W4_ERR_UNSUPPORTED, "w4_quantize: group_size too large");
   if (N == 0) return W4_OK;
   if (!w || !qweight || !scales || !zeros) return fail(W4_ERR_INVALID, "w4_quantize: null pointer");
-  if (((N + 63) / 64) * (K / G) >= (int64_t)1 << 31)
+  // (the tiles of the kernel that runs, and the rows of its statistics pass)
+  if (((N + 63) / 64) * (K / (G > 512 ? w4::QPACK : G)) >= (int64_t)1 << 31 || (G > 512 && N * (K / G) >= (int64_t)1 << 31))
     return fail(W4_ERR_UNSUPPORTED, "w4_quantize: %lld x %lld weight has too many tiles", (long long)N,
                 (long long)K);
   const uint16_t* wp = static_cast<const uint16_t*>(w);
@@ -611,13 +685,15 @@ extern "C" int w4_quantize_grouped(const w4_quantize_problem* problems, int coun
       return fail(W4_ERR_INVALID, "w4_quantize_grouped: null pointer in problem %d", i);
     const bool vec = q.stride_wk == 1 && (q.stride_wn % 8) == 0 && ((uintptr_t)q.w % 16) == 0 &&
                      ((q.N - 1) * q.stride_wn + q.K) * 2 < (1LL << 31) && ((q.N + 63) / 64) * (q.K / G) < (1LL << 30);
-    one_launch = one_launch && q.N > 0 && vec && G <= 512 && (G0 < 0 || G == G0);
+    // all of one group size up to 512, or all above it (each its own: -1 is K)
+    one_launch = one_launch && q.N > 0 && vec && (G0 < 0 || G == G0 || (G > 512 && G0 > 512));
     G0 = G;
     if (!one_launch) continue;
-    const int64_t tiles_n = (q.N + w4::QROWS - 1) / w4::QROWS, tiles_total = tiles_n * (q.K / G);
-    const int64_t tpb = w4::QSWAVES / w4::quantize_waves_per_tile((int)G);
+    const int64_t tile_k = G > 512 ? w4::QPACK : G;
+    const int64_t tiles_n = (q.N + w4::QROWS - 1) / w4::QROWS, tiles_total = tiles_n * (q.K / tile_k);
+    const int64_t tpb = w4::QSWAVES / w4::quantize_waves_per_tile((int)tile_k);
     ga.prob[i] = w4::QuantArgs{static_cast<const uint16_t*>(q.w), q.qweight, q.scales, q.zeros, q.N, q.K,
-                               q.stride_wn, q.stride_wk, tiles_n, tiles_total};
+                               q.stride_wn, q.stride_wk, tiles_n, tiles_total, ilog2(G), 1};
     ga.wg_start[i] = (int)wgs;
     wgs += (tiles_total + tpb - 1) / tpb;
     one_launch = wgs < (1LL << 30);
@@ -631,6 +707,11 @@ extern "C" int w4_quantize_grouped(const w4_quantize_problem* problems, int coun
       if (rc != W4_OK) return rc;
     }
     return W4_OK;
+  }
+  if (G0 > 512) {
+    if (w_dtype == W4_DTYPE_BF16) launch_large<W4_DTYPE_BF16, true>(ga, count, st);
+    else launch_large<W4_DTYPE_FP16, true>(ga, count, st);
+    return check_launch("w4_quantize_grouped");
   }
   for (int i = count; i <= w4::kQuantMaxGrouped; ++i) ga.wg_start[i] = (int)wgs;
   ga.count = count;

@@ -236,6 +236,42 @@ def test_quantize_grouped_fallbacks(case):
             assert torch.equal(o[0], q) and torch.equal(o[1].view(torch.int16), s.view(torch.int16))
 
 
+# group sizes above 512: a statistics pass (one to eight waves per row: few or
+# many rows, groups of two up to 32 loads per lane) and a packing pass, on dense
+# and strided rows, NaN and infinite weights included; grouped with a group
+# size per weight (-1 is each weight's K)
+@pytest.mark.parametrize("dt", ["bf16", "fp16"])
+@pytest.mark.parametrize("N,K,g,layout", [
+    (1, 1024, 1024, "dense"), (3, 16384, -1, "dense"), (70, 8192, 2048, "dense"), (2048, 2048, -1, "dense"),
+    (65, 2048, 1024, "transposed"), (9, 4096, -1, "unaligned"), (4100, 1024, -1, "dense")])
+def test_quantize_large_groups(dt, N, K, g, layout):
+    print(f"[quantize large] {N}x{K} G={g} {dt} {layout}", flush=True)
+    w = randn((N, K), seed=N + K, sigma=0.02, dtype=TDT[dt])
+    if N > 8:
+        w[2, 7], w[5, K - 1], w[6, 600] = float("nan"), float("inf"), float("-inf")
+        w[7] = 0
+    dev = w.to(DEV)
+    if layout == "transposed":
+        dev = dev.t().contiguous().t()
+    elif layout == "unaligned":
+        flat = torch.empty(N * (K + 3) + 1, dtype=dev.dtype, device=DEV)
+        view = flat[1:].view(N, K + 3)[:, :K]
+        view.copy_(dev)
+        dev = view
+    qw, s, z = _quantize_np(dev, g)
+    rq, rs, rz = O.quantize_int4(bits_of(w), dt, g)
+    np.testing.assert_array_equal(qw, rq)
+    np.testing.assert_array_equal(s, rs)
+    np.testing.assert_array_equal(z, rz)
+
+
+def test_quantize_grouped_large_groups_match_lone():
+    ws = [randn(s, seed=970 + i, sigma=0.02).to(DEV) for i, s in enumerate([(300, 2048), (40, 8192), (1, 1024)])]
+    for w, o in zip(ws, int4_hip.quantize_int4_grouped(ws, -1)):
+        for a, b in zip(o, int4_hip.quantize_int4(w, -1)):
+            assert torch.equal(a.view(torch.int16), b.view(torch.int16))
+
+
 # tiles cut off in columns and words, groups from one word to more than a tile
 @pytest.mark.parametrize("dt", ["bf16", "fp16", "fp32"])
 @pytest.mark.parametrize("N,K,g", [(1, 8, 8), (63, 520, 8), (65, 512, 16), (64, 528, 16), (130, 1536, 512),
