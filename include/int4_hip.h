@@ -224,6 +224,26 @@ int w4a16_gemm_noalloc(const void* x, int x_dtype, int64_t M, int64_t N, int64_t
                        int group_size, void* y, int64_t ldy, void* stream);
 
 /*
+ * One-row products of a decoder layer with the operation in front of them done
+ * in the same launch:
+ *   w4a16_decode_norm: y_i = rmsnorm(x + delta) * W_hat_i^T, all problems on the
+ *   same x row (K values; `delta` may be NULL), norm `weight` and `eps` as in
+ *   w4_rmsnorm, x + delta written to `sum` (may be NULL; neither x nor delta);
+ *   w4a16_decode_silu: y = (silu(x) * up) @ W_hat^T.
+ * The activations are rounded to the dtype as w4_rmsnorm / w4_silu_mul round
+ * them.  Workspace: w4a16_grouped_workspace_bytes(problems, count, 1).
+ * W4_ERR_UNSUPPORTED with nothing enqueued where no such launch exists (group
+ * sizes below 32, N % 8 != 0, misaligned operands, a norm over more than 8192
+ * values, a K that one round of loads does not hold): use the separate calls.
+ * No counterpart in the reference.
+ */
+int w4a16_decode_norm(const w4a16_problem* problems, int count, int x_dtype, const void* delta,
+                      const void* weight, float eps, void* sum, void* workspace, size_t workspace_bytes,
+                      void* stream);
+int w4a16_decode_silu(const w4a16_problem* problem, int x_dtype, const void* up, void* workspace,
+                      size_t workspace_bytes, void* stream);
+
+/*
  * Attention of one decode step of a Llama-style layer, in one launch: rotary
  * embedding of q and k (cos, sin: the position's rows [head_dim / 2]; fp32
  * products rounded separately), the new key and value written to the fp32

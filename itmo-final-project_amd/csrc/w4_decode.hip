@@ -121,6 +121,19 @@ struct DecGroupedArgs {
   int count;
 };
 
+// What a one-row launch computes its activations from (dec_kernel_pro): the
+// operation in front of the linears of a decoder layer, done while the weights
+// are on their way instead of in a launch of its own.
+constexpr int kProNone = 0;
+constexpr int kProNorm = 1;  // rmsnorm(x + a) * w; x + a (16-bit) is written to sum
+constexpr int kProSilu = 2;  // silu(x) * a
+struct DecPrologue {
+  const uint16_t* a;  // kProNorm: may be null (no residual addition)
+  const uint16_t* w;
+  uint16_t* sum;
+  float eps;
+};
+
 constexpr int kDecWaves = 8;
 constexpr int kDecThreads = 64 * kDecWaves;
 constexpr uint32_t kDecOOB = 0x80000000u;  // offset the buffer range check rejects
@@ -189,6 +202,29 @@ __device__ __forceinline__ u32x4 dec_perm_x(u32x4 v) {
   r[2] = __builtin_amdgcn_perm(v[3], v[1], 0x05040100u);
   r[3] = __builtin_amdgcn_perm(v[3], v[1], 0x07060302u);
   return r;
+}
+
+// Eight consecutive 16-bit values as floats, and back.
+template <int DT>
+__device__ __forceinline__ void dec_unpack8(const u32x4 r, float v[8]) {
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    v[2 * j] = act_bits_to_float((uint16_t)(r[j] & 0xFFFFu), DT);
+    v[2 * j + 1] = act_bits_to_float((uint16_t)(r[j] >> 16), DT);
+  }
+}
+template <int DT>
+__device__ __forceinline__ u32x4 dec_pack8(const float v[8]) {
+  u32x4 r;
+#pragma unroll
+  for (int j = 0; j < 4; ++j)
+    r[j] = (uint32_t)float_to_act_bits<DT>(v[2 * j]) | ((uint32_t)float_to_act_bits<DT>(v[2 * j + 1]) << 16);
+  return r;
+}
+
+template <int CTRL>
+__device__ __forceinline__ uint32_t dec_dpp(uint32_t v) {
+  return (uint32_t)__builtin_amdgcn_mov_dpp((int)v, CTRL, 0xF, 0xF, true);
 }
 
 template <int VEC>
@@ -547,8 +583,7 @@ constexpr int kMaxRowSlices = 8;  // 16-row slices of one problem (M <= 128)
 // column nl at red[w * RSTR + nl]
 template <int DT, int TW, int RSTR>
 __device__ __forceinline__ void dec_split_finish(const DecArgs& a, const float* red, int ct, int kp, int ks, int n0,
-                                                 int lane) {
-  typedef DecNum<DT> Num;
+                                                 int lane, float factor) {
   static_assert(TW % 64 == 0, "split tiles: whole lanes per column");
   constexpr int C = TW / 64;
   unsigned long long* words = a.pair + (int64_t)ct * (ks - 1) * TW;
@@ -561,7 +596,7 @@ __device__ __forceinline__ void dec_split_finish(const DecArgs& a, const float* 
     float v = 0.0f;
 #pragma unroll
     for (int w = 0; w < kOneWaves; ++w) v += pv[w];
-    v *= 1.0f / Num::QS;
+    v *= factor;
     bool live = true;
     int base = 0;
     for (int width = ks >> 1, node = kp >> 1; width >= 1; base += width, width >>= 1, node >>= 1) {
@@ -587,8 +622,12 @@ __device__ __forceinline__ void dec_split_finish(const DecArgs& a, const float* 
 
 // WV: waves of the workgroup.  sl0: the 16-row slice of the problem this
 // workgroup computes (the eight-wave sixteen-row kernel; otherwise 0)
-template <int DT, int TW, int GSI, int NL, int D, int MR, int WV = kOneWaves>
-__device__ __forceinline__ void dec_tile_one(const DecArgs& a, int tile, uint8_t* lds, int sl0 = 0) {
+// PRO: kPro* (one row, single-round tilings); pro_red: 16 floats of LDS of its
+// own for the norm's sum of squares
+template <int DT, int TW, int GSI, int NL, int D, int MR, int WV = kOneWaves, int PRO = kProNone>
+__device__ __forceinline__ void dec_tile_one(const DecArgs& a, int tile, uint8_t* lds, int sl0 = 0,
+                                             const DecPrologue* pro = nullptr, float* pro_red = nullptr) {
+  static_assert(PRO == kProNone || (MR == 1 && D == 1), "prologue: one row, one round");
   typedef typename Act<DT>::frag F;
   typedef DecNum<DT> Num;
   constexpr int RPS = TW == 128 ? 2 : TW == 64 ? 4 : 8;  // qweight rows per load step
@@ -709,14 +748,25 @@ __device__ __forceinline__ void dec_tile_one(const DecArgs& a, int tile, uint8_t
   struct Round {
     u32x4 w[NL];
     u32x4 x[XLD], s, z;
+    u32x4 pa[PRO != kProNone ? XLD : 1], pw[PRO == kProNorm ? XLD : 1];
   };
+  const bool pro_a = PRO == kProSilu || (PRO == kProNorm && pro->a != nullptr);
+  const __amdgpu_buffer_rsrc_t rpa = __builtin_amdgcn_make_buffer_rsrc(
+      (void*)(PRO != kProNone ? pro->a : nullptr), (short)0, pro_a ? (int)a.x_bytes : 0, kDecBufFlags);
+  const __amdgpu_buffer_rsrc_t rpw = __builtin_amdgcn_make_buffer_rsrc(
+      (void*)(PRO == kProNorm ? pro->w : nullptr), (short)0, PRO == kProNorm ? (int)a.x_bytes : 0, kDecBufFlags);
   // Issue order = order of use: activations, scales, zeros, weights.
   auto load_round = [&](Round& r, int sb) {
     const uint32_t oob = sb < we ? 0u : kDecOOB;  // scalar
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int j = 0; j < XLD; ++j)
-      r.x[j] = __builtin_amdgcn_raw_buffer_load_b128(rx, (x_lane[j] + (uint32_t)sb * RPS * 16u) | oob, 0, 0);
+    {
+      const uint32_t xo = (x_lane[j] + (uint32_t)sb * RPS * 16u) | oob;
+      r.x[j] = __builtin_amdgcn_raw_buffer_load_b128(rx, xo, 0, 0);
+      if constexpr (PRO != kProNone) r.pa[j] = __builtin_amdgcn_raw_buffer_load_b128(rpa, xo, 0, 0);
+      if constexpr (PRO == kProNorm) r.pw[j] = __builtin_amdgcn_raw_buffer_load_b128(rpw, xo, 0, 0);
+    }
     const uint32_t g0 = (uint32_t)((sb * SK) >> a.gshift);
     const uint32_t so = (g0 * (uint32_t)N * 2u + sz_lane) | sz_oob | oob;
     r.s = __builtin_amdgcn_raw_buffer_load_b128(rs, so, 0, kDecWeightAux);
@@ -733,13 +783,58 @@ __device__ __forceinline__ void dec_tile_one(const DecArgs& a, int tile, uint8_t
   f32x4 xs;
   float tot[4][RE];
 
+  // The prologue's activations of one 16-byte chunk, rounded to 16 bits once
+  // (the residual sum before it, as the separate kernel does).  The norm's
+  // factor 1 / rms needs the whole row, so it is left out here and multiplies
+  // the finished sums: no wave waits for another before its products.  bf16 has
+  // the range for that; fp16 activations are scaled by a power of two per wave
+  // (`unscale` is its inverse) that puts the wave's largest at 2^10, which keeps
+  // every bit that rounding the normalized values would.
+  float unscale = 1.0f;
+  auto pro_apply = [&](const u32x4 xv, const u32x4 av, const u32x4 pw) {
+    float x[8], b[8];
+    dec_unpack8<DT>(xv, x);
+    dec_unpack8<DT>(av, b);
+    if constexpr (PRO == kProNorm) {
+#pragma unroll
+      for (int j = 0; j < 8; ++j) x[j] += b[j];
+      dec_unpack8<DT>(dec_pack8<DT>(x), x);
+      dec_unpack8<DT>(pw, b);
+#pragma unroll
+      for (int j = 0; j < 8; ++j) x[j] *= b[j];
+      if constexpr (DT == W4_DTYPE_FP16) {
+        uint32_t top = 0;
+#pragma unroll
+        for (int j = 0; j < 8; ++j) top = max(top, __builtin_bit_cast(uint32_t, x[j]) & 0x7FFFFFFFu);
+        top = max(top, dec_dpp<0xB1>(top));
+        top = max(top, dec_dpp<0x4E>(top));
+        top = max(top, dec_dpp<0x141>(top));
+        top = max(top, dec_dpp<0x140>(top));
+        const uint32_t all = max(max(__builtin_amdgcn_readlane(top, 0), __builtin_amdgcn_readlane(top, 16)),
+                                 max(__builtin_amdgcn_readlane(top, 32), __builtin_amdgcn_readlane(top, 48)));
+        const uint32_t e = min(max(all >> 23, 20u), 240u);  // a zero, infinite or NaN slice: any scale
+        const float scale = __builtin_bit_cast(float, (264u - e) << 23);
+        unscale = __builtin_bit_cast(float, (e - 10u) << 23);
+#pragma unroll
+        for (int j = 0; j < 8; ++j) x[j] *= scale;
+      }
+    } else {
+#pragma unroll
+      for (int j = 0; j < 8; ++j) x[j] = x[j] / (1.0f + __expf(-x[j])) * b[j];
+    }
+    return dec_pack8<DT>(x);
+  };
+
   // stage the round's activations (permuted), scales and zeros
   auto stage_round = [&](const Round& r) {
 #pragma unroll
     for (int j = 0; j < XLD; ++j) {
       const int f = 64 * j + lane, m = f / XE, e = f % XE;
+      u32x4 xv = r.x[j];
+      if constexpr (PRO == kProNorm) xv = pro_apply(xv, r.pa[j], r.pw[j]);
+      if constexpr (PRO == kProSilu) xv = pro_apply(xv, r.pa[j], xv);
       if (f < MR * XE)
-        *reinterpret_cast<u32x4*>(x_lds + xpos(m, (e / RPS) * SLOTS + e % RPS)) = dec_perm_x(r.x[j]);
+        *reinterpret_cast<u32x4*>(x_lds + xpos(m, (e / RPS) * SLOTS + e % RPS)) = dec_perm_x(xv);
     }
     *reinterpret_cast<u32x4*>(s_lds + lane * 16) = r.s;
     *reinterpret_cast<u32x4*>(z_lds + lane * 16) = r.z;
@@ -803,6 +898,16 @@ __device__ __forceinline__ void dec_tile_one(const DecArgs& a, int tile, uint8_t
   // them; the last part to arrive stores the sum).  Slice sl0 has its own
   // rows of y, arrival counters and partial tiles.
   const int sl = sl0;
+  // what multiplies the finished sums (after the reduction's barrier)
+  auto out_factor = [&]() {
+    if constexpr (PRO == kProNorm) {
+      float t = 0.f;
+#pragma unroll
+      for (int w = 0; w < WV; ++w) t += pro_red[w];
+      return (1.0f / Num::QS) * __builtin_amdgcn_rsqf(t / (float)K + pro->eps);
+    }
+    return 1.0f / Num::QS;
+  };
   auto finish = [&]() {
     uint16_t* const y = a.y + (int64_t)(16 * sl) * a.ldy;
     if (owner) {
@@ -872,7 +977,7 @@ __device__ __forceinline__ void dec_tile_one(const DecArgs& a, int tile, uint8_t
     }
     if constexpr (MR == 1 && TW % 64 == 0) {
       if (ks > 1) {
-        if (wv == 0) dec_split_finish<DT, TW, RSTR>(a, red, ct, kp, ks, n0, lane);
+        if (wv == 0) dec_split_finish<DT, TW, RSTR>(a, red, ct, kp, ks, n0, lane, out_factor());
         return;
       }
     }
@@ -933,6 +1038,7 @@ __device__ __forceinline__ void dec_tile_one(const DecArgs& a, int tile, uint8_t
         return;
       }
     }
+    const float factor = out_factor();
     for (int el = tid; el < MR * TW; el += WV * 64) {
       const int m = el / TW, nl = el - m * TW;
       const int n = n0 + nl;
@@ -955,7 +1061,7 @@ __device__ __forceinline__ void dec_tile_one(const DecArgs& a, int tile, uint8_t
         float v = 0.0f;
 #pragma unroll
         for (int i = 0; i < NPART; ++i) v += pv[i];
-        y[(int64_t)m * a.ldy + n] = float_to_act_bits<DT>(v * (1.0f / Num::QS));
+        y[(int64_t)m * a.ldy + n] = float_to_act_bits<DT>(v * factor);
       }
     }
   };
@@ -963,7 +1069,41 @@ __device__ __forceinline__ void dec_tile_one(const DecArgs& a, int tile, uint8_t
   if constexpr (D == 1) {
     // the host picks D == 1 only when a wave's run fits in one round
     clear_tot();
-    if (wb < we) {
+    if constexpr (PRO == kProNorm) {
+      // The row's sum of squares, one 16-byte chunk per thread (K <= 8192): its
+      // loads go first, its result is needed after the reduction's barrier.
+      const bool sums = wv * 512 < K;
+      u32x4 sx, sa;
+      if (sums) {
+        sx = __builtin_amdgcn_raw_buffer_load_b128(rx, (uint32_t)tid * 16u, 0, 0);
+        sa = __builtin_amdgcn_raw_buffer_load_b128(rpa, (uint32_t)tid * 16u, 0, 0);
+      }
+      if (wb < we) {
+        Round r;
+        load_round(r, wb);
+        stage_round(r);
+        compute_round(r, wb);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) tot[j][0] *= unscale;
+      }
+      float sq = 0.f;
+      if (sums) {
+        float v[8], d[8];
+        dec_unpack8<DT>(sx, v);
+        dec_unpack8<DT>(sa, d);
+#pragma unroll
+        for (int j = 0; j < 8; ++j) v[j] += d[j];
+        const u32x4 sum = dec_pack8<DT>(v);
+        dec_unpack8<DT>(sum, v);
+#pragma unroll
+        for (int j = 0; j < 8; ++j) sq = __builtin_fmaf(v[j], v[j], sq);
+#pragma unroll
+        for (int o = 32; o > 0; o >>= 1) sq += __shfl_xor(sq, o, 64);
+        if (blockIdx.x == 0 && pro->sum != nullptr && tid * 8 < K)
+          *reinterpret_cast<u32x4*>(pro->sum + tid * 8) = sum;
+      }
+      if (lane == 0) pro_red[wv] = sq;
+    } else if (wb < we) {
       Round r;
       load_round(r, wb);
       stage_round(r);
@@ -1026,6 +1166,37 @@ __global__ __launch_bounds__(kOneThreads) void dec_kernel_one(DecGroupedArgs g) 
       case kCfgT64: dec_tile_one<DT, 64, G64, 8, 1, MR>(a, tile, lds); break;
       default: dec_tile_one<DT, 32, G32, 8, 1, MR>(a, tile, lds); break;
     }
+  }
+}
+
+// One row, activations from a prologue (DecPrologue); the host gives it
+// single-round tilings only.  Doing the norm or the gated activation in every
+// workgroup costs a few hundred vector instructions that run while the weights
+// are in flight; as launches of their own they are a launch and a trip to
+// memory each.  A decode step of the 1B model (fp16, three such launches less
+// per layer) 730 -> 632 us: the gated activation adds 0.2 us to down_proj's 6.6,
+// the norm 0.2 .. 0.6 us to gate/up's 6.6 and q/k/v's 4.8.  With the norm's
+// factor applied to the activations every wave waited for the row's sum before
+// its products, 2.2 us each.
+template <int DT, int GC, int PRO>
+__global__ __launch_bounds__(kOneThreads) void dec_kernel_pro(DecGroupedArgs g, DecPrologue pro) {
+  __shared__ __attribute__((aligned(16))) float dec_smem[one_lds(1) / 4];
+  __shared__ float pro_red[kOneWaves];
+  const int t = blockIdx.x;
+  int p = 0;
+#pragma unroll
+  for (int i = 1; i < W4_MAX_GROUPED; ++i)
+    if (i < g.count && t >= g.wg_start[i]) p = i;
+  const DecArgs& a = g.prob[p];
+  const int tile = t - g.wg_start[p];
+  uint8_t* lds = reinterpret_cast<uint8_t*>(dec_smem);
+  constexpr int G128 = 2 << GC;
+  constexpr int G64 = 1 << GC;
+  constexpr int G32 = GC >= 1 ? (1 << (GC - 1)) : 1;
+  switch (a.cfg) {
+    case kCfgT128: dec_tile_one<DT, 128, G128, 8, 1, 1, kOneWaves, PRO>(a, tile, lds, 0, &pro, pro_red); break;
+    case kCfgT64: dec_tile_one<DT, 64, G64, 8, 1, 1, kOneWaves, PRO>(a, tile, lds, 0, &pro, pro_red); break;
+    default: dec_tile_one<DT, 32, G32, 8, 1, 1, kOneWaves, PRO>(a, tile, lds, 0, &pro, pro_red); break;
   }
 }
 
@@ -1506,6 +1677,58 @@ int w4_decode_launch(const w4a16_problem* problems, const int64_t* sxm, const in
     dec_launch<W4_DTYPE_BF16>(dp, M, st);
   else
     dec_launch<W4_DTYPE_FP16>(dp, M, st);
+  return check_launch("w4a16 decode");
+}
+
+namespace {
+
+template <int DT, int PRO>
+void dec_launch_pro(const DecPlan& dp, const w4::DecPrologue& pro, hipStream_t st) {
+  const dim3 grid((unsigned)dp.wgs), block(w4::kOneThreads);
+  switch (dp.gs) {
+    case 0: hipLaunchKernelGGL((w4::dec_kernel_pro<DT, 0, PRO>), grid, block, 0, st, dp.g, pro); break;
+    case 1: hipLaunchKernelGGL((w4::dec_kernel_pro<DT, 1, PRO>), grid, block, 0, st, dp.g, pro); break;
+    case 2: hipLaunchKernelGGL((w4::dec_kernel_pro<DT, 2, PRO>), grid, block, 0, st, dp.g, pro); break;
+    case 3: hipLaunchKernelGGL((w4::dec_kernel_pro<DT, 3, PRO>), grid, block, 0, st, dp.g, pro); break;
+    default: hipLaunchKernelGGL((w4::dec_kernel_pro<DT, 4, PRO>), grid, block, 0, st, dp.g, pro); break;
+  }
+}
+
+}  // namespace
+
+// One-row launch with a prologue; every problem has the same x pointer and K
+// (pro_kind kProNorm) or there is one problem (kProSilu).  Returns
+// W4_ERR_UNSUPPORTED, with nothing launched and no error message, when the
+// problems do not take the one-workgroup-per-CU kernel's single-round tilings
+// (or, kProNorm, K > 8192: one chunk per thread holds the row).
+int w4_decode_pro_launch(const w4a16_problem* problems, int count, int x_dtype, int pro_kind, const void* a,
+                         const void* w, float eps, void* sum, unsigned* counters, hipStream_t st) {
+  int64_t sxm[W4_MAX_GROUPED];
+  for (int i = 0; i < count; ++i) sxm[i] = problems[i].K;
+  DecPlan dp;
+  if (!dec_plan_final(problems, sxm, nullptr, count, 1, dp, nullptr) || !dp.cu_tiles) return W4_ERR_UNSUPPORTED;
+  if (pro_kind == w4::kProNorm && problems[0].K > 8192) return W4_ERR_UNSUPPORTED;
+  for (int s = 0; s < count; ++s)
+    if (dp.g.prob[s].cfg == w4::kCfgT64Ring || dp.g.prob[s].cfg == w4::kCfgT32Ring) return W4_ERR_UNSUPPORTED;
+  if (dp.pair_words > 0) {
+    if (dp.pair_words * 8 > W4_WORKSPACE_COUNTER_BYTES) return W4_ERR_UNSUPPORTED;
+    if (counters == nullptr)
+      return fail(W4_ERR_WORKSPACE, "w4a16 decode: a workspace of %d bytes is required",
+                  (int)W4_WORKSPACE_COUNTER_BYTES);
+    for (int s = 0; s < dp.g.count; ++s) {
+      w4::DecArgs& d = dp.g.prob[s];
+      if (d.ksplit > 1) d.pair = reinterpret_cast<unsigned long long*>(counters) + dp.pair_off[s];
+    }
+  }
+  const w4::DecPrologue pro{static_cast<const uint16_t*>(a), static_cast<const uint16_t*>(w),
+                            static_cast<uint16_t*>(sum), eps};
+  if (x_dtype == W4_DTYPE_BF16) {
+    if (pro_kind == w4::kProNorm) dec_launch_pro<W4_DTYPE_BF16, w4::kProNorm>(dp, pro, st);
+    else dec_launch_pro<W4_DTYPE_BF16, w4::kProSilu>(dp, pro, st);
+  } else {
+    if (pro_kind == w4::kProNorm) dec_launch_pro<W4_DTYPE_FP16, w4::kProNorm>(dp, pro, st);
+    else dec_launch_pro<W4_DTYPE_FP16, w4::kProSilu>(dp, pro, st);
+  }
   return check_launch("w4a16 decode");
 }
 

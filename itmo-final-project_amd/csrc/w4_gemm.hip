@@ -72,6 +72,9 @@ size_t w4_decode_workspace_bytes(const w4a16_problem* problems, const int64_t* s
                                  const int64_t* mrows = nullptr);
 size_t w4_decode_single_workspace_bytes(int64_t M, int64_t N, int64_t K, int G);
 
+int w4_decode_pro_launch(const w4a16_problem* problems, int count, int x_dtype, int pro_kind, const void* a,
+                         const void* w, float eps, void* sum, unsigned* counters, hipStream_t st);
+
 // Every workspace starts with a W4_WORKSPACE_COUNTER_BYTES area of per-tile
 // arrival counters (zero before first use, left zero by every call), then
 // scratch (fp32 partial sums).
@@ -287,6 +290,48 @@ extern "C" int w4a16_gemm_grouped(const w4a16_problem* problems, int count, int 
                 "w4a16_gemm_grouped: a problem exceeds 2 GiB of packed weights or the column tiles of the "
                 "split problems exceed the counter area");
   return lrc;
+}
+
+// One row, activations from the operation in front of the linears.
+extern "C" int w4a16_decode_norm(const w4a16_problem* problems, int count, int x_dtype, const void* delta,
+                                 const void* weight, float eps, void* sum, void* workspace, size_t workspace_bytes,
+                                 void* stream) {
+  clear_error();
+  if (x_dtype != W4_DTYPE_BF16 && x_dtype != W4_DTYPE_FP16)
+    return fail(W4_ERR_INVALID, "w4a16_decode_norm: x dtype must be bf16 or fp16");
+  const int rc = check_grouped(problems, count, 1);
+  if (rc != W4_OK) return rc;
+  if (!weight) return fail(W4_ERR_INVALID, "w4a16_decode_norm: null pointer");
+  if ((((uintptr_t)delta | (uintptr_t)weight | (uintptr_t)sum) % 16) != 0)
+    return fail(W4_ERR_INVALID, "w4a16_decode_norm: delta, weight and sum must be 16-byte aligned");
+  for (int i = 1; i < count; ++i)
+    if (problems[i].x != problems[0].x || problems[i].K != problems[0].K)
+      return fail(W4_ERR_INVALID, "w4a16_decode_norm: the problems share one activation row");
+  if (sum != nullptr && (sum == problems[0].x || sum == delta))
+    return fail(W4_ERR_INVALID, "w4a16_decode_norm: sum must not overwrite its operands");
+  unsigned* counters;
+  void* scratch;
+  size_t scratch_bytes;
+  split_workspace(workspace, workspace_bytes, &counters, &scratch, &scratch_bytes);
+  return w4_decode_pro_launch(problems, count, x_dtype, 1, delta, weight, eps, sum, counters,
+                              static_cast<hipStream_t>(stream));
+}
+
+extern "C" int w4a16_decode_silu(const w4a16_problem* problem, int x_dtype, const void* up, void* workspace,
+                                 size_t workspace_bytes, void* stream) {
+  clear_error();
+  if (x_dtype != W4_DTYPE_BF16 && x_dtype != W4_DTYPE_FP16)
+    return fail(W4_ERR_INVALID, "w4a16_decode_silu: x dtype must be bf16 or fp16");
+  const int rc = check_grouped(problem, 1, 1);
+  if (rc != W4_OK) return rc;
+  if (!up || ((uintptr_t)up % 16) != 0)
+    return fail(W4_ERR_INVALID, "w4a16_decode_silu: up must be a 16-byte aligned pointer");
+  unsigned* counters;
+  void* scratch;
+  size_t scratch_bytes;
+  split_workspace(workspace, workspace_bytes, &counters, &scratch, &scratch_bytes);
+  return w4_decode_pro_launch(problem, 1, x_dtype, 2, up, nullptr, 0.f, nullptr, counters,
+                              static_cast<hipStream_t>(stream));
 }
 
 // ------------------------------------------------------------------------

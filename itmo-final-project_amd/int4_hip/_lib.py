@@ -79,6 +79,9 @@ SIGNATURES = {
     "w4a16_gemm_grouped": (_c_int, [ctypes.POINTER(Problem), _c_int, _c_int, _c_i64, _c_vp, _c_sz, _c_vp]),
     "w4a16_gemm_noalloc": (_c_int, [_c_vp, _c_int, _c_i64, _c_i64, _c_i64, _c_i64, _c_i64, _c_vp, _c_vp, _c_vp,
                                     _c_int, _c_vp, _c_i64, _c_vp]),
+    "w4a16_decode_norm": (_c_int, [ctypes.POINTER(Problem), _c_int, _c_int, _c_vp, _c_vp, ctypes.c_float, _c_vp, _c_vp,
+                                   _c_sz, _c_vp]),
+    "w4a16_decode_silu": (_c_int, [ctypes.POINTER(Problem), _c_int, _c_vp, _c_vp, _c_sz, _c_vp]),
     "w4_attention_decode_workspace_bytes": (_c_sz, [_c_i64, _c_i64, _c_i64, _c_i64]),
     "w4_attention_decode": (_c_int, [_c_vp, _c_vp, _c_vp, _c_int, _c_i64, _c_i64, _c_i64, _c_vp, _c_vp, _c_vp, _c_vp,
                                      _c_i64, _c_vp, _c_vp, _c_vp, _c_sz, _c_vp]),

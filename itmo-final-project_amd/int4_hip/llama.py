@@ -69,12 +69,17 @@ class RMSNorm(nn.Module):
         return F.rms_norm(x, (x.shape[-1],), self.weight, self.eps)
 
 
+def _plain(module: nn.Module, cls: type) -> bool:
+    """Whether calling ``module`` runs ``cls.forward`` and nothing else (no subclass,
+    replaced forward or hook), so that a fused kernel may stand for the call."""
+    return (type(module) is cls and "forward" not in module.__dict__ and not module._forward_hooks
+            and not module._forward_pre_hooks and not nn.modules.module._has_any_global_hook())
+
+
 def _add_norm(x: torch.Tensor, delta: torch.Tensor, norm: nn.Module) -> tuple:
     """(x + delta, norm(x + delta)), in one launch where ``norm`` is a plain RMSNorm
     that nothing hooks into."""
-    if (type(norm) is RMSNorm and "forward" not in norm.__dict__ and not norm._forward_hooks
-            and not norm._forward_pre_hooks and not nn.modules.module._has_any_global_hook()
-            and llama_ops.rms_norm_ok(x, norm.weight, delta)):
+    if _plain(norm, RMSNorm) and llama_ops.rms_norm_ok(x, norm.weight, delta):
         return llama_ops.rms_norm(x, norm.weight, norm.eps, delta)
     x = x + delta
     return x, norm(x)
@@ -196,6 +201,35 @@ class MLP(nn.Module):
         return self.down_proj(_silu_mul(self.gate_proj(x), self.up_proj(x)))
 
 
+def _norm_linears(x: torch.Tensor, delta: torch.Tensor | None, norm: RMSNorm, mods) -> tuple:
+    """(x + delta, outputs of the plain Int4Linear ``mods`` on its norm)."""
+    fused = llama_ops.norm_linears(x, delta, norm.weight, norm.eps, [(m.qweight, m.scales, m.zeros) for m in mods])
+    if fused is not None:
+        return fused
+    x, h = (x, norm(x)) if delta is None else _add_norm(x, delta, norm)
+    return x, _grouped(h, mods) if _all_int4(mods) else [m(h) for m in mods]
+
+
+def _decode_layer(layer, x, delta, cos, sin, kc, vc, pos_t) -> tuple | None:
+    """One decode step of a layer whose parts are all plain and whose linears are
+    Int4Linear without bias: five launches, the norms and the gated activation
+    computed by the linears that read them.  ``delta`` is the residual addition
+    still to be made; returns the new (x, delta), or None for any other layer."""
+    from .qlinear import Int4Linear
+    at, mlp = layer.self_attn, layer.mlp
+    qkv, gate_up = (at.q_proj, at.k_proj, at.v_proj), (mlp.gate_proj, mlp.up_proj)
+    if not (_plain(at, Attention) and _plain(mlp, MLP) and _plain(layer.input_layernorm, RMSNorm)
+            and _plain(layer.post_attention_layernorm, RMSNorm)
+            and all(_plain(m, Int4Linear) and m.bias is None for m in (*qkv, *gate_up, at.o_proj, mlp.down_proj))):
+        return None
+    x, (q, k, v) = _norm_linears(x, delta, layer.input_layernorm, qkv)
+    o = at.o_proj(llama_ops.attention_decode(q, k, v, cos, sin, kc, vc, pos_t, at.nh, at.nkv, at.d))
+    x, (g, u) = _norm_linears(x, o, layer.post_attention_layernorm, gate_up)
+    down = mlp.down_proj
+    y = llama_ops.silu_linear(g, u, (down.qweight, down.scales, down.zeros))
+    return x, down(_silu_mul(g, u)) if y is None else y
+
+
 class DecoderLayer(nn.Module):
     def __init__(self, cfg: LlamaConfig):
         super().__init__()
@@ -256,14 +290,20 @@ class LlamaForCausalLM(nn.Module):
                                                                    c.head_dim):
             mask_bias = torch.zeros(self.max_len, device=x.device).masked_fill_(self.key_pos > pos_t, float("-inf"))
         # each residual addition is fused with the norm that follows it
-        layers = self.model.layers
-        norms = [layer.input_layernorm for layer in layers] + [self.model.norm]
-        h = norms[0](x)
-        for i, layer in enumerate(layers):
-            a = layer.self_attn(h, cos, sin, self.kc[i], self.vc[i], pos0, pos_t, mask_bias)
-            x, h = _add_norm(x, a, layer.post_attention_layernorm)
-            x, h = _add_norm(x, layer.mlp(h), norms[i + 1])
-        return self.lm_head(h)
+        delta = None
+        for i, layer in enumerate(self.model.layers):
+            step = None
+            if pos_t is not None and mask_bias is None:
+                step = _decode_layer(layer, x, delta, cos, sin, self.kc[i], self.vc[i], pos_t)
+            if step is None:
+                norm = layer.input_layernorm
+                x, h = (x, norm(x)) if delta is None else _add_norm(x, delta, norm)
+                a = layer.self_attn(h, cos, sin, self.kc[i], self.vc[i], pos0, pos_t, mask_bias)
+                x, h = _add_norm(x, a, layer.post_attention_layernorm)
+                step = x, layer.mlp(h)
+            x, delta = step
+        norm = self.model.norm
+        return self.lm_head(norm(x) if delta is None else _add_norm(x, delta, norm)[1])
 
     @torch.no_grad()
     def prefill(self, ids: torch.Tensor) -> torch.Tensor:

@@ -15,7 +15,7 @@ from torch.autograd import forward_ad
 from torch.compiler import is_compiling as _is_compiling
 
 from . import _lib
-from .gemm import _with_workspace
+from .gemm import _check_weight, _with_workspace
 
 _XDT = {torch.bfloat16: _lib.DTYPE_BF16, torch.float16: _lib.DTYPE_FP16}
 _PLAIN = (torch.Tensor, nn.Parameter)
@@ -156,3 +156,62 @@ def silu_mul(gate, up) -> torch.Tensor:
     if rc:
         _lib.check(rc, "w4_silu_mul")
     return y
+
+
+def _row_problems(x, weights):
+    """(problem array, outputs) of one-row products on ``x`` [1, K], or None where the
+    weights are not plain dense buffers on x's GPU."""
+    K, dev = x.shape[-1], x.device
+    probs = (_lib.Problem * len(weights))()
+    outs = []
+    for i, (qw, s, z) in enumerate(weights):
+        if not (fusable(x, qw, s, z) and qw.is_contiguous() and s.is_contiguous() and z.is_contiguous()):
+            return None
+        assert qw.shape[0] * 8 == K
+        G, N = _check_weight(qw, s, z, K), qw.shape[1]
+        y = torch.empty((1, N), dtype=x.dtype, device=dev)
+        probs[i] = _lib.Problem(x.data_ptr(), qw.data_ptr(), s.data_ptr(), z.data_ptr(), y.data_ptr(), N, K, G, 0)
+        outs.append(y)
+    return probs, outs
+
+
+def norm_linears(x, delta, weight, eps: float, weights):
+    """(x + delta, [rmsnorm(x + delta) @ W_i^T ...]) of one row in one launch; None where
+    no such launch exists (nothing has been launched then)."""
+    if not (x.dim() == 2 and x.shape[0] == 1 and 1 <= len(weights) <= _lib.MAX_GROUPED
+            and rms_norm_ok(x, weight, delta)):
+        return None
+    row = _row_problems(x, weights)
+    if row is None:
+        return None
+    probs, outs = row
+    total = x if delta is None else torch.empty_like(x)
+    lib, dev = _lib.load(), x.device
+    nbytes = lib.w4a16_grouped_workspace_bytes(probs, len(weights), 1)
+    rc = _on(dev, lambda st: _with_workspace(dev, st, nbytes, lambda ws, nb: lib.w4a16_decode_norm(
+        probs, len(weights), _XDT[x.dtype], None if delta is None else delta.data_ptr(), weight.data_ptr(), eps,
+        None if delta is None else total.data_ptr(), ws, nb, st)))
+    if rc == _lib.ERR_UNSUPPORTED:
+        return None
+    if rc:
+        _lib.check(rc, "w4a16_decode_norm")
+    return total, outs
+
+
+def silu_linear(gate, up, weight):
+    """(silu(gate) * up) @ W^T of one row in one launch; None where no such launch exists."""
+    if not (gate.dim() == 2 and gate.shape[0] == 1 and silu_mul_ok(gate, up)):
+        return None
+    row = _row_problems(gate, [weight])
+    if row is None:
+        return None
+    probs, outs = row
+    lib, dev = _lib.load(), gate.device
+    nbytes = lib.w4a16_grouped_workspace_bytes(probs, 1, 1)
+    rc = _on(dev, lambda st: _with_workspace(dev, st, nbytes, lambda ws, nb: lib.w4a16_decode_silu(
+        probs, _XDT[gate.dtype], up.data_ptr(), ws, nb, st)))
+    if rc == _lib.ERR_UNSUPPORTED:
+        return None
+    if rc:
+        _lib.check(rc, "w4a16_decode_silu")
+    return outs[0]

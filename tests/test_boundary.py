@@ -116,6 +116,29 @@ def test_c_abi_rejects_bad_norm_and_activation_arguments(lib):
     assert lib.w4_silu_mul(None, None, 0, 0, None, None) == _lib.OK
 
 
+def test_c_abi_rejects_bad_prologue_arguments(lib):
+    fake, odd = ctypes.c_void_p(256), ctypes.c_void_p(264)
+
+    def problems(x1=256, K1=64):
+        p = (_lib.Problem * 2)()
+        p[0] = _lib.Problem(256, 256, 256, 256, 256, 8, 64, 32, 0)
+        p[1] = _lib.Problem(x1, 256, 256, 256, 256, 8, K1, 32, 0)
+        return p
+
+    def norm(p=None, n=2, dt=0, d=None, w=fake, s=None):
+        return lib.w4a16_decode_norm(p if p is not None else problems(), n, dt, d, w, 1e-5, s, None, 0, None)
+
+    assert norm(dt=2) == _lib.ERR_INVALID and norm(n=0) == _lib.ERR_INVALID and norm(w=None) == _lib.ERR_INVALID
+    assert norm(d=odd) == _lib.ERR_INVALID and norm(s=fake) == _lib.ERR_INVALID  # sum over x
+    assert norm(problems(x1=512)) == _lib.ERR_INVALID and norm(problems(K1=128)) == _lib.ERR_INVALID
+    assert lib.w4a16_decode_silu(problems(), 2, fake, None, 0, None) == _lib.ERR_INVALID
+    assert lib.w4a16_decode_silu(problems(), 0, None, None, 0, None) == _lib.ERR_INVALID
+    assert lib.w4a16_decode_silu(problems(), 0, odd, None, 0, None) == _lib.ERR_INVALID
+    p = problems()
+    p[0].group_size = 16  # valid, but no such launch
+    assert lib.w4a16_decode_silu(p, 0, fake, None, 0, None) == _lib.ERR_UNSUPPORTED
+
+
 def test_workspace_queries_over_regime_boundaries(lib):
     """The size queries run the launch planners on the host only: a sweep over
     the regime boundaries (M around 1 / 4 / 8 / 16 / 64 / 128, K around 4096 and

@@ -5,6 +5,7 @@ import math
 import pytest
 import torch
 
+import int4_hip
 from _synth import randn
 from int4_hip import llama_ops
 
@@ -191,3 +192,134 @@ def test_fused_ops_leave_the_general_path_alone():
     with torch.autocast("cuda", dtype=torch.float16):
         assert not llama_ops.rms_norm_ok(x, w)
     assert not torch.func.vmap(lambda t: torch.zeros(()) + llama_ops.silu_mul_ok(t, t))(x).any()
+
+
+def _rows(shapes, G, dtype, seed):
+    """Quantized weights of the shapes, and their exact 64-bit values."""
+    qs = [int4_hip.quantize_int4(randn(s, seed + i, 0.02, dtype=dtype).to(DEV), G) for i, s in enumerate(shapes)]
+    return qs, [int4_hip.dequantize_int4(*q, torch.float32).double().cpu() for q in qs]
+
+
+# one-row products behind a norm or a gated activation: the tile widths (128 / 64 /
+# 32 columns, picked by K and the number of workgroups), K parts joined across
+# workgroups, waves without steps (K = 256), the longest row of the norm.  Against
+# the 64-bit result of the unrounded activations.  Bound per output, relative to
+# the outputs' rms: one rounding of the output; one rounding of each activation,
+# independent errors of at most ROUND / sqrt(3) rms, six deviations; 1e-3 for the
+# fp32 accumulation of 128 x + x q terms (2^-24 of 143 sum |x| s).  The launch
+# rounds as often as the separate ones, so its total error may not be larger
+# (15 % for chance)
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("K,Ns,G", [(256, (64, 8), 32), (2048, (2048, 512, 512), 128), (2048, (8192, 8192), 64),
+                                    (4096, (1000,), 128), (8192, (72, 40), 512), (6144, (256,), 256)])
+def test_norm_linears(dtype, K, Ns, G):
+    print(f"[norm linears] {dtype} K={K} N={Ns} G={G}", flush=True)
+    qs, ws = _rows([(n, K) for n in Ns], G, dtype, 40)
+    x, d, w = randn((1, K), 1, dtype=dtype), randn((1, K), 2, 0.3, dtype=dtype), randn((K,), 3, dtype=dtype)
+    xd, dd, wd = (t.to(DEV) for t in (x, d, w))
+    for delta in (None, dd):
+        got = llama_ops.norm_linears(xd, delta, wd, 1e-5, qs)
+        assert got is not None
+        total, ys = got
+        if delta is None:
+            h = llama_ops.rms_norm(xd, wd, 1e-5)
+            assert total is xd
+        else:
+            s, h = llama_ops.rms_norm(xd, wd, 1e-5, dd)
+            assert torch.equal(total, s)
+        t = total.double().cpu()
+        exact = t * torch.rsqrt(t.square().mean() + 1e-5) * w.double()
+        for y, q, wx in zip(ys, qs, ws):
+            want = exact @ wx.T
+            _check_rows(y, int4_hip.w4a16_matmul(h, *q), want, dtype)
+            again = llama_ops.norm_linears(xd, delta, wd, 1e-5, [q])[1][0]  # another tiling
+            _check_rows(again, y, want, dtype)
+
+
+def _check_rows(got, separate, want, dtype):
+    got, separate = got.double().cpu(), separate.double().cpu()
+    err = (got - want).abs() / torch.maximum(want.abs(), want.square().mean().sqrt())
+    assert err.max().item() <= ROUND[dtype] * (1 + 6 / math.sqrt(3)) + 1e-3, err.max().item()
+    if want.numel() >= 256:
+        assert (got - want).norm() <= 1.15 * (separate - want).norm()
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("K,N,G", [(256, 8, 32), (8192, 2048, 128), (2048, 520, 64), (8192, 64, 1024)])
+def test_silu_linear(dtype, K, N, G):
+    print(f"[silu linear] {dtype} K={K} N={N} G={G}", flush=True)
+    (q,), (wx,) = _rows([(N, K)], G, dtype, 50)
+    g, u = randn((1, K), 1, 2.0, dtype=dtype).to(DEV), randn((1, K), 2, dtype=dtype).to(DEV)
+    got = llama_ops.silu_linear(g, u, q)
+    assert got is not None
+    gd, ud = g.double().cpu(), u.double().cpu()
+    _check_rows(got, int4_hip.w4a16_matmul(llama_ops.silu_mul(g, u), *q),
+                (torch.nn.functional.silu(gd) * ud) @ wx.T, dtype)
+    assert torch.equal(got, llama_ops.silu_linear(g, u, q))
+
+
+def test_prologue_launches_refuse_what_they_do_not_hold():
+    """No launch for group sizes below 32, ragged N, several rows or a norm past 8192
+    values: the callers then run the separate operations."""
+    x, w = torch.ones((1, 512), device=DEV, dtype=torch.bfloat16), torch.ones(512, device=DEV, dtype=torch.bfloat16)
+    for N, G in ((64, 16), (12, 64)):
+        q = int4_hip.quantize_int4(randn((N, 512), 1).to(DEV), G)
+        assert llama_ops.norm_linears(x, None, w, 1e-5, [q]) is None and llama_ops.silu_linear(x, x, q) is None
+    q = int4_hip.quantize_int4(randn((64, 512), 1).to(DEV), 64)
+    two = x.expand(2, 512).contiguous()
+    assert llama_ops.norm_linears(two, None, w, 1e-5, [q]) is None and llama_ops.silu_linear(two, two, q) is None
+    long = torch.ones((1, 16384), device=DEV, dtype=torch.bfloat16)
+    q = int4_hip.quantize_int4(randn((64, 16384), 1).to(DEV), 64)
+    assert llama_ops.norm_linears(long, None, long[0], 1e-5, [q]) is None
+
+
+def test_decode_step_respects_hooks_and_replaced_modules():
+    """A hook or a subclass anywhere in a layer keeps that layer on the module calls,
+    with the same logits up to rounding."""
+    from int4_hip.llama import LlamaConfig, LlamaForCausalLM
+    cfg = LlamaConfig(vocab_size=512, hidden_size=512, intermediate_size=1024, num_hidden_layers=2,
+                      num_attention_heads=8, num_key_value_heads=2, head_dim=64)
+    with torch.device(DEV):
+        m = LlamaForCausalLM(cfg)
+    m.init_weights(3)
+    m = int4_hip.quantize_model_linears(m.to(torch.bfloat16).eval(), 128)
+    m.allocate_cache(16, torch.bfloat16, DEV)
+    ids, pos = torch.tensor([7], device=DEV), torch.tensor([0], device=DEV)
+    want = m.decode_step(ids, pos).float()
+    seen = []
+    layer = m.model.layers[1]
+    for mod in (layer.post_attention_layernorm, layer.mlp, layer.self_attn.o_proj):
+        handle = mod.register_forward_hook(lambda *a: seen.append(a[0]))
+        got = m.decode_step(ids, pos).float()
+        handle.remove()
+        assert seen and seen.pop() is mod and not seen
+        assert (got - want).abs().max() <= 3e-2 * want.abs().max()
+
+
+@pytest.mark.parametrize("scale", [1e-4, 1.0, 3e3, 6e4])
+def test_norm_linears_fp16_range(scale):
+    """Large and small rows whose x * weight leaves fp16's range before the norm's factor,
+    with outliers of the size of the rest's sum: no overflow, no lost bits."""
+    K = 2048
+    (q,), (wx,) = _rows([(512, K)], 128, torch.float16, 60)
+    x = (randn((1, K), 1, dtype=torch.float32) * scale / 8).clamp(-6e4, 6e4)
+    x[0, 5] = scale
+    x, w = x.half(), (randn((K,), 2, dtype=torch.float32) * 20).half()
+    _, (y,) = llama_ops.norm_linears(x.to(DEV), None, w.to(DEV), 1e-5, [q])
+    t = x.double()
+    want = (t * torch.rsqrt(t.square().mean() + 1e-5) * w.double()) @ wx.T
+    h = llama_ops.rms_norm(x.to(DEV), w.to(DEV), 1e-5)
+    _check_rows(y, int4_hip.w4a16_matmul(h, *q), want, torch.float16)
+
+
+def test_norm_linears_non_finite_rows():
+    """A NaN or an infinity in the row makes every output NaN (inf * 0 in the norm); a zero
+    row gives zeros."""
+    K = 2048
+    (q,), _ = _rows([(64, K)], 128, torch.float16, 61)
+    w = torch.ones(K, device=DEV, dtype=torch.float16)
+    for bad in (float("nan"), float("inf")):
+        x = randn((1, K), 1, dtype=torch.float16).to(DEV)
+        x[0, 300] = bad
+        assert llama_ops.norm_linears(x, None, w, 1e-5, [q])[1][0].isnan().all()
+    assert not llama_ops.norm_linears(torch.zeros_like(x), None, w, 1e-5, [q])[1][0].any()
