@@ -1,9 +1,10 @@
-"""Build libint4_hip.so (gfx950) in-tree with hipcc.
+"""Build libint4_hip.so (gfx950) in-tree with hipcc, and _int4_torch.so (host) with g++.
 
     python itmo-final-project_amd/build_lib.py [--jobs N]
 
 Every call recompiles every source (object files go to ``_build/``, the
-library to ``int4_hip/libint4_hip.so``).  hipcc cross-compiles for gfx950 on a
+library to ``int4_hip/libint4_hip.so``, the torch binding of the Python entry
+points' fast path to ``int4_hip/_int4_torch.so``).  hipcc cross-compiles for gfx950 on a
 machine without a GPU.
 """
 from __future__ import annotations
@@ -24,6 +25,9 @@ LIB = HERE / "int4_hip" / "libint4_hip.so"
 # measurement helpers for bench.py (not part of the library)
 BENCH_SRC = CSRC / "bench"
 BENCH_LIB = HERE / "int4_hip" / "libw4_bench.so"
+# the Python entry points' native call path (built against the installed torch)
+EXT_SRC = CSRC / "torch_ext" / "int4_torch.cpp"
+EXT_LIB = HERE / "int4_hip" / "_int4_torch.so"
 ARCH = "gfx950"
 
 COMMON_FLAGS = [
@@ -62,12 +66,35 @@ def _compile(src: Path) -> Path:
     return obj
 
 
+def build_ext() -> Path:
+    """Compile int4_hip/_int4_torch.so (host code only) against the installed torch."""
+    import sysconfig
+
+    import torch
+
+    root = Path(torch.__file__).resolve().parent
+    tmp = EXT_LIB.with_suffix(".so.tmp")
+    cmd = [shutil.which("g++") or "g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-D__HIP_PLATFORM_AMD__=1",
+           "-DUSE_ROCM=1", f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+           "-I", str(root / "include"), "-I", str(root / "include" / "torch" / "csrc" / "api" / "include"),
+           "-I", str(Path(os.environ.get("ROCM_PATH", "/opt/rocm")) / "include"),
+           "-I", sysconfig.get_paths()["include"], "-I", str(ROOT / "include"), str(EXT_SRC), "-o", str(tmp),
+           "-L", str(root / "lib"), "-ltorch", "-ltorch_cpu", "-ltorch_python", "-lc10", "-lc10_hip"]
+    r = subprocess.run(cmd, capture_output=True, text=True)
+    if r.returncode != 0:
+        raise RuntimeError(f"compile failed: {EXT_SRC.name}\n{' '.join(cmd)}\n{r.stderr}")
+    os.replace(tmp, EXT_LIB)
+    return EXT_LIB
+
+
 def build(jobs: int | None = None, verbose: bool = True) -> Path:
     BUILD.mkdir(exist_ok=True)
     srcs = sources()
     jobs = jobs or min(len(srcs), os.cpu_count() or 4, 8)
-    with ThreadPoolExecutor(jobs) as ex:
+    with ThreadPoolExecutor(jobs + 1) as ex:
+        ext = ex.submit(build_ext)
         objs = list(ex.map(_compile, srcs))
+        ext.result()
     tmp = LIB.with_suffix(".so.tmp")
     cmd = [hipcc(), f"--offload-arch={ARCH}", "-shared", "-fPIC", "-o", str(tmp), *map(str, objs)]
     r = subprocess.run(cmd, capture_output=True, text=True)
@@ -84,7 +111,7 @@ def build(jobs: int | None = None, verbose: bool = True) -> Path:
             raise RuntimeError(f"link failed\n{' '.join(cmd)}\n{r.stderr}")
         os.replace(btmp, BENCH_LIB)
     if verbose:
-        print(f"built {LIB} from {len(srcs)} sources (+ {BENCH_LIB.name})", file=sys.stderr)
+        print(f"built {LIB} from {len(srcs)} sources (+ {EXT_LIB.name}, {BENCH_LIB.name})", file=sys.stderr)
     return LIB
 
 

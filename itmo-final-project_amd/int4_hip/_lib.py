@@ -93,11 +93,28 @@ SIGNATURES = {
 
 _lock = threading.Lock()
 _lib = None
+# int4_hip._int4_torch once the library is loaded: the entry points' native call
+# path for plain operands (csrc/torch_ext/int4_torch.cpp).  Its functions return
+# None for everything else, which the Python code then handles.
+ext = None
+
+
+def _load_ext(lib):
+    from . import gemm
+    try:
+        from . import _int4_torch
+    except ImportError as e:
+        raise RuntimeError(f"int4_hip: the torch binding _int4_torch.so is not built or does not fit the installed "
+                           f"torch ({e}); run `python itmo-final-project_amd/build_lib.py`") from e
+    names = ("w4a16_gemm", "w4a16_workspace_bytes", "w4a16_gemm_grouped", "w4a16_grouped_workspace_bytes",
+             "w4_quantize_grouped", "w4_quantize", "w4_dequantize")
+    _int4_torch.init(tuple(ctypes.cast(getattr(lib, n), _c_vp).value for n in names), gemm._workspace_address, check)
+    return _int4_torch
 
 
 def load(path: Path | str | None = None) -> ctypes.CDLL:
     """Load (once) and type the library; raise RuntimeError if it is unusable."""
-    global _lib
+    global _lib, ext
     if _lib is not None and path is None:
         return _lib
     with _lock:
@@ -117,6 +134,7 @@ def load(path: Path | str | None = None) -> ctypes.CDLL:
         if v != ABI_VERSION:
             raise RuntimeError(f"int4_hip: {p} has ABI version {v}, bindings expect {ABI_VERSION}; rebuild it")
         if path is None:
+            ext = _load_ext(lib)
             _lib = lib
         return lib
 

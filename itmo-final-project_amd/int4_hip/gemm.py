@@ -118,6 +118,11 @@ def _with_workspace(device: torch.device, stream: int, nbytes: int, launch) -> i
     return launch(ws.data_ptr(), ws.numel())
 
 
+def _workspace_address(index: int, stream: int, nbytes: int) -> tuple:
+    """(address, bytes) of the workspace of a call on ``stream`` of GPU ``index``."""
+    return _with_workspace(torch.device("cuda", index), stream, nbytes, lambda ws, nb: (ws, nb))
+
+
 _WS_BYTES: dict = {}
 
 
@@ -146,6 +151,10 @@ def w4a16_matmul(x: torch.Tensor, qweight: torch.Tensor, scales: torch.Tensor, z
 
     Mirrors int4_triton/gemm.py:303-309 (assertions included).
     """
+    if _lib.ext is not None:  # plain operands: the same call without Python's share of its cost
+        y = _lib.ext.matmul(x, qweight, scales, zeros)
+        if y is not None:
+            return y
     assert x.dtype in (torch.bfloat16, torch.float16)
     K = x.shape[-1]
     assert qweight.shape[0] * 8 == K, (qweight.shape, K)
@@ -183,6 +192,10 @@ def w4a16_matmul_grouped(xs: Sequence[torch.Tensor], weights: Sequence[tuple],
     one launch each.  This fuses the per-linear launches
     of a transformer block; it has no single counterpart in the reference.
     """
+    if _lib.ext is not None:
+        ys = _lib.ext.matmul_grouped(xs, weights, out)
+        if ys is not None:
+            return ys
     assert 1 <= len(xs) == len(weights) <= _lib.MAX_GROUPED
     dt = xs[0].dtype
     assert dt in _XDT

@@ -58,6 +58,10 @@ def quantize_int4(w: torch.Tensor, group_size: int = 128):
     zeros fp16 [K/G, N])``; ``group_size=-1`` means one group per row (G = K).
     Misuse raises ``AssertionError`` as int4_triton/quantize.py:69-75 does.
     """
+    if _lib.ext is not None:  # plain operands: the same call without Python's share of its cost
+        out = _lib.ext.quantize(w, group_size)
+        if out is not None:
+            return out
     assert w.dim() == 2 and w.is_cuda
     assert w.dtype in (torch.float16, torch.bfloat16)
     N, K = w.shape
@@ -85,6 +89,10 @@ def quantize_int4_grouped(ws, group_size: int = 128):
     per-linear ``quantize_int4`` calls of one block
     (int4_triton/qlinear.py:55-68)."""
     ws = list(ws)
+    if _lib.ext is not None:
+        outs = _lib.ext.quantize_grouped(ws, group_size)
+        if outs is not None:
+            return outs
     assert 1 <= len(ws) <= _lib.MAX_GROUPED
     dt, dev = ws[0].dtype, ws[0].device
     assert dt in (torch.float16, torch.bfloat16)
@@ -115,6 +123,10 @@ def dequantize_int4(qweight: torch.Tensor, scales: torch.Tensor, zeros: torch.Te
 
     Bit-identical to ``dequantize_int4_ref`` on the same buffers.
     """
+    if _lib.ext is not None:
+        out = _lib.ext.dequantize(qweight, scales, zeros, dtype)
+        if out is not None:
+            return out
     assert qweight.is_cuda and scales.is_cuda and zeros.is_cuda
     assert qweight.dtype == torch.int32 and scales.dtype == torch.float16 and zeros.dtype == torch.float16
     assert dtype in _DT, dtype
