@@ -356,8 +356,6 @@ __global__ __launch_bounds__(256) void rope_cache_kernel(AttnPrefillArgs a) {
       a.kc[((int64_t)h * D + d) * a.max_len + a.pos0 + t] = tile[d][lane];
 }
 
-typedef float f32x4_u __attribute__((ext_vector_type(4), aligned(4)));
-
 // Causal attention of a prompt over the fp32 caches (rope_cache_kernel has
 // filled them up to pos0 + T), online softmax, fp32 MFMA 16x16x4 for both
 // products, one rounding of the output.
@@ -374,15 +372,18 @@ typedef float f32x4_u __attribute__((ext_vector_type(4), aligned(4)));
 // free, so row 4j + r of the S^T tile c is position 16j + 4r + c (a lane's
 // 128-bit key load covers four tiles), and the r-th step over tile c multiplies
 // by V rows 16j + 4r + c.  What bounds it: the matrix cores' fp32 rate (157
-// TFLOP/s), loads of the next block overlapping only with the other wave of
-// the SIMD.  Four layers of the 1B model and its head on 500 tokens: 1764 us
-// with torch's batched fp32 products, masks and copies, 818 us with this.
+// TFLOP/s) and the latency that stays visible: half of a block's values travel
+// under its softmax, the rest and half of the next block's keys under its second
+// product (all of it would not fit the registers of two waves per SIMD).  Four layers of the 1B model and its head on 500 tokens: 1764 us
+// with torch's batched fp32 products, masks and copies; this kernel takes 21 us
+// of a layer there (29 us with each load next to its use).
 template <int DT, int D>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D == 64 ? 2 : 1))) void attn_prefill_kernel(
     AttnPrefillArgs a) {
   constexpr int DQ = D / 4;   // head elements per lane (keys and queries)
   constexpr int NT = D / 16;  // row tiles of O^T
   constexpr int VH = D / 64;  // 128-bit value loads per position
+  constexpr int DH = DQ / 2;
   __shared__ __attribute__((aligned(16))) float o_s[4][2][16][D + 4];
   __shared__ float m_s[4][2][16], l_s[4][2][16];
 
@@ -418,8 +419,12 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D == 64 ? 2
     }
   }
 
-  const float* __restrict__ kc = a.kc + ((int64_t)kvh * D + j * DQ) * a.max_len;
-  const float* __restrict__ vc = a.vc + (int64_t)kvh * a.max_len * D;
+  // the head's keys and values (below 2 GiB each, the host checks)
+  const int64_t head = (int64_t)kvh * D * a.max_len;
+  const __amdgpu_buffer_rsrc_t rk =
+      __builtin_amdgcn_make_buffer_rsrc((void*)(a.kc + head), (short)0, D * a.max_len * 4, 0x00020000);
+  const __amdgpu_buffer_rsrc_t rv =
+      __builtin_amdgcn_make_buffer_rsrc((void*)(a.vc + head), (short)0, D * a.max_len * 4, 0x00020000);
   const int L = a.pos0 + a.T;
   const int blocks = (min(a.pos0 + tb + (two_heads ? 15 : 31), L - 1) >> 6) + 1;
   float m[2], l[2];
@@ -430,6 +435,49 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D == 64 ? 2
 #pragma unroll
     for (int n = 0; n < NT; ++n) o[c][n] = f32x4{0.f, 0.f, 0.f, 0.f};
   }
+  // Keys of a block, lane i of part j: positions p0 + 4 i .. + 3 of elements
+  // j DQ + d.  The last block of a cache whose end lies inside it is read
+  // element by element, clamped.
+  // (Buffer loads: the element enters through the scalar offset, so the 16 or 32
+  // rows need no address registers of their own.)
+  const uint32_t k_lane = (uint32_t)(j * DQ) * (uint32_t)a.max_len * 4u;
+  // half h: elements [h DQ / 2, + DQ / 2)
+  auto load_k = [&](int p0, int h, f32x4* kk) {
+    const uint32_t row = (uint32_t)a.max_len * 4u;
+    if (p0 + 64 <= a.max_len) {
+      const uint32_t vo = k_lane + (uint32_t)(p0 + 4 * i) * 4u;
+#pragma unroll
+      for (int d = h * DH; d < (h + 1) * DH; ++d)
+        kk[d] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rk, vo, (uint32_t)d * row, 0));
+    } else {
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        const uint32_t vo = k_lane + (uint32_t)min(p0 + 4 * i + u, a.max_len - 1) * 4u;
+#pragma unroll
+        for (int d = h * DH; d < (h + 1) * DH; ++d)
+          kk[d][u] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rk, vo, (uint32_t)d * row, 0));
+      }
+    }
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  // values of a block, r in {2 h, 2 h + 1}; rows past the prompt hold nothing yet:
+  // a valid row, whose weight is 0
+  f32x4 vv[2][8][VH];
+  auto load_v = [&](int p0, int h) {
+#pragma unroll
+    for (int x = 0; x < 8; ++x) {
+      const uint32_t vo = (uint32_t)(min(p0 + 16 * j + 8 * h + x, L - 1) * D + 4 * i) * 4u;
+#pragma unroll
+      for (int hh = 0; hh < VH; ++hh)
+        vv[h][x][hh] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rv, vo, 256u * (uint32_t)hh, 0));
+    }
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  f32x4 kk[DQ];
+  if (wv < blocks) {
+    load_k(wv * 64, 0, kk);
+    load_k(wv * 64, 1, kk);
+  }
   for (int b = wv; b < blocks; b += 4) {
     const int p0 = b * 64;
     f32x4 s[2][4];
@@ -437,22 +485,15 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D == 64 ? 2
     for (int c = 0; c < 2; ++c)
 #pragma unroll
       for (int u = 0; u < 4; ++u) s[c][u] = f32x4{0.f, 0.f, 0.f, 0.f};
-    const bool whole = p0 + 64 <= a.max_len;  // else the last positions are read one by one, clamped
 #pragma unroll
-    for (int d = 0; d < DQ; ++d) {
-      const float* kp = kc + (int64_t)d * a.max_len;
-      f32x4 kk;
-      if (whole) {
-        kk = *reinterpret_cast<const f32x4_u*>(kp + p0 + 4 * i);
-      } else {
-#pragma unroll
-        for (int u = 0; u < 4; ++u) kk[u] = kp[min(p0 + 4 * i + u, a.max_len - 1)];
-      }
+    for (int d = 0; d < DQ; ++d)
 #pragma unroll
       for (int u = 0; u < 4; ++u)
 #pragma unroll
-        for (int c = 0; c < 2; ++c) s[c][u] = __builtin_amdgcn_mfma_f32_16x16x4f32(kk[u], qf[c][d], s[c][u], 0, 0, 0);
-    }
+        for (int c = 0; c < 2; ++c)
+          s[c][u] = __builtin_amdgcn_mfma_f32_16x16x4f32(kk[d][u], qf[c][d], s[c][u], 0, 0, 0);
+    __builtin_amdgcn_sched_barrier(0);
+    load_v(p0, 0);  // in flight under the softmax
 #pragma unroll
     for (int c = 0; c < 2; ++c) {
       float mx = -__builtin_inff();
@@ -483,22 +524,26 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D == 64 ? 2
 #pragma unroll
       for (int n = 0; n < NT; ++n) o[c][n] *= al;
     }
+    __builtin_amdgcn_sched_barrier(0);
+    auto product = [&](int h) {
 #pragma unroll
-    for (int r = 0; r < 4; ++r)
+      for (int x = 0; x < 8; ++x)
 #pragma unroll
-      for (int u = 0; u < 4; ++u) {
-        // rows past the prompt hold nothing yet: a valid row, whose weight is 0
-        const float* vp = vc + (int64_t)min(p0 + 16 * j + 4 * r + u, L - 1) * D + 4 * i;
-#pragma unroll
-        for (int hh = 0; hh < VH; ++hh) {
-          const f32x4 vv = *reinterpret_cast<const f32x4*>(vp + 64 * hh);
+        for (int hh = 0; hh < VH; ++hh)
 #pragma unroll
           for (int e = 0; e < 4; ++e)
 #pragma unroll
             for (int c = 0; c < 2; ++c)
-              o[c][4 * hh + e] = __builtin_amdgcn_mfma_f32_16x16x4f32(vv[e], s[c][u][r], o[c][4 * hh + e], 0, 0, 0);
-        }
-      }
+              o[c][4 * hh + e] = __builtin_amdgcn_mfma_f32_16x16x4f32(
+                  vv[h][x][hh][e], s[c][x & 3][2 * h + (x >> 2)], o[c][4 * hh + e], 0, 0, 0);
+      __builtin_amdgcn_sched_barrier(0);
+    };
+    // each half of the loads ahead goes out as soon as registers for it are free
+    load_v(p0, 1);
+    product(0);
+    if (b + 4 < blocks) load_k(p0 + 256, 0, kk);
+    product(1);
+    if (b + 4 < blocks) load_k(p0 + 256, 1, kk);
   }
   // join the four waves: lane (j, i) holds O[query i][64 hh + 16 j + 4 r + e]
 #pragma unroll
@@ -668,7 +713,7 @@ extern "C" int w4_attention_prefill(const void* q, const void* k, const void* v,
   if (dtype != W4_DTYPE_BF16 && dtype != W4_DTYPE_FP16)
     return fail(W4_ERR_INVALID, "w4_attention_prefill: dtype must be bf16 or fp16 (got code %d)", dtype);
   if (num_kv_heads < 1 || num_kv_heads > 65535 || num_heads < num_kv_heads || num_heads % num_kv_heads != 0 ||
-      num_heads >= (1LL << 24) || (head_dim != 64 && head_dim != 128) || max_len >= (1LL << 24))
+      num_heads >= (1LL << 24) || (head_dim != 64 && head_dim != 128) || max_len >= (1LL << 22))
     return fail(W4_ERR_UNSUPPORTED,
                 "w4_attention_prefill: %lld query / %lld key-value heads of %lld over %lld positions "
                 "(heads of 64 or 128)",

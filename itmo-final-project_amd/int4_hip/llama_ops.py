@@ -93,7 +93,7 @@ def attention_prefill_ok(x, kc, vc, cos, sin, pos0, nh: int, nkv: int, d: int) -
     pos0.. of the caches ``kc`` [nkv, d, L], ``vc`` [nkv, L, d]."""
     T, L = x.shape[0], kc.shape[-1]
     return (x.dim() == 2 and T >= 1 and d in (64, 128) and nh % nkv == 0 and type(pos0) is int
-            and 0 <= pos0 <= L - T and L < 1 << 24 and T <= 65535 * 16 and nkv <= 65535
+            and 0 <= pos0 <= L - T and L < 1 << 22 and T <= 65535 * 16 and nkv <= 65535
             and x.dtype in _XDT and kc.dtype == vc.dtype == cos.dtype == sin.dtype == torch.float32
             and kc.shape == (nkv, d, L) and vc.shape == (nkv, L, d) and cos.shape == sin.shape == (T, d // 2)
             and kc.is_contiguous() and cos.is_contiguous() and sin.is_contiguous()
