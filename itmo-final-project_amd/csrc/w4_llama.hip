@@ -195,7 +195,7 @@ __global__ __launch_bounds__(kAttnThreads) void attn_decode_kernel(AttnDecodeArg
         for (int u = 0; u < 4; ++u)
 #pragma unroll
           for (int e = 0; e < VE; ++e) {
-            const float vv = p0 + wv * PW + i + u == pos ? v_s[lane * VE + e] : vr[i + u][e];
+            const float vv = p0 + wv * PW + i + u >= pos ? v_s[lane * VE + e] : vr[i + u][e];
             o[h][e] = __builtin_fmaf(pv[u], vv, o[h][e]);
           }
       }

@@ -285,9 +285,11 @@ class LlamaForCausalLM(nn.Module):
     def _layers(self, x, cos, sin, pos0, pos_t):
         mask_bias = None
         c = self.config
-        if pos_t is not None and not llama_ops.attention_decode_ok(x, self.kc, self.vc, cos, sin, pos_t,
-                                                                   c.num_attention_heads, c.num_key_value_heads,
-                                                                   c.head_dim):
+        # (another attention module, or a hook on one, gets the mask)
+        if pos_t is not None and not (all(_plain(layer.self_attn, Attention) for layer in self.model.layers)
+                                      and llama_ops.attention_decode_ok(
+                                          x, self.kc, self.vc, cos, sin, pos_t, c.num_attention_heads,
+                                          c.num_key_value_heads, c.head_dim)):
             mask_bias = torch.zeros(self.max_len, device=x.device).masked_fill_(self.key_pos > pos_t, float("-inf"))
         # each residual addition is fused with the norm that follows it
         delta = None

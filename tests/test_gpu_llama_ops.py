@@ -61,9 +61,9 @@ def test_attention_decode(dtype, nh, nkv, d, max_len, pos):
     print(f"[attn decode] {dtype} {nh}/{nkv}x{d} L={max_len} pos={pos}", flush=True)
     q, k, v = (randn((1, n * d), seed=i, dtype=dtype) for i, n in enumerate((nh, nkv, nkv)))
     kc, vc = randn((nkv, d, max_len), 5, dtype=torch.float32), randn((nkv, max_len, d), 6, dtype=torch.float32)
-    # what lies past the position takes no part, whatever it holds
-    kc[..., pos + 1:] = float("nan")
-    vc[:, pos + 1:] = float("inf")
+    # what lies at the position and past it takes no part, whatever it holds
+    kc[..., pos:] = float("nan")
+    vc[:, pos:] = float("inf")
     cos, sin = (t[pos:pos + 1] for t in _tables(max_len, d))
     p = torch.tensor([pos], device=DEV)
     args = [t.to(DEV) for t in (q, k, v, cos.contiguous(), sin.contiguous(), kc, vc)]
@@ -294,6 +294,12 @@ def test_decode_step_respects_hooks_and_replaced_modules():
         handle.remove()
         assert seen and seen.pop() is mod and not seen
         assert (got - want).abs().max() <= 3e-2 * want.abs().max()
+    # a hook on an attention module sees the mask, as without the fused kernel
+    handle = layer.self_attn.register_forward_pre_hook(lambda mod, args: seen.append(args[7]))
+    got = m.decode_step(ids, pos).float()
+    handle.remove()
+    assert seen[0].tolist() == [0.0] + [float("-inf")] * 15
+    assert (got - want).abs().max() <= 3e-2 * want.abs().max()
 
 
 @pytest.mark.parametrize("scale", [1e-4, 1.0, 3e3, 6e4])
