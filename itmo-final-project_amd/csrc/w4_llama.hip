@@ -41,31 +41,50 @@ __device__ __forceinline__ void rope_pair(float x1, float x2, float c, float s, 
   *r2 = x2 * c + x1 * s;
 }
 
+// Reductions over the 64 lanes (all active), the result in every lane: four DPP
+// steps within the rows of 16, then the four rows through scalar registers (a
+// shuffle through LDS per step is ten times the latency).
+template <int CTRL>
+__device__ __forceinline__ float lane_perm(float v) {
+  return __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, v), CTRL, 0xF, 0xF, true));
+}
+__device__ __forceinline__ float lane_read(float v, int lane) {
+  return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), lane));
+}
 __device__ __forceinline__ float wave_max(float v) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) v = fmaxf(v, __shfl_xor(v, o, 64));
-  return v;
+  v = fmaxf(v, lane_perm<0xB1>(v));   // lane ^ 1
+  v = fmaxf(v, lane_perm<0x4E>(v));   // lane ^ 2
+  v = fmaxf(v, lane_perm<0x141>(v));  // half rows mirrored
+  v = fmaxf(v, lane_perm<0x140>(v));  // rows mirrored
+  return fmaxf(fmaxf(lane_read(v, 0), lane_read(v, 16)), fmaxf(lane_read(v, 32), lane_read(v, 48)));
 }
 __device__ __forceinline__ float wave_sum(float v) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
-  return v;
+  v += lane_perm<0xB1>(v);
+  v += lane_perm<0x4E>(v);
+  v += lane_perm<0x141>(v);
+  v += lane_perm<0x140>(v);
+  return (lane_read(v, 0) + lane_read(v, 16)) + (lane_read(v, 32) + lane_read(v, 48));
 }
 
 // One workgroup = one key-value head x one chunk of cache positions (a
 // multiple of 64) x up to four of its query heads (eight would need 256
 // registers), fp32 throughout.
 //
-// What bounds it: the latency of one trip to memory (at 576 positions a head's
-// keys and values are 288 KB).  So positions are cut into chunks over
+// What bounds it: the latency of a chain of trips to memory (at 576 positions a
+// head's keys and values are 288 KB).  So positions are cut into chunks over
 // workgroups (9 x 8 heads there), each lane issues its D/4 key loads (lane =
 // position, the cache keeps K transposed, so a wave reads 256 contiguous
-// bytes) and its value loads before the first use, and the chunks of a head
-// meet without a second launch: each publishes (max, sum, unnormalised
-// output), and the last to arrive joins them in chunk order (same bits every
-// run).  The chunk that holds the position writes the new key and value to
-// the cache and uses them from LDS.  A decode step of the 1B model (16 layers,
-// position 575, fp16): 1559 us with the torch operations, 848 us with this.
+// bytes) and its value loads before the position itself has arrived, and the
+// chunks of a head meet without a second launch: each publishes (max, sum,
+// unnormalised output), and the last to arrive joins them in chunk order (same
+// bits every run), their outputs loaded together with their maxima and sums.
+// The chunk that holds the position writes the new key and value to the cache
+// and uses them from LDS.  A decode step of the 1B model (16 layers, position
+// 575, fp16): 1559 us with the torch operations, 848 us with the first form of
+// this kernel alone.  There a layer's launch takes 6.4 us; 8.7 us with the keys
+// loaded after the position and the query, the outputs to join after their
+// weights, a branch per element for the new key and value, and reductions by
+// LDS shuffles.
 template <int DT, int D, int GP>
 __global__ __launch_bounds__(kAttnThreads) void attn_decode_kernel(AttnDecodeArgs a) {
   constexpr int DW = D / kAttnWaves;   // head elements per wave (keys)
@@ -88,32 +107,56 @@ __global__ __launch_bounds__(kAttnThreads) void attn_decode_kernel(AttnDecodeArg
   const int c = blockIdx.x, kvh = blockIdx.y, z = blockIdx.z;
   const int h0 = kvh * a.g + z * kAttnHeads;  // first query head
   const int g = min(a.g - z * kAttnHeads, GP);
+  const int c0 = c * a.chunk;
+  const float* __restrict__ kc = a.kc + (int64_t)kvh * D * a.max_len;
+  const float* __restrict__ vc = a.vc + (int64_t)kvh * a.max_len * D;
+
   const int64_t pos64 = *a.pos;
+  // Everything the chunk's first block needs, in the order of its use.  Clamped
+  // to the cache and not to the position, so that nothing waits for the
+  // position: what lies past it is not used below.
+  static_assert(GP * (D / 2) <= kAttnThreads && kAttnThreads % D == 0, "one rotary pair per thread");
+  const int qh = tid / (D / 2), qd = tid % (D / 2);
+  const uint16_t* const qp = a.q + (int64_t)(h0 + min(qh, g - 1)) * D + qd;
+  const uint16_t q1 = qp[0], q2 = qp[D / 2];
+  const float rc = a.cos[qd], rs = a.sin[qd];
+  const uint16_t* const kp = a.k + (int64_t)kvh * D + qd;
+  const uint16_t k1 = kp[0], k2 = kp[D / 2], v1 = a.v[(int64_t)kvh * D + tid % D];
+  float kr[DW], vr[PW][VE];
+  auto load_k = [&](int p0) {
+    const int p = min(p0 + lane, a.max_len - 1);
+#pragma unroll
+    for (int i = 0; i < DW; ++i) kr[i] = kc[(int64_t)(wv * DW + i) * a.max_len + p];
+  };
+  auto load_v = [&](int p0) {
+#pragma unroll
+    for (int i = 0; i < PW; ++i) {
+      const float* vp = vc + (int64_t)min(p0 + wv * PW + i, a.max_len - 1) * D + lane * VE;
+#pragma unroll
+      for (int e = 0; e < VE; ++e) vr[i][e] = vp[e];
+    }
+  };
+  __builtin_amdgcn_sched_barrier(0);
+  load_k(c0);
+  load_v(c0);
+  __builtin_amdgcn_sched_barrier(0);
+
   if (pos64 < 0 || pos64 >= a.max_len) return;  // the caller's table lookup refuses such a position
   const int pos = (int)pos64;
   const int active = pos / a.chunk + 1;
   if (c >= active) return;
-  const int c0 = c * a.chunk;
   const int c1 = min(c0 + a.chunk, pos + 1);
-  const float* __restrict__ kc = a.kc + (int64_t)kvh * D * a.max_len;
-  const float* __restrict__ vc = a.vc + (int64_t)kvh * a.max_len * D;
 
-  for (int i = tid; i < GP * (D / 2); i += kAttnThreads) {
-    const int h = i / (D / 2), d = i % (D / 2);
-    float r1 = 0.f, r2 = 0.f;
-    if (h < g) {
-      const uint16_t* q = a.q + (int64_t)(h0 + h) * D;
-      rope_pair(act_bits_to_float(q[d], DT), act_bits_to_float(q[d + D / 2], DT), a.cos[d], a.sin[d], &r1, &r2);
-    }
-    q_s[h][d] = r1 * a.qscale;
-    q_s[h][d + D / 2] = r2 * a.qscale;
+  if (tid < GP * (D / 2)) {
+    float r1, r2;
+    rope_pair(act_bits_to_float(q1, DT), act_bits_to_float(q2, DT), rc, rs, &r1, &r2);
+    q_s[qh][qd] = qh < g ? r1 * a.qscale : 0.f;
+    q_s[qh][qd + D / 2] = qh < g ? r2 * a.qscale : 0.f;
   }
   if (c == active - 1) {
     if (tid < D / 2) {
-      const uint16_t* k = a.k + (int64_t)kvh * D;
       float r1, r2;
-      rope_pair(act_bits_to_float(k[tid], DT), act_bits_to_float(k[tid + D / 2], DT), a.cos[tid], a.sin[tid], &r1,
-                &r2);
+      rope_pair(act_bits_to_float(k1, DT), act_bits_to_float(k2, DT), rc, rs, &r1, &r2);
       k_s[tid] = r1;
       k_s[tid + D / 2] = r2;
       if (z == 0) {
@@ -121,7 +164,7 @@ __global__ __launch_bounds__(kAttnThreads) void attn_decode_kernel(AttnDecodeArg
         a.kc[((int64_t)kvh * D + tid + D / 2) * a.max_len + pos] = r2;
       }
     } else if (tid >= 128 && tid < 128 + D) {
-      const float v = act_bits_to_float(a.v[(int64_t)kvh * D + tid - 128], DT);
+      const float v = act_bits_to_float(v1, DT);
       v_s[tid - 128] = v;
       if (z == 0) a.vc[((int64_t)kvh * a.max_len + pos) * D + tid - 128] = v;
     }
@@ -138,33 +181,36 @@ __global__ __launch_bounds__(kAttnThreads) void attn_decode_kernel(AttnDecodeArg
     for (int e = 0; e < VE; ++e) o[h][e] = 0.f;
 
   for (int p0 = c0; p0 < c1; p0 += 64) {
-    const int p = p0 + lane, pc = min(p, pos);
-    float kr[DW], vr[PW][VE];
+    const int p = p0 + lane;
+    if (p0 + 64 > pos) {  // uniform: the block of the position (values past it: any finite one)
 #pragma unroll
-    for (int i = 0; i < DW; ++i) kr[i] = kc[(int64_t)(wv * DW + i) * a.max_len + pc];
+      for (int i = 0; i < DW; i += 4) {
+        const f32x4 kn = *reinterpret_cast<const f32x4*>(&k_s[wv * DW + i]);
 #pragma unroll
-    for (int i = 0; i < PW; ++i) {
-      const float* vp = vc + (int64_t)min(p0 + wv * PW + i, pos) * D + lane * VE;
+        for (int e = 0; e < 4; ++e) kr[i + e] = p == pos ? kn[e] : kr[i + e];
+      }
 #pragma unroll
-      for (int e = 0; e < VE; ++e) vr[i][e] = vp[e];
+      for (int e = 0; e < VE; ++e) {
+        const float vn = v_s[lane * VE + e];
+#pragma unroll
+        for (int i = 0; i < PW; ++i) vr[i][e] = p0 + wv * PW + i >= pos ? vn : vr[i][e];
+      }
     }
     float s[GP];
 #pragma unroll
     for (int h = 0; h < GP; ++h) s[h] = 0.f;
 #pragma unroll
     for (int i = 0; i < DW; i += 4) {
-      float kk[4];
-#pragma unroll
-      for (int e = 0; e < 4; ++e) kk[e] = p == pos ? k_s[wv * DW + i + e] : kr[i + e];
 #pragma unroll
       for (int h = 0; h < GP; ++h) {
         const f32x4 qv = *reinterpret_cast<const f32x4*>(&q_s[h][wv * DW + i]);
 #pragma unroll
-        for (int e = 0; e < 4; ++e) s[h] = __builtin_fmaf(qv[e], kk[e], s[h]);
+        for (int e = 0; e < 4; ++e) s[h] = __builtin_fmaf(qv[e], kr[i + e], s[h]);
       }
     }
 #pragma unroll
     for (int h = 0; h < GP; ++h) red[wv][h][lane] = s[h];
+    if (p0 + 64 < c1) load_k(p0 + 64);  // the next block's, under this one's softmax
     __syncthreads();
 #pragma unroll
     for (int j = 0; j < HW; ++j) {
@@ -194,12 +240,10 @@ __global__ __launch_bounds__(kAttnThreads) void attn_decode_kernel(AttnDecodeArg
 #pragma unroll
         for (int u = 0; u < 4; ++u)
 #pragma unroll
-          for (int e = 0; e < VE; ++e) {
-            const float vv = p0 + wv * PW + i + u >= pos ? v_s[lane * VE + e] : vr[i + u][e];
-            o[h][e] = __builtin_fmaf(pv[u], vv, o[h][e]);
-          }
+          for (int e = 0; e < VE; ++e) o[h][e] = __builtin_fmaf(pv[u], vr[i + u][e], o[h][e]);
       }
     }
+    if (p0 + 64 < c1) load_v(p0 + 64);
     // red is next written after every wave has passed the barrier above
   }
 #pragma unroll
@@ -242,6 +286,14 @@ __global__ __launch_bounds__(kAttnThreads) void attn_decode_kernel(AttnDecodeArg
   if (arrived != (unsigned)(active - 1)) return;
   if (tid == 0) __hip_atomic_store(a.cnt + slice, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   const float* const all = a.part + slice * a.chunks * stride;
+  // the first chunks' outputs travel with the maxima and sums
+  constexpr int AHEAD = 12;
+  auto part_at = [&](int cc, int i) {
+    return __hip_atomic_load(all + min(cc, active - 1) * stride + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  };
+  float first[AHEAD];
+#pragma unroll
+  for (int u = 0; u < AHEAD; ++u) first[u] = part_at(u, min(tid, n - 1));
   // lane = chunk (at most 64): its weight relative to the head's maximum
 #pragma unroll
   for (int j = 0; j < HW; ++j) {
@@ -263,18 +315,21 @@ __global__ __launch_bounds__(kAttnThreads) void attn_decode_kernel(AttnDecodeArg
   for (int i = tid; i < n; i += kAttnThreads) {
     const int h = i / D;
     float t = 0.f;
-    int cc = 0;
-    for (; cc + 8 <= active; cc += 8) {
+    if (i != tid) {
+#pragma unroll
+      for (int u = 0; u < AHEAD; ++u) first[u] = part_at(u, i);
+    }
+#pragma unroll
+    for (int u = 0; u < AHEAD; ++u)
+      if (u < active) t = __builtin_fmaf(w_s[u][h], first[u], t);
+    for (int cc = AHEAD; cc < active; cc += 8) {
       float r[8];
 #pragma unroll
-      for (int u = 0; u < 8; ++u)
-        r[u] = __hip_atomic_load(all + (cc + u) * stride + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      for (int u = 0; u < 8; ++u) r[u] = part_at(cc + u, i);
 #pragma unroll
-      for (int u = 0; u < 8; ++u) t = __builtin_fmaf(w_s[cc + u][h], r[u], t);
+      for (int u = 0; u < 8; ++u)
+        if (cc + u < active) t = __builtin_fmaf(w_s[cc + u][h], r[u], t);
     }
-    for (; cc < active; ++cc)
-      t = __builtin_fmaf(w_s[cc][h],
-                         __hip_atomic_load(all + cc * stride + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT), t);
     a.out[(int64_t)h0 * D + i] = float_to_act_bits<DT>(t / l_s[h]);
   }
 }
