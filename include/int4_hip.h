@@ -292,6 +292,15 @@ int w4_rmsnorm(const void* x, const void* delta, const void* weight, int dtype, 
                float eps, void* sum, void* y, void* stream);
 int w4_silu_mul(const void* gate, const void* up, int dtype, int64_t count, void* y, void* stream);
 
+/*
+ * Logits of one token: y [N] = rmsnorm(x + delta) * weight^T with a 16-bit
+ * weight [N, K] (K a multiple of 8, at most 4096; `delta` may be NULL), norm as
+ * in w4_rmsnorm, its result rounded to the dtype, fp32 sums.
+ * No counterpart in the reference (see w4_attention_decode).
+ */
+int w4_norm_head(const void* x, const void* delta, const void* norm_weight, float eps, const void* weight,
+                 int dtype, int64_t N, int64_t K, void* y, void* stream);
+
 #ifdef __cplusplus
 }
 #endif

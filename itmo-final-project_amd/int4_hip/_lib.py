@@ -89,6 +89,7 @@ SIGNATURES = {
                                       _c_vp, _c_vp, _c_i64, _c_i64, _c_vp, _c_vp]),
     "w4_rmsnorm": (_c_int, [_c_vp, _c_vp, _c_vp, _c_int, _c_i64, _c_i64, ctypes.c_float, _c_vp, _c_vp, _c_vp]),
     "w4_silu_mul": (_c_int, [_c_vp, _c_vp, _c_int, _c_i64, _c_vp, _c_vp]),
+    "w4_norm_head": (_c_int, [_c_vp, _c_vp, _c_vp, ctypes.c_float, _c_vp, _c_int, _c_i64, _c_i64, _c_vp, _c_vp]),
 }
 
 _lock = threading.Lock()

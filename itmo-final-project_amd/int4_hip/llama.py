@@ -304,8 +304,12 @@ class LlamaForCausalLM(nn.Module):
                 x, h = _add_norm(x, a, layer.post_attention_layernorm)
                 step = x, layer.mlp(h)
             x, delta = step
-        norm = self.model.norm
-        return self.lm_head(norm(x) if delta is None else _add_norm(x, delta, norm)[1])
+        norm, head = self.model.norm, self.lm_head
+        if x.shape[0] == 1 and _plain(norm, RMSNorm) and _plain(head, nn.Linear) and head.bias is None:
+            y = llama_ops.norm_head(x, delta, norm.weight, norm.eps, head.weight)
+            if y is not None:
+                return y
+        return head(norm(x) if delta is None else _add_norm(x, delta, norm)[1])
 
     @torch.no_grad()
     def prefill(self, ids: torch.Tensor) -> torch.Tensor:

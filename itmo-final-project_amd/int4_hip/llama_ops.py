@@ -215,3 +215,21 @@ def silu_linear(gate, up, weight):
     if rc:
         _lib.check(rc, "w4a16_decode_silu")
     return outs[0]
+
+
+def norm_head(x, delta, weight, eps: float, head):
+    """rmsnorm(x + delta) @ head^T of one row for a 16-bit ``head`` [N, K] in one launch;
+    None where no such launch exists."""
+    if not (x.dim() == 2 and x.shape[0] == 1 and x.shape[1] <= 4096 and head.dim() == 2 and head.dtype == x.dtype
+            and head.shape[1] == x.shape[1] and 0 < head.shape[0] < 1 << 30 and rms_norm_ok(x, weight, delta)
+            and fusable(x, head) and _dense(head)):
+        return None
+    N, K = head.shape
+    y = torch.empty((1, N), dtype=x.dtype, device=x.device)
+    lib = _lib.load()
+    rc = _on(x.device, lambda st: lib.w4_norm_head(
+        x.data_ptr(), None if delta is None else delta.data_ptr(), weight.data_ptr(), eps, head.data_ptr(),
+        _XDT[x.dtype], N, K, y.data_ptr(), st))
+    if rc:
+        _lib.check(rc, "w4_norm_head")
+    return y

@@ -329,3 +329,34 @@ def test_norm_linears_non_finite_rows():
         x[0, 300] = bad
         assert llama_ops.norm_linears(x, None, w, 1e-5, [q])[1][0].isnan().all()
     assert not llama_ops.norm_linears(torch.zeros_like(x), None, w, 1e-5, [q])[1][0].any()
+
+
+# rows at the edges of a wave's 2 / 4 / 8 and of a full round of the grid; widths of
+# one to eight chunks of 512, whole, ragged and short of a chunk
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("K,N", [(8, 1), (512, 9), (520, 40), (1024, 32769), (1536, 130), (2048, 1000),
+                                 (2056, 16385), (2560, 17), (3072, 64), (3584, 33), (4096, 8193), (2048, 66001)])
+def test_norm_head(dtype, K, N):
+    print(f"[norm head] {dtype} K={K} N={N}", flush=True)
+    x, d = randn((1, K), 1, 3.0, dtype=dtype).to(DEV), randn((1, K), 2, dtype=dtype).to(DEV)
+    w, head = (1 + randn((K,), 3, 0.2, dtype=torch.float32)).to(dtype).to(DEV), randn((N, K), 4, 0.02, dtype=dtype).to(DEV)
+    for delta in (None, d):
+        got = llama_ops.norm_head(x, delta, w, 1e-5, head)
+        h = llama_ops.rms_norm(x, w, 1e-5) if delta is None else llama_ops.rms_norm(x, w, 1e-5, delta)[1]
+        want = h.double().cpu() @ head.double().cpu().T  # the rounded norm: its sum is all that may differ
+        # K products of 2^-24 each (random walk), and a last bit of the norm here and there
+        err = (got.double().cpu() - want).abs() / torch.maximum(want.abs(), want.square().mean().sqrt())
+        assert err.max().item() <= 2 * ROUND[dtype] + 1e-4, err.max().item()
+    for bad in (torch.nan, torch.inf):
+        x[0, K - 1] = bad
+        assert llama_ops.norm_head(x, None, w, 1e-5, head).isnan().all()
+
+
+def test_norm_head_refuses_other_heads():
+    x, w = torch.ones((1, 64), device=DEV, dtype=torch.bfloat16), torch.ones(64, device=DEV, dtype=torch.bfloat16)
+    head = torch.ones((16, 64), device=DEV, dtype=torch.bfloat16)
+    assert llama_ops.norm_head(x, None, w, 1e-5, head) is not None
+    wide = torch.ones((16, 128), device=DEV, dtype=torch.bfloat16)
+    for h in (head.half(), head.float(), head.t(), wide, wide[:, :64], wide.view(-1)[4:4 + 1024].view(16, 64)):
+        assert llama_ops.norm_head(x, None, w, 1e-5, h) is None
+    assert llama_ops.norm_head(x.expand(2, 64).contiguous(), None, w, 1e-5, head) is None
