@@ -305,8 +305,15 @@ class LlamaForCausalLM(nn.Module):
                 step = x, layer.mlp(h)
             x, delta = step
         norm, head = self.model.norm, self.lm_head
-        if x.shape[0] == 1 and _plain(norm, RMSNorm) and _plain(head, nn.Linear) and head.bias is None:
-            y = llama_ops.norm_head(x, delta, norm.weight, norm.eps, head.weight)
+        if x.shape[0] == 1 and _plain(norm, RMSNorm) and getattr(head, "bias", head) is None:
+            # the norm inside the launch that reads it
+            from .qlinear import Int4Linear
+            y = None
+            if _plain(head, nn.Linear):
+                y = llama_ops.norm_head(x, delta, norm.weight, norm.eps, head.weight)
+            elif _plain(head, Int4Linear):
+                y = llama_ops.norm_linears(x, delta, norm.weight, norm.eps, [(head.qweight, head.scales, head.zeros)])
+                y = y and y[1][0]
             if y is not None:
                 return y
         return head(norm(x) if delta is None else _add_norm(x, delta, norm)[1])
