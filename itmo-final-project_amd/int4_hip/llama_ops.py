@@ -57,6 +57,8 @@ def _attn_ws_bytes(nh: int, nkv: int, d: int, max_len: int) -> int:
     key = (nh, nkv, d, max_len)
     b = _ATTN_WS.get(key)
     if b is None:
+        if len(_ATTN_WS) > 4096:
+            _ATTN_WS.clear()
         b = _ATTN_WS[key] = _lib.load().w4_attention_decode_workspace_bytes(nh, nkv, d, max_len)
     return b
 
