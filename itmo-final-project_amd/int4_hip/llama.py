@@ -141,8 +141,8 @@ class Attention(nn.Module):
 
     def forward(self, x, cos, sin, kc, vc, pos0: int | None, pos_t: torch.Tensor | None, mask_bias):
         """Prefill (pos0 = 0, T tokens) or one decode token (pos_t = device position,
-        mask_bias [positions] = 0 up to pos_t, -inf past it, or None where
-        the fused decode kernel applies)."""
+        mask_bias [positions] = 0 up to pos_t, -inf past it, or None to let
+        the fused decode kernel take its place where it applies)."""
         T = x.shape[0]
         nq, nk = self.nh * self.d, self.nkv * self.d
         g = self.nh // self.nkv
@@ -150,7 +150,7 @@ class Attention(nn.Module):
         mods = (self.q_proj, self.k_proj, self.v_proj)
         if pos_t is None:
             qo, ko, vo = _grouped(x, mods) if _all_int4(mods) else [m(x) for m in mods]
-            if llama_ops.attention_prefill_ok(x, kc, vc, cos, sin, pos0, self.nh, self.nkv, self.d):
+            if llama_ops.attention_prefill_ok(x, kc, vc, cos, sin, pos0, self.nh, self.nkv, self.d, (qo, ko, vo)):
                 return self.o_proj(llama_ops.attention_prefill(qo, ko, vo, cos, sin, kc, vc, pos0, self.nh, self.nkv,
                                                                self.d))
             q = apply_rope(qo.view(T, self.nh, self.d), cos, sin)
@@ -169,11 +169,15 @@ class Attention(nn.Module):
             o = torch.bmm(torch.softmax(s, dim=-1), vv)                   # [kv, g*T, D]
             o = o.view(self.nkv, g, T, self.d).permute(2, 0, 1, 3).reshape(T, nq)
         else:
-            if mask_bias is None:  # one fused launch (the caller found it applicable)
+            if mask_bias is None:  # one fused launch, unless a projection's output has to stay a torch operand
                 qo, ko, vo = _grouped(x, mods) if _all_int4(mods) else [m(x) for m in mods]
-                return self.o_proj(llama_ops.attention_decode(qo, ko, vo, cos, sin, kc, vc, pos_t, self.nh, self.nkv,
-                                                              self.d))
-            if _all_int4(mods):
+                if llama_ops.attention_decode_ok(x, kc, vc, cos, sin, pos_t, self.nh, self.nkv, self.d, (qo, ko, vo)):
+                    return self.o_proj(llama_ops.attention_decode(qo, ko, vo, cos, sin, kc, vc, pos_t, self.nh,
+                                                                  self.nkv, self.d))
+                past = torch.arange(kc.shape[-1], device=x.device) > pos_t
+                mask_bias = torch.zeros(kc.shape[-1], device=x.device).masked_fill_(past, float("-inf"))
+                qkv = torch.cat([t.reshape(1, -1) for t in (qo, ko, vo)], dim=-1)
+            elif _all_int4(mods):
                 qkv = torch.empty((1, nq + 2 * nk), dtype=x.dtype, device=x.device)
                 _grouped(x, mods, qkv)
             else:

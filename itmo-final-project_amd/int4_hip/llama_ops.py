@@ -63,13 +63,24 @@ def _attn_ws_bytes(nh: int, nkv: int, d: int, max_len: int) -> int:
     return b
 
 
-def attention_decode_ok(x, kc, vc, cos, sin, pos, nh: int, nkv: int, d: int) -> bool:
+def _qkv_fit(x, qkv, nh: int, nkv: int, d: int) -> bool:
+    """Projections of ``x`` [.., hidden] in its dtype and in the shapes the attention
+    kernels read by pointer (``fusable`` answers for the rest)."""
+    q, k, v = qkv
+    lead = x.shape[:-1]
+    return (q.dtype == k.dtype == v.dtype == x.dtype and q.shape == (*lead, nh * d)
+            and k.shape == v.shape == (*lead, nkv * d))
+
+
+def attention_decode_ok(x, kc, vc, cos, sin, pos, nh: int, nkv: int, d: int, qkv=()) -> bool:
     """Whether ``attention_decode`` takes a step with activations like ``x``
-    ([1, hidden]) and the caches ``kc`` [.., nkv, d, L], ``vc`` [.., nkv, L, d]."""
+    ([1, hidden]), the caches ``kc`` [.., nkv, d, L], ``vc`` [.., nkv, L, d] and, where
+    they are known, the projections ``qkv``."""
     return (x.shape[0] == 1 and x.dtype in _XDT and kc.dtype == vc.dtype == cos.dtype == sin.dtype == torch.float32
             and pos.dtype == torch.int64 and pos.numel() == 1 and cos.shape == sin.shape == (1, d // 2)
             and kc.is_contiguous() and vc.is_contiguous() and cos.is_contiguous() and sin.is_contiguous()
-            and fusable(x, kc, vc, cos, sin, pos) and _attn_ws_bytes(nh, nkv, d, kc.shape[-1]) > 0)
+            and (not qkv or _qkv_fit(x, qkv, nh, nkv, d))
+            and fusable(x, kc, vc, cos, sin, pos, *qkv) and _attn_ws_bytes(nh, nkv, d, kc.shape[-1]) > 0)
 
 
 def attention_decode(q, k, v, cos, sin, kc, vc, pos, nh: int, nkv: int, d: int) -> torch.Tensor:
@@ -90,16 +101,16 @@ def attention_decode(q, k, v, cos, sin, kc, vc, pos, nh: int, nkv: int, d: int) 
     return out
 
 
-def attention_prefill_ok(x, kc, vc, cos, sin, pos0, nh: int, nkv: int, d: int) -> bool:
+def attention_prefill_ok(x, kc, vc, cos, sin, pos0, nh: int, nkv: int, d: int, qkv=()) -> bool:
     """Whether ``attention_prefill`` takes the tokens of ``x`` [T, hidden] at positions
-    pos0.. of the caches ``kc`` [nkv, d, L], ``vc`` [nkv, L, d]."""
+    pos0.. of the caches ``kc`` [nkv, d, L], ``vc`` [nkv, L, d], and their projections ``qkv``."""
     T, L = x.shape[0], kc.shape[-1]
     return (x.dim() == 2 and T >= 1 and d in (64, 128) and nh % nkv == 0 and type(pos0) is int
             and 0 <= pos0 <= L - T and L < 1 << 22 and T <= 65535 * 16 and nkv <= 65535
             and x.dtype in _XDT and kc.dtype == vc.dtype == cos.dtype == sin.dtype == torch.float32
             and kc.shape == (nkv, d, L) and vc.shape == (nkv, L, d) and cos.shape == sin.shape == (T, d // 2)
             and kc.is_contiguous() and cos.is_contiguous() and sin.is_contiguous()
-            and fusable(x, kc, vc, cos, sin) and _dense(vc))
+            and (not qkv or _qkv_fit(x, qkv, nh, nkv, d)) and fusable(x, kc, vc, cos, sin, *qkv) and _dense(vc))
 
 
 def attention_prefill(q, k, v, cos, sin, kc, vc, pos0: int, nh: int, nkv: int, d: int) -> torch.Tensor:

@@ -360,3 +360,74 @@ def test_norm_head_refuses_other_heads():
     for h in (head.half(), head.float(), head.t(), wide, wide[:, :64], wide.view(-1)[4:4 + 1024].view(16, 64)):
         assert llama_ops.norm_head(x, None, w, 1e-5, h) is None
     assert llama_ops.norm_head(x.expand(2, 64).contiguous(), None, w, 1e-5, head) is None
+
+
+def _attention_pair(dtype):
+    """An Attention module on the GPU and its copy on the CPU, trainable 16-bit projections."""
+    import copy
+    from int4_hip.llama import Attention, LlamaConfig
+    cpu = Attention(LlamaConfig(hidden_size=128, num_attention_heads=4, num_key_value_heads=2, head_dim=64))
+    with torch.no_grad():
+        for i, w in enumerate(cpu.parameters()):
+            w.copy_(randn(tuple(w.shape), 70 + i, 0.1, dtype=torch.float32))
+    cpu = cpu.to(dtype)
+    return copy.deepcopy(cpu).to(DEV), cpu
+
+
+def _run_attention(att, dev, x, decode):
+    cos, sin = (t[3:4] if decode else t[:x.shape[0]] for t in _tables(16, 64))
+    kc, vc = torch.zeros((2, 64, 16)), torch.zeros((2, 16, 64))
+    kc[..., :3], vc[:, :3] = randn((2, 64, 3), 80, dtype=torch.float32), randn((2, 3, 64), 81, dtype=torch.float32)
+    args = [t.to(dev) for t in (x, cos.contiguous(), sin.contiguous(), kc, vc)]
+    return att(*args, None, torch.tensor([3], device=dev), None) if decode else att(*args, 0, None, None)
+
+
+# x plain, the projections trainable (a frozen embedding, adapters): every gradient
+# flows.  Both sides round each projection, the attention output and their gradients
+# to 16 bits (on the CPU one side is at most 1.5 half-ulps from 32-bit arithmetic)
+@pytest.mark.parametrize("decode", [False, True])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_attention_keeps_the_gradients_of_its_projections(dtype, decode):
+    gpu, cpu = _attention_pair(dtype)
+    x = randn((1 if decode else 9, 128), 82, dtype=dtype)
+    outs = [_run_attention(a, dev, x, decode) for a, dev in ((gpu, DEV), (cpu, "cpu"))]
+    for o in outs:
+        o.float().square().sum().backward()
+    assert (outs[0].cpu().float() - outs[1].float()).norm() <= 4 * ROUND[dtype] * outs[1].float().norm()
+    for (name, a), b in zip(gpu.named_parameters(), cpu.parameters()):
+        assert a.grad is not None, name
+        assert (a.grad.cpu().float() - b.grad.float()).norm() <= 8 * ROUND[dtype] * b.grad.float().norm(), name
+
+
+class _Out(torch.nn.Module):
+    """A projection whose output is changed by ``f``."""
+
+    def __init__(self, inner, f):
+        super().__init__()
+        self.inner, self.f = inner, f
+
+    def forward(self, x):
+        return self.f(self.inner(x))
+
+
+class _Sub(torch.Tensor):
+    pass
+
+
+@pytest.mark.parametrize("decode", [False, True])
+@pytest.mark.parametrize("form", ["fp32", "one_fp32", "heads", "subclass"])
+def test_attention_takes_other_projection_outputs(form, decode):
+    """Outputs the kernels do not read as they are (fp32, [T, heads, d], a subclass) go through
+    the torch operations, as on the CPU."""
+    f = {"fp32": torch.Tensor.float, "one_fp32": torch.Tensor.float, "heads": lambda t: t.view(t.shape[0], -1, 64),
+         "subclass": lambda t: t.as_subclass(_Sub)}[form]
+    x = randn((1 if decode else 9, 128), 83)
+    outs = []
+    for att, dev in zip(_attention_pair(torch.bfloat16), (DEV, "cpu")):
+        for n in ("k_proj",) if form == "one_fp32" else ("q_proj", "k_proj", "v_proj"):
+            setattr(att, n, _Out(getattr(att, n), f))
+        with torch.no_grad():
+            outs.append(_run_attention(att, dev, x, decode))
+    assert outs[0].dtype == outs[1].dtype == x.dtype and isinstance(outs[0], _Sub) == (form == "subclass")
+    got, want = (o.as_subclass(torch.Tensor).cpu().float() for o in outs)
+    assert (got - want).norm() <= 4 * ROUND[x.dtype] * want.norm()
