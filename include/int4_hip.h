@@ -252,7 +252,7 @@ int w4a16_decode_silu(const w4a16_problem* problem, int x_dtype, const void* up,
  * V over positions 0..*pos in fp32, rounded once into out [num_heads *
  * head_dim].  q [num_heads * head_dim], k and v [num_kv_heads * head_dim] of
  * dtype bf16 / fp16, dense.  head_dim 64 or 128; num_heads a multiple of
- * num_kv_heads.  A *pos outside [0, max_len) leaves caches and out untouched.
+ * num_kv_heads.  A *pos outside [0, max_len) leaves the caches untouched and out all NaN.
  * workspace: as for w4a16_gemm (256-byte aligned, counter area zero),
  * w4_attention_decode_workspace_bytes long (0: not a supported shape).
  * No counterpart in the reference, whose model is Hugging Face's

@@ -141,7 +141,12 @@ __global__ __launch_bounds__(kAttnThreads) void attn_decode_kernel(AttnDecodeArg
   load_v(c0);
   __builtin_amdgcn_sched_barrier(0);
 
-  if (pos64 < 0 || pos64 >= a.max_len) return;  // the caller's table lookup refuses such a position
+  if (pos64 < 0 || pos64 >= a.max_len) {  // no such place in the cache: a defined output, nothing else
+    if (c == 0)
+      for (int i = tid; i < g * D; i += kAttnThreads)
+        a.out[(int64_t)h0 * D + i] = float_to_act_bits<DT>(__builtin_nanf(""));
+    return;
+  }
   const int pos = (int)pos64;
   const int active = pos / a.chunk + 1;
   if (c >= active) return;

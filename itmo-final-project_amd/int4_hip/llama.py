@@ -289,11 +289,15 @@ class LlamaForCausalLM(nn.Module):
     def _layers(self, x, cos, sin, pos0, pos_t):
         mask_bias = None
         c = self.config
-        # (another attention module, or a hook on one, gets the mask)
-        if pos_t is not None and not (all(_plain(layer.self_attn, Attention) for layer in self.model.layers)
-                                      and llama_ops.attention_decode_ok(
-                                          x, self.kc, self.vc, cos, sin, pos_t, c.num_attention_heads,
-                                          c.num_key_value_heads, c.head_dim)):
+        heads = (c.num_attention_heads, c.num_key_value_heads, c.head_dim)
+        # Another attention module, or a hook on one, gets the mask.  So do tables
+        # longer than the cache: looking the angles up refuses a position past the
+        # cache only if the tables end with it.
+        if pos_t is not None and not (
+                all(_plain(a, Attention) and (a.nh, a.nkv, a.d) == heads
+                    for a in (layer.self_attn for layer in self.model.layers))
+                and max(len(self.cos), len(self.sin)) <= self.kc.shape[-1]
+                and llama_ops.attention_decode_ok(x, self.kc, self.vc, cos, sin, pos_t, *heads)):
             mask_bias = torch.zeros(self.max_len, device=x.device).masked_fill_(self.key_pos > pos_t, float("-inf"))
         # each residual addition is fused with the norm that follows it
         delta = None

@@ -76,11 +76,14 @@ def attention_decode_ok(x, kc, vc, cos, sin, pos, nh: int, nkv: int, d: int, qkv
     """Whether ``attention_decode`` takes a step with activations like ``x``
     ([1, hidden]), the caches ``kc`` [.., nkv, d, L], ``vc`` [.., nkv, L, d] and, where
     they are known, the projections ``qkv``."""
-    return (x.shape[0] == 1 and x.dtype in _XDT and kc.dtype == vc.dtype == cos.dtype == sin.dtype == torch.float32
-            and pos.dtype == torch.int64 and pos.numel() == 1 and cos.shape == sin.shape == (1, d // 2)
+    L = kc.shape[-1]
+    return (kc.shape[-3:] == (nkv, d, L) and vc.shape == (*kc.shape[:-3], nkv, L, d)
+            and x.shape[0] == 1 and x.dtype in _XDT
+            and kc.dtype == vc.dtype == cos.dtype == sin.dtype == torch.float32 and pos.dtype == torch.int64
+            and pos.numel() == 1 and cos.shape == sin.shape == (1, d // 2)
             and kc.is_contiguous() and vc.is_contiguous() and cos.is_contiguous() and sin.is_contiguous()
             and (not qkv or _qkv_fit(x, qkv, nh, nkv, d))
-            and fusable(x, kc, vc, cos, sin, pos, *qkv) and _attn_ws_bytes(nh, nkv, d, kc.shape[-1]) > 0)
+            and fusable(x, kc, vc, cos, sin, pos, *qkv) and _attn_ws_bytes(nh, nkv, d, L) > 0)
 
 
 def attention_decode(q, k, v, cos, sin, kc, vc, pos, nh: int, nkv: int, d: int) -> torch.Tensor:

@@ -77,6 +77,19 @@ def test_attention_decode(dtype, nh, nkv, d, max_len, pos):
     _check_out(got, _attention(_rope(q.float().view(1, nh, d), cos, sin), kc, vc, pos), dtype)
 
 
+@pytest.mark.parametrize("nh,nkv,d", [(1, 1, 64), (6, 1, 128), (8, 2, 64)])
+@pytest.mark.parametrize("pos", [-1, 70, 1 << 40])
+def test_attention_decode_outside_the_cache(nh, nkv, d, pos):
+    """A position the cache does not hold: the caches as they were, a NaN output."""
+    q, k, v = (randn((1, n * d), seed=i).to(DEV) for i, n in enumerate((nh, nkv, nkv)))
+    kc, vc = randn((nkv, d, 70), 5, dtype=torch.float32).to(DEV), randn((nkv, 70, d), 6, dtype=torch.float32).to(DEV)
+    row = torch.ones((1, d // 2), device=DEV)
+    before = kc.clone(), vc.clone()
+    out = llama_ops.attention_decode(q, k, v, row, row, kc, vc, torch.tensor([pos], device=DEV), nh, nkv, d)
+    assert out.shape == (1, nh * d) and out.isnan().all()
+    assert torch.equal(kc, before[0]) and torch.equal(vc, before[1])
+
+
 # tokens at the edges of a 16- / 32-query tile and of the 64-position blocks, a
 # prompt continued at pos0, cache ends inside a block, odd and even heads per
 # key-value head, cache rows that are no multiple of 16 bytes

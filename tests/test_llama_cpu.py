@@ -4,7 +4,8 @@ static-cache decode step against the prefill logits."""
 import pytest
 import torch
 
-from int4_hip.llama import LlamaConfig, LlamaForCausalLM
+from int4_hip import llama_ops
+from int4_hip.llama import Attention, LlamaConfig, LlamaForCausalLM
 
 TINY = LlamaConfig(vocab_size=97, hidden_size=64, intermediate_size=160, num_hidden_layers=2,
                    num_attention_heads=8, num_key_value_heads=2, head_dim=8, rope_theta=500000.0,
@@ -55,3 +56,40 @@ def test_decode_steps_match_prefill():
     for t in range(10, 30):
         step = m2.decode_step(ids[t:t + 1], torch.tensor([t]))
         torch.testing.assert_close(step[0], full[t], rtol=1e-4, atol=1e-4)
+
+
+def test_decode_kernel_takes_only_caches_of_its_shapes(monkeypatch):
+    """The host rule alone (what it asks about devices set aside): the kernel indexes both
+    caches by the heads, the head size and the keys' length."""
+    monkeypatch.setattr(llama_ops, "fusable", lambda *a: True)
+    monkeypatch.setattr(llama_ops, "_attn_ws_bytes", lambda *a: 1)
+    x, row, pos = torch.zeros(1, 8, dtype=torch.bfloat16), torch.zeros(1, 32), torch.zeros(1, dtype=torch.long)
+
+    def ok(k, v):
+        return llama_ops.attention_decode_ok(x, torch.zeros(k), torch.zeros(v), row, row, pos, 4, 2, 64)
+
+    assert ok((2, 64, 20), (2, 20, 64)) and ok((3, 2, 64, 20), (3, 2, 20, 64))
+    for k, v in (((2, 64, 20), (2, 19, 64)), ((2, 64, 20), (2, 21, 64)), ((2, 64, 20), (1, 20, 64)),
+                 ((1, 64, 20), (1, 20, 64)), ((2, 32, 20), (2, 20, 32)), ((2, 64, 20), (2, 20, 32)),
+                 ((3, 2, 64, 20), (2, 2, 20, 64)), ((64, 20), (20, 64)), ((2, 64, 20), (2 * 20 * 64,))):
+        assert not ok(k, v), (k, v)
+
+
+def _no_kernel(*a):
+    raise AssertionError("the decode kernel was chosen")
+
+
+def test_decode_step_leaves_other_tables_and_heads_to_torch(monkeypatch):
+    """Tables longer than the cache would let a position past it through; an attention module
+    with other heads does not fit the caches (torch says so)."""
+    monkeypatch.setattr(llama_ops, "attention_decode_ok", lambda *a: True)
+    monkeypatch.setattr(llama_ops, "attention_decode", _no_kernel)
+    m, tok, pos = _model(), torch.tensor([3]), torch.tensor([0])
+    with pytest.raises(AssertionError, match="chosen"):
+        m.decode_step(tok, pos)
+    m.cos, m.sin = (torch.cat((t, t)) for t in (m.cos, m.sin))
+    m.decode_step(tok, pos)
+    m = _model()
+    m.model.layers[1].self_attn = Attention(LlamaConfig(**{**vars(TINY), "num_key_value_heads": 4}))
+    with pytest.raises((RuntimeError, IndexError)):
+        m.decode_step(tok, pos)
