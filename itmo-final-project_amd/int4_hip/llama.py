@@ -221,10 +221,11 @@ def _decode_layer(layer, x, delta, cos, sin, kc, vc, pos_t) -> tuple | None:
     still to be made; returns the new (x, delta), or None for any other layer."""
     from .qlinear import Int4Linear
     at, mlp = layer.self_attn, layer.mlp
-    qkv, gate_up = (at.q_proj, at.k_proj, at.v_proj), (mlp.gate_proj, mlp.up_proj)
     if not (_plain(at, Attention) and _plain(mlp, MLP) and _plain(layer.input_layernorm, RMSNorm)
-            and _plain(layer.post_attention_layernorm, RMSNorm)
-            and all(_plain(m, Int4Linear) and m.bias is None for m in (*qkv, *gate_up, at.o_proj, mlp.down_proj))):
+            and _plain(layer.post_attention_layernorm, RMSNorm)):
+        return None  # (another module need not have these linears)
+    qkv, gate_up = (at.q_proj, at.k_proj, at.v_proj), (mlp.gate_proj, mlp.up_proj)
+    if not all(_plain(m, Int4Linear) and m.bias is None for m in (*qkv, *gate_up, at.o_proj, mlp.down_proj)):
         return None
     x, (q, k, v) = _norm_linears(x, delta, layer.input_layernorm, qkv)
     o = at.o_proj(llama_ops.attention_decode(q, k, v, cos, sin, kc, vc, pos_t, at.nh, at.nkv, at.d))

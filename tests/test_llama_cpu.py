@@ -4,7 +4,7 @@ static-cache decode step against the prefill logits."""
 import pytest
 import torch
 
-from int4_hip import llama_ops
+from int4_hip import llama, llama_ops
 from int4_hip.llama import Attention, LlamaConfig, LlamaForCausalLM
 
 TINY = LlamaConfig(vocab_size=97, hidden_size=64, intermediate_size=160, num_hidden_layers=2,
@@ -93,3 +93,12 @@ def test_decode_step_leaves_other_tables_and_heads_to_torch(monkeypatch):
     m.model.layers[1].self_attn = Attention(LlamaConfig(**{**vars(TINY), "num_key_value_heads": 4}))
     with pytest.raises((RuntimeError, IndexError)):
         m.decode_step(tok, pos)
+
+
+def test_decode_layer_leaves_other_modules_alone():
+    """An MLP of another kind need not have this one's linears: not this function's layer."""
+    layer = _model().model.layers[0]
+    assert llama._decode_layer(layer, *[None] * 7) is None  # its linears are not int4
+    for other in (torch.nn.Identity(), torch.nn.Sequential(layer.mlp)):
+        layer.mlp = other
+        assert llama._decode_layer(layer, *[None] * 7) is None
