@@ -64,7 +64,7 @@ class RMSNorm(nn.Module):
     def forward(self, x: torch.Tensor) -> torch.Tensor:
         # one fused kernel; fp32 statistics (the weight is applied before the
         # final rounding, where the Hugging Face layer rounds first)
-        if llama_ops.rms_norm_ok(x, self.weight):
+        if self.eps is not None and llama_ops.rms_norm_ok(x, self.weight):
             return llama_ops.rms_norm(x, self.weight, self.eps)
         return F.rms_norm(x, (x.shape[-1],), self.weight, self.eps)
 
@@ -76,10 +76,15 @@ def _plain(module: nn.Module, cls: type) -> bool:
             and not module._forward_pre_hooks and not nn.modules.module._has_any_global_hook())
 
 
+def _plain_norm(module: nn.Module) -> bool:
+    """A plain RMSNorm with an epsilon of its own (None: the one torch picks)."""
+    return _plain(module, RMSNorm) and module.eps is not None
+
+
 def _add_norm(x: torch.Tensor, delta: torch.Tensor, norm: nn.Module) -> tuple:
     """(x + delta, norm(x + delta)), in one launch where ``norm`` is a plain RMSNorm
     that nothing hooks into."""
-    if _plain(norm, RMSNorm) and llama_ops.rms_norm_ok(x, norm.weight, delta):
+    if _plain_norm(norm) and llama_ops.rms_norm_ok(x, norm.weight, delta):
         return llama_ops.rms_norm(x, norm.weight, norm.eps, delta)
     x = x + delta
     return x, norm(x)
@@ -221,8 +226,8 @@ def _decode_layer(layer, x, delta, cos, sin, kc, vc, pos_t) -> tuple | None:
     still to be made; returns the new (x, delta), or None for any other layer."""
     from .qlinear import Int4Linear
     at, mlp = layer.self_attn, layer.mlp
-    if not (_plain(at, Attention) and _plain(mlp, MLP) and _plain(layer.input_layernorm, RMSNorm)
-            and _plain(layer.post_attention_layernorm, RMSNorm)):
+    if not (_plain(at, Attention) and _plain(mlp, MLP) and _plain_norm(layer.input_layernorm)
+            and _plain_norm(layer.post_attention_layernorm)):
         return None  # (another module need not have these linears)
     qkv, gate_up = (at.q_proj, at.k_proj, at.v_proj), (mlp.gate_proj, mlp.up_proj)
     if not all(_plain(m, Int4Linear) and m.bias is None for m in (*qkv, *gate_up, at.o_proj, mlp.down_proj)):
@@ -314,7 +319,7 @@ class LlamaForCausalLM(nn.Module):
                 step = x, layer.mlp(h)
             x, delta = step
         norm, head = self.model.norm, self.lm_head
-        if x.shape[0] == 1 and _plain(norm, RMSNorm) and getattr(head, "bias", head) is None:
+        if x.shape[0] == 1 and _plain_norm(norm) and getattr(head, "bias", head) is None:
             # the norm inside the launch that reads it
             from .qlinear import Int4Linear
             y = None

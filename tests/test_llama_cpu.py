@@ -102,3 +102,16 @@ def test_decode_layer_leaves_other_modules_alone():
     for other in (torch.nn.Identity(), torch.nn.Sequential(layer.mlp)):
         layer.mlp = other
         assert llama._decode_layer(layer, *[None] * 7) is None
+
+
+def test_norm_without_an_epsilon_is_left_to_torch(monkeypatch):
+    """eps=None means torch's choice; the kernels take a number."""
+    m = _model()
+    for n in [m.model.norm] + [n for l in m.model.layers for n in (l.input_layernorm, l.post_attention_layernorm)]:
+        n.eps = None
+    want = m.prefill(torch.arange(5)), m.decode_step(torch.tensor([3]), torch.tensor([5]))
+    monkeypatch.setattr(llama_ops, "rms_norm_ok", lambda *a: True)
+    for f in ("rms_norm", "norm_linears", "norm_head"):
+        monkeypatch.setattr(llama_ops, f, _no_kernel)
+    assert torch.equal(m.prefill(torch.arange(5)), want[0])
+    assert torch.equal(m.decode_step(torch.tensor([3]), torch.tensor([5])), want[1])
