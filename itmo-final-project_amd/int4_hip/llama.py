@@ -36,6 +36,7 @@ import torch.nn as nn
 import torch.nn.functional as F
 
 from . import llama_ops
+from .qlinear import Int4Linear
 
 
 @dataclass
@@ -70,10 +71,12 @@ class RMSNorm(nn.Module):
 
 
 def _plain(module: nn.Module, cls: type) -> bool:
-    """Whether calling ``module`` runs ``cls.forward`` and nothing else (no subclass,
-    replaced forward or hook), so that a fused kernel may stand for the call."""
-    return (type(module) is cls and "forward" not in module.__dict__ and not module._forward_hooks
-            and not module._forward_pre_hooks and not nn.modules.module._has_any_global_hook())
+    """Whether calling ``module`` runs ``cls``'s own forward and nothing else (no subclass,
+    hook, or forward replaced on the module or the class), so that a fused kernel may
+    stand for the call."""
+    return (type(module) is cls and cls.forward is _FORWARD[cls] and "forward" not in module.__dict__
+            and not module._forward_hooks and not module._forward_pre_hooks
+            and not nn.modules.module._has_any_global_hook())
 
 
 def _plain_norm(module: nn.Module) -> bool:
@@ -117,7 +120,6 @@ def apply_rope(x: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor) -> torch.T
 
 
 def _all_int4(mods) -> bool:
-    from .qlinear import Int4Linear
     return all(isinstance(m, Int4Linear) for m in mods) and len({m.group_size for m in mods}) == 1
 
 
@@ -224,7 +226,6 @@ def _decode_layer(layer, x, delta, cos, sin, kc, vc, pos_t) -> tuple | None:
     Int4Linear without bias: five launches, the norms and the gated activation
     computed by the linears that read them.  ``delta`` is the residual addition
     still to be made; returns the new (x, delta), or None for any other layer."""
-    from .qlinear import Int4Linear
     at, mlp = layer.self_attn, layer.mlp
     if not (_plain(at, Attention) and _plain(mlp, MLP) and _plain_norm(layer.input_layernorm)
             and _plain_norm(layer.post_attention_layernorm)):
@@ -247,6 +248,10 @@ class DecoderLayer(nn.Module):
         self.self_attn = Attention(cfg)
         self.post_attention_layernorm = RMSNorm(cfg.hidden_size, cfg.rms_norm_eps)
         self.mlp = MLP(cfg)
+
+
+# the forwards that the fused kernels stand for
+_FORWARD = {cls: cls.forward for cls in (RMSNorm, Attention, MLP, Int4Linear, nn.Linear)}
 
 
 class LlamaBody(nn.Module):
@@ -321,7 +326,6 @@ class LlamaForCausalLM(nn.Module):
         norm, head = self.model.norm, self.lm_head
         if x.shape[0] == 1 and _plain_norm(norm) and getattr(head, "bias", head) is None:
             # the norm inside the launch that reads it
-            from .qlinear import Int4Linear
             y = None
             if _plain(head, nn.Linear):
                 y = llama_ops.norm_head(x, delta, norm.weight, norm.eps, head.weight)
@@ -350,7 +354,6 @@ class LlamaForCausalLM(nn.Module):
 
 def linear_weight_bytes(model: nn.Module, include_lm_head: bool = False) -> int:
     """Bytes of the decoder linears' weights (eval_llama.py:52-62)."""
-    from .qlinear import Int4Linear
     total = 0
     for name, m in model.named_modules():
         if "lm_head" in name and not include_lm_head:
@@ -514,7 +517,6 @@ def run_eval(prompt_len: int = 512, new_tokens: int = 128, group_size: int = 128
 def dequantize_model_linears(model: nn.Module) -> nn.Module:
     """Replace every Int4Linear by an nn.Linear holding its dequantized weight
     (the state quantize_model_linears(..., fake=True) produces)."""
-    from .qlinear import Int4Linear
     for prefix, parent in list(model.named_modules()):
         for name, child in list(parent.named_children()):
             if isinstance(child, Int4Linear):

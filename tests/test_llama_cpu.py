@@ -4,6 +4,7 @@ static-cache decode step against the prefill logits."""
 import pytest
 import torch
 
+import int4_hip
 from int4_hip import llama, llama_ops
 from int4_hip.llama import Attention, LlamaConfig, LlamaForCausalLM
 
@@ -115,3 +116,18 @@ def test_norm_without_an_epsilon_is_left_to_torch(monkeypatch):
         monkeypatch.setattr(llama_ops, f, _no_kernel)
     assert torch.equal(m.prefill(torch.arange(5)), want[0])
     assert torch.equal(m.decode_step(torch.tensor([3]), torch.tensor([5])), want[1])
+
+
+@pytest.mark.parametrize("cls", [llama.RMSNorm, llama.Attention, llama.MLP, int4_hip.Int4Linear, torch.nn.Linear])
+def test_a_forward_replaced_on_the_class_counts(cls, monkeypatch):
+    """A forward patched on the class (profilers, other kernels) is no longer the one the fused
+    launches stand for."""
+    m = _model()
+    mod = {llama.RMSNorm: m.model.norm, llama.Attention: m.model.layers[0].self_attn,
+           llama.MLP: m.model.layers[0].mlp, torch.nn.Linear: m.lm_head}.get(cls) or int4_hip.Int4Linear(64, 64, 32)
+    assert llama._plain(mod, cls)
+    own = cls.forward
+    with monkeypatch.context() as patch:
+        patch.setattr(cls, "forward", lambda self, *a: own(self, *a))
+        assert not llama._plain(mod, cls)
+    assert llama._plain(mod, cls)
