@@ -263,13 +263,19 @@ PyObject* quant_triple(Quant* a) {
                        THPVariable_Wrap(std::move(a->z)));
 }
 
+// The group size an int names, or 0 (never valid) if it is no int or does not fit 32 bits.
+int64_t group_arg(PyObject* o) {
+  if (!PyLong_CheckExact(o)) return 0;
+  int overflow = 0;
+  const long long g = PyLong_AsLongLongAndOverflow(o, &overflow);
+  return overflow || g < -1 || g > INT32_MAX ? 0 : g;
+}
+
 PyObject* quantize(PyObject*, PyObject* const* args, Py_ssize_t n) {
   HANDLE_TH_ERRORS
-  if (n != 2 || !quiet() || !PyLong_CheckExact(args[1])) Py_RETURN_NONE;
-  const int64_t group = PyLong_AsLongLong(args[1]);
-  if (group == -1 && PyErr_Occurred()) return nullptr;
+  if (n != 2 || !quiet()) Py_RETURN_NONE;
   Quant a;
-  if (!quant_item(args[0], group, &a) || group > INT32_MAX || !current(a.w->device())) Py_RETURN_NONE;
+  if (!quant_item(args[0], group_arg(args[1]), &a) || !current(a.w->device())) Py_RETURN_NONE;
   if (a.G > INT32_MAX) Py_RETURN_NONE;
   quant_outputs(&a);
   void* const stream = c10::hip::getCurrentHIPStream(a.w->device().index()).stream();
@@ -287,11 +293,10 @@ PyObject* quantize(PyObject*, PyObject* const* args, Py_ssize_t n) {
 
 PyObject* quantize_grouped(PyObject*, PyObject* const* args, Py_ssize_t n) {
   HANDLE_TH_ERRORS
-  if (n != 2 || !quiet() || !PyList_CheckExact(args[0]) || !PyLong_CheckExact(args[1])) Py_RETURN_NONE;
-  const int64_t group = PyLong_AsLongLong(args[1]);
-  if (group == -1 && PyErr_Occurred()) return nullptr;
+  if (n != 2 || !quiet() || !PyList_CheckExact(args[0])) Py_RETURN_NONE;
+  const int64_t group = group_arg(args[1]);
   const Py_ssize_t count = PyList_GET_SIZE(args[0]);
-  if (count < 1 || count > W4_MAX_GROUPED || group > INT32_MAX) Py_RETURN_NONE;
+  if (count < 1 || count > W4_MAX_GROUPED) Py_RETURN_NONE;
   std::array<Quant, W4_MAX_GROUPED> it;
   for (Py_ssize_t i = 0; i < count; ++i)
     if (!quant_item(PyList_GET_ITEM(args[0], i), group, &it[i]) || it[i].G > INT32_MAX ||

@@ -142,3 +142,14 @@ def test_threads_and_streams():
     for t in ts:
         t.join()
     assert not bad
+
+
+@pytest.mark.parametrize("group", [1 << 31, 1 << 63, 1 << 70, -(1 << 70), -2])
+def test_group_sizes_no_weight_has(group):
+    """Refused as the general path refuses them, whatever their size."""
+    w = randn((8, 64), 1).to(DEV)
+    int4_hip.quantize_int4(w, 64)  # (loads the library)
+    assert _lib.ext.quantize(w, group) is None and _lib.ext.quantize_grouped([w], group) is None
+    for call in (lambda: int4_hip.quantize_int4(w, group), lambda: int4_hip.quantize_int4_grouped([w], group)):
+        with pytest.raises(AssertionError):
+            call()
