@@ -160,60 +160,59 @@ PyObject* matmul_grouped(PyObject*, PyObject* const* args, Py_ssize_t n) {
   if (count < 1 || count > W4_MAX_GROUPED || PySequence_Fast_GET_SIZE(args[1]) != count ||
       (args[2] != Py_None && PySequence_Fast_GET_SIZE(args[2]) < count))
     Py_RETURN_NONE;
+  // Owned: the workspace callback and the launch let other threads run, which may
+  // take the operands out of the caller's lists.
   struct Item {
-    const at::Tensor *x, *q, *s, *z, *out;
+    at::Tensor x, q, s, z, out;
     int64_t K, N, G;
-  } it[W4_MAX_GROUPED];
+  };
+  std::array<Item, W4_MAX_GROUPED> it;
   int64_t M = 0;
   for (Py_ssize_t i = 0; i < count; ++i) {
     Item& a = it[i];
-    a.x = plain(PySequence_Fast_GET_ITEM(args[0], i));
-    if (!a.x || a.x->dim() < 1 || !a.x->is_contiguous() || a.x->numel() == 0 ||
-        ((uintptr_t)a.x->const_data_ptr() % 16) != 0)
+    const at::Tensor* x = plain(PySequence_Fast_GET_ITEM(args[0], i));
+    if (!x || x->dim() < 1 || !x->is_contiguous() || x->numel() == 0 || ((uintptr_t)x->const_data_ptr() % 16) != 0)
       Py_RETURN_NONE;
-    a.K = a.x->size(-1);
-    const int64_t rows = a.x->numel() / a.K;
+    a.x = *x;
+    a.K = x->size(-1);
+    const int64_t rows = x->numel() / a.K;
     if (i == 0) M = rows;
-    if (rows != M || a.x->scalar_type() != it[0].x->scalar_type() || a.x->device() != it[0].x->device())
-      Py_RETURN_NONE;
+    if (rows != M || x->scalar_type() != it[0].x.scalar_type() || x->device() != it[0].x.device()) Py_RETURN_NONE;
     PyObject* w = PySequence_Fast_GET_ITEM(args[1], i);
     if (!seq(w) || PySequence_Fast_GET_SIZE(w) != 3) Py_RETURN_NONE;
-    a.q = plain(PySequence_Fast_GET_ITEM(w, 0));
-    a.s = plain(PySequence_Fast_GET_ITEM(w, 1));
-    a.z = plain(PySequence_Fast_GET_ITEM(w, 2));
-    a.G = weight_group(a.q, a.s, a.z, a.x->device(), a.K);
+    const at::Tensor *q = plain(PySequence_Fast_GET_ITEM(w, 0)), *s = plain(PySequence_Fast_GET_ITEM(w, 1)),
+                     *z = plain(PySequence_Fast_GET_ITEM(w, 2));
+    a.G = weight_group(q, s, z, x->device(), a.K);
     if (a.G == 0 || a.G > INT32_MAX) Py_RETURN_NONE;
-    a.N = a.q->size(1);
+    a.q = *q;
+    a.s = *s;
+    a.z = *z;
+    a.N = q->size(1);
     if (a.N == 0) Py_RETURN_NONE;
-    a.out = nullptr;
     if (args[2] != Py_None) {
-      a.out = plain(PySequence_Fast_GET_ITEM(args[2], i));
-      if (!a.out || a.x->dim() != 2 || a.out->dim() != 2 || a.out->size(0) != M || a.out->size(1) != a.N ||
-          !a.out->is_contiguous() || a.out->scalar_type() != a.x->scalar_type() ||
-          a.out->device() != a.x->device())
+      const at::Tensor* out = plain(PySequence_Fast_GET_ITEM(args[2], i));
+      if (!out || x->dim() != 2 || out->dim() != 2 || out->size(0) != M || out->size(1) != a.N ||
+          !out->is_contiguous() || out->scalar_type() != x->scalar_type() || out->device() != x->device())
         Py_RETURN_NONE;
+      a.out = *out;
     }
   }
-  const c10::Device dev = it[0].x->device();
-  const int dt = act_code(it[0].x->scalar_type());
+  const c10::Device dev = it[0].x.device();
+  const int dt = act_code(it[0].x.scalar_type());
   if (dt < 0 || !current(dev)) Py_RETURN_NONE;
   w4a16_problem probs[W4_MAX_GROUPED];
-  std::vector<at::Tensor> ys;
-  ys.reserve(count);
   for (Py_ssize_t i = 0; i < count; ++i) {
-    const Item& a = it[i];
-    if (a.out) {
-      ys.push_back(*a.out);
-    } else {
-      std::vector<int64_t> sizes(a.x->sizes().begin(), a.x->sizes().end());
+    Item& a = it[i];
+    if (!a.out.defined()) {
+      std::vector<int64_t> sizes(a.x.sizes().begin(), a.x.sizes().end());
       sizes.back() = a.N;
-      ys.push_back(empty(sizes, a.x->scalar_type(), dev));
+      a.out = empty(sizes, a.x.scalar_type(), dev);
     }
-    probs[i] = w4a16_problem{a.x->const_data_ptr(),
-                             static_cast<const int32_t*>(a.q->const_data_ptr()),
-                             static_cast<const uint16_t*>(a.s->const_data_ptr()),
-                             static_cast<const uint16_t*>(a.z->const_data_ptr()),
-                             ys.back().mutable_data_ptr(),
+    probs[i] = w4a16_problem{a.x.const_data_ptr(),
+                             static_cast<const int32_t*>(a.q.const_data_ptr()),
+                             static_cast<const uint16_t*>(a.s.const_data_ptr()),
+                             static_cast<const uint16_t*>(a.z.const_data_ptr()),
+                             a.out.mutable_data_ptr(),
                              a.N,
                              a.K,
                              (int32_t)a.G,
@@ -230,7 +229,7 @@ PyObject* matmul_grouped(PyObject*, PyObject* const* args, Py_ssize_t n) {
   if (!check(rc, "w4a16_gemm_grouped")) return nullptr;
   PyObject* list = PyList_New(count);
   if (!list) return nullptr;
-  for (Py_ssize_t i = 0; i < count; ++i) PyList_SET_ITEM(list, i, THPVariable_Wrap(ys[i]));
+  for (Py_ssize_t i = 0; i < count; ++i) PyList_SET_ITEM(list, i, THPVariable_Wrap(std::move(it[i].out)));
   return list;
   END_HANDLE_TH_ERRORS
 }

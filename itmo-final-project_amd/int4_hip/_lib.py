@@ -100,7 +100,7 @@ _lib = None
 ext = None
 
 
-def _load_ext(lib):
+def _load_ext(lib, workspace=None):
     from . import gemm
     try:
         from . import _int4_torch
@@ -109,7 +109,8 @@ def _load_ext(lib):
                            f"torch ({e}); run `python itmo-final-project_amd/build_lib.py`") from e
     names = ("w4a16_gemm", "w4a16_workspace_bytes", "w4a16_gemm_grouped", "w4a16_grouped_workspace_bytes",
              "w4_quantize_grouped", "w4_quantize", "w4_dequantize")
-    _int4_torch.init(tuple(ctypes.cast(getattr(lib, n), _c_vp).value for n in names), gemm._workspace_address, check)
+    _int4_torch.init(tuple(ctypes.cast(getattr(lib, n), _c_vp).value for n in names),
+                     workspace or gemm._workspace_address, check)
     return _int4_torch
 
 

@@ -153,3 +153,28 @@ def test_group_sizes_no_weight_has(group):
     for call in (lambda: int4_hip.quantize_int4(w, group), lambda: int4_hip.quantize_int4_grouped([w], group)):
         with pytest.raises(AssertionError):
             call()
+
+
+def test_grouped_operands_outlive_the_callers_lists():
+    """Another thread may take the operands out of the lists while the call waits for its
+    workspace: it holds them itself."""
+    from int4_hip import gemm
+    q = int4_hip.quantize_int4(randn((2048, 8192), 1, 0.02).to(DEV), 128)
+    x = randn((1, 8192), 2).to(DEV)
+    assert int4_hip.gemm.grouped_workspace_bytes([x], [q]) > 0
+    want = int4_hip.w4a16_matmul_grouped([x], [q])[0].clone()
+    xs, ws, seen = [x.clone()], [tuple(t.clone() for t in q)], []
+
+    def workspace(*args):
+        sizes = [(t.shape, t.dtype) for t in (xs[0], *ws[0])]
+        xs.clear(), ws.clear()
+        seen.extend(torch.empty(s, dtype=d, device=DEV).fill_(1) for s, d in sizes)  # where they were, if freed
+        return gemm._workspace_address(*args)
+
+    lib = _lib.load()
+    try:
+        _lib._load_ext(lib, workspace)
+        got = _lib.ext.matmul_grouped(xs, ws, None)[0]
+    finally:
+        _lib._load_ext(lib)
+    assert len(seen) == 4 and torch.equal(got, want)
