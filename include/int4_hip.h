@@ -280,12 +280,12 @@ int w4_attention_prefill(const void* q, const void* k, const void* v, int dtype,
                          void* out, void* stream);
 
 /*
- * RMSNorm of `rows` dense rows of n values (bf16 / fp16; n a multiple of 8, at
- * most 16384; operands 16-byte aligned): y = x / sqrt(mean(x^2) + eps) *
+ * RMSNorm of `rows` (below 2^24) dense rows of n values (bf16 / fp16; n a
+ * multiple of 8, at most 16384; operands 16-byte aligned): y = x / sqrt(mean(x^2) + eps) *
  * weight, fp32 inside, rounded once.  With `delta` (else NULL, and sum NULL)
  * the input is x + delta rounded to the dtype, which is written to `sum`.
- * w4_silu_mul: y = silu(gate) * up over `count` values (a multiple of 8),
- * fp32 inside, rounded once.
+ * w4_silu_mul: y = silu(gate) * up over `count` values (a multiple of 8 below
+ * 2^35), fp32 inside, rounded once.
  * No counterpart in the reference (see w4_attention_decode).
  */
 int w4_rmsnorm(const void* x, const void* delta, const void* weight, int dtype, int64_t rows, int64_t n,

@@ -984,6 +984,9 @@ extern "C" int w4_attention_decode(const void* q, const void* k, const void* v, 
 
 namespace {
 
+// HIP refuses launches of 2^32 threads and more.
+constexpr int64_t kMaxGrid256 = 0xFFFFFFFFll / 256;
+
 template <int DT, bool ADD>
 void launch_rmsnorm(const uint16_t* x, const uint16_t* delta, const uint16_t* weight, int64_t rows, int n, float eps,
                     uint16_t* sum, uint16_t* y, hipStream_t st) {
@@ -1005,7 +1008,7 @@ extern "C" int w4_rmsnorm(const void* x, const void* delta, const void* weight, 
   clear_error();
   if (dtype != W4_DTYPE_BF16 && dtype != W4_DTYPE_FP16)
     return fail(W4_ERR_INVALID, "w4_rmsnorm: dtype must be bf16 or fp16 (got code %d)", dtype);
-  if (rows < 0 || rows >= (1LL << 31) || n < 8 || n % 8 != 0 || n > 8 * w4::kNormThreads * w4::kNormMaxVecs)
+  if (rows < 0 || rows > kMaxGrid256 || n < 8 || n % 8 != 0 || n > 8 * w4::kNormThreads * w4::kNormMaxVecs)
     return fail(W4_ERR_UNSUPPORTED, "w4_rmsnorm: %lld rows of %lld (a multiple of 8, at most %d)", (long long)rows,
                 (long long)n, 8 * w4::kNormThreads * w4::kNormMaxVecs);
   if (rows == 0) return W4_OK;
@@ -1031,8 +1034,8 @@ extern "C" int w4_silu_mul(const void* gate, const void* up, int dtype, int64_t 
   clear_error();
   if (dtype != W4_DTYPE_BF16 && dtype != W4_DTYPE_FP16)
     return fail(W4_ERR_INVALID, "w4_silu_mul: dtype must be bf16 or fp16 (got code %d)", dtype);
-  if (count < 0 || count % 8 != 0 || count / 8 >= (1LL << 31) * 256)
-    return fail(W4_ERR_UNSUPPORTED, "w4_silu_mul: %lld values (a multiple of 8)", (long long)count);
+  if (count < 0 || count % 8 != 0 || count / 8 > kMaxGrid256 * 256)
+    return fail(W4_ERR_UNSUPPORTED, "w4_silu_mul: %lld values (a multiple of 8, below 2^35)", (long long)count);
   if (count == 0) return W4_OK;
   if (!gate || !up || !y) return fail(W4_ERR_INVALID, "w4_silu_mul: null pointer");
   if ((((uintptr_t)gate | (uintptr_t)up | (uintptr_t)y) % 16) != 0)

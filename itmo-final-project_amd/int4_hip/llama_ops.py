@@ -132,7 +132,8 @@ def attention_prefill(q, k, v, cos, sin, kc, vc, pos0: int, nh: int, nkv: int, d
     return out
 
 
-MAX_NORM = 16384  # widest row of w4_rmsnorm
+MAX_NORM = 16384                # widest row of w4_rmsnorm
+MAX_GRID = (2**32 - 1) // 256   # workgroups of 256 threads in a launch: a row, or 2048 values, each
 
 
 def rms_norm_ok(x, weight, delta=None) -> bool:
@@ -140,6 +141,7 @@ def rms_norm_ok(x, weight, delta=None) -> bool:
     n = x.shape[-1] if x.dim() else 0
     ts = (x, weight) if delta is None else (x, weight, delta)
     return (x.dtype in _XDT and 0 < n <= MAX_NORM and n % 8 == 0 and weight.shape == (n,)
+            and x.numel() <= MAX_GRID * n
             and all(t.dtype == x.dtype for t in ts) and (delta is None or delta.shape == x.shape)
             and fusable(*ts) and _dense(*ts))
 
@@ -160,7 +162,7 @@ def rms_norm(x, weight, eps: float, delta=None):
 
 def silu_mul_ok(gate, up) -> bool:
     return (gate.dtype in _XDT and up.dtype == gate.dtype and up.shape == gate.shape and gate.numel() % 8 == 0
-            and fusable(gate, up) and _dense(gate, up))
+            and gate.numel() <= MAX_GRID * 2048 and fusable(gate, up) and _dense(gate, up))
 
 
 def silu_mul(gate, up) -> torch.Tensor:

@@ -114,6 +114,9 @@ def test_c_abi_rejects_bad_norm_and_activation_arguments(lib):
     assert lib.w4_silu_mul(fake, None, 0, 8, fake, None) == _lib.ERR_INVALID
     assert lib.w4_silu_mul(fake, fake, 0, 12, fake, None) == _lib.ERR_UNSUPPORTED
     assert lib.w4_silu_mul(None, None, 0, 0, None, None) == _lib.OK
+    # launches of 2^32 threads and more
+    assert norm(rows=1 << 24) == _lib.ERR_UNSUPPORTED
+    assert lib.w4_silu_mul(fake, fake, 0, 1 << 35, fake, None) == _lib.ERR_UNSUPPORTED
     assert lib.w4_norm_head(fake, None, fake, 1e-5, fake, 2, 8, 64, fake, None) == _lib.ERR_INVALID
     assert lib.w4_norm_head(fake, None, fake, 1e-5, odd, 0, 8, 64, fake, None) == _lib.ERR_INVALID
     assert lib.w4_norm_head(fake, None, None, 1e-5, fake, 0, 8, 64, fake, None) == _lib.ERR_INVALID

@@ -131,3 +131,18 @@ def test_a_forward_replaced_on_the_class_counts(cls, monkeypatch):
         patch.setattr(cls, "forward", lambda self, *a: own(self, *a))
         assert not llama._plain(mod, cls)
     assert llama._plain(mod, cls)
+
+
+def test_norm_and_activation_kernels_leave_launches_hip_refuses(monkeypatch):
+    """A workgroup per row, or per 2048 values, of 256 threads: below 2^32 threads in all."""
+    monkeypatch.setattr(llama_ops, "fusable", lambda *a: True)
+    monkeypatch.setattr(llama_ops, "_dense", lambda *a: True)
+
+    def meta(*shape):
+        return torch.empty(shape, dtype=torch.bfloat16, device="meta")
+
+    assert llama_ops.rms_norm_ok(meta((1 << 24) - 1, 8), meta(8))
+    assert not llama_ops.rms_norm_ok(meta(1 << 24, 8), meta(8))
+    assert not llama_ops.rms_norm_ok(meta(1 << 12, 1 << 12, 8), meta(8), meta(1 << 12, 1 << 12, 8))
+    for n, ok in (((1 << 24) - 1, True), (1 << 24, False)):
+        assert llama_ops.silu_mul_ok(meta(n, 2048), meta(n, 2048)) == ok
