@@ -66,16 +66,24 @@ def _compile(src: Path) -> Path:
     return obj
 
 
-def build_ext() -> Path:
-    """Compile int4_hip/_int4_torch.so (host code only) against the installed torch."""
+def build_ext() -> Path | None:
+    """Compile int4_hip/_int4_torch.so (host code only) against the installed torch;
+    None, and no binding, without torch or g++ (the library itself needs neither)."""
     import sysconfig
 
-    import torch
-
+    try:
+        import torch
+    except ImportError:
+        torch = None
+    gxx = shutil.which("g++")
+    if torch is None or gxx is None:
+        print(f"{EXT_LIB.name} not built: {'g++' if torch else 'torch'} not found", file=sys.stderr)
+        EXT_LIB.unlink(missing_ok=True)
+        return None
     root = Path(torch.__file__).resolve().parent
     tmp = EXT_LIB.with_suffix(".so.tmp")
-    cmd = [shutil.which("g++") or "g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-D__HIP_PLATFORM_AMD__=1",
-           "-DUSE_ROCM=1", f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+    cmd = [gxx, "-O2", "-std=c++17", "-fPIC", "-shared", "-D__HIP_PLATFORM_AMD__=1",
+           "-DUSE_ROCM=1", f'-DW4_TORCH_VERSION="{torch.__version__}"', f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
            "-I", str(root / "include"), "-I", str(root / "include" / "torch" / "csrc" / "api" / "include"),
            "-I", str(Path(os.environ.get("ROCM_PATH", "/opt/rocm")) / "include"),
            "-I", sysconfig.get_paths()["include"], "-I", str(ROOT / "include"), str(EXT_SRC), "-o", str(tmp),
@@ -94,7 +102,7 @@ def build(jobs: int | None = None, verbose: bool = True) -> Path:
     with ThreadPoolExecutor(jobs + 1) as ex:
         ext = ex.submit(build_ext)
         objs = list(ex.map(_compile, srcs))
-        ext.result()
+        ext = ext.result()
     tmp = LIB.with_suffix(".so.tmp")
     cmd = [hipcc(), f"--offload-arch={ARCH}", "-shared", "-fPIC", "-o", str(tmp), *map(str, objs)]
     r = subprocess.run(cmd, capture_output=True, text=True)
@@ -111,7 +119,8 @@ def build(jobs: int | None = None, verbose: bool = True) -> Path:
             raise RuntimeError(f"link failed\n{' '.join(cmd)}\n{r.stderr}")
         os.replace(btmp, BENCH_LIB)
     if verbose:
-        print(f"built {LIB} from {len(srcs)} sources (+ {EXT_LIB.name}, {BENCH_LIB.name})", file=sys.stderr)
+        more = ", ".join(p.name for p in (ext, BENCH_LIB) if p)
+        print(f"built {LIB} from {len(srcs)} sources (+ {more})", file=sys.stderr)
     return LIB
 
 

@@ -394,4 +394,9 @@ PyModuleDef module = {PyModuleDef_HEAD_INIT, "_int4_torch", nullptr, -1, methods
 
 }  // namespace
 
-PyMODINIT_FUNC PyInit__int4_torch() { return PyModule_Create(&module); }
+PyMODINIT_FUNC PyInit__int4_torch() {
+  PyObject* m = PyModule_Create(&module);
+  // the torch whose headers this was built from: tensors are read through them
+  if (m && PyModule_AddStringConstant(m, "torch_version", W4_TORCH_VERSION) != 0) Py_CLEAR(m);
+  return m;
+}

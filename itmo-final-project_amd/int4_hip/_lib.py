@@ -8,6 +8,7 @@ from __future__ import annotations
 import ctypes
 import os
 import threading
+import warnings
 from pathlib import Path
 
 LIB_PATH = Path(os.environ.get("INT4_HIP_LIB", Path(__file__).resolve().parent / "libint4_hip.so"))
@@ -96,17 +97,24 @@ _lock = threading.Lock()
 _lib = None
 # int4_hip._int4_torch once the library is loaded: the entry points' native call
 # path for plain operands (csrc/torch_ext/int4_torch.cpp).  Its functions return
-# None for everything else, which the Python code then handles.
+# None for everything else, which the Python code then handles.  None where the
+# binding is not built or was built for another torch: the Python code, which
+# depends on no torch ABI, then makes the same calls, a few microseconds slower.
 ext = None
 
 
 def _load_ext(lib, workspace=None):
+    import torch
+
     from . import gemm
     try:
         from . import _int4_torch
+        if _int4_torch.torch_version != torch.__version__:
+            raise ImportError(f"built for torch {_int4_torch.torch_version}, running {torch.__version__}")
     except ImportError as e:
-        raise RuntimeError(f"int4_hip: the torch binding _int4_torch.so is not built or does not fit the installed "
-                           f"torch ({e}); run `python itmo-final-project_amd/build_lib.py`") from e
+        warnings.warn(f"int4_hip: the native call path _int4_torch.so cannot be used ({e}); calls go through ctypes. "
+                      "Run `python itmo-final-project_amd/build_lib.py` to build it.", RuntimeWarning, stacklevel=3)
+        return None
     names = ("w4a16_gemm", "w4a16_workspace_bytes", "w4a16_gemm_grouped", "w4a16_grouped_workspace_bytes",
              "w4_quantize_grouped", "w4_quantize", "w4_dequantize")
     _int4_torch.init(tuple(ctypes.cast(getattr(lib, n), _c_vp).value for n in names),

@@ -2,7 +2,11 @@
 (C side and Python side, mirroring the reference's assertions), module
 structure.  No GPU compute is issued here."""
 import ctypes
+import os
 import re
+import shutil
+import subprocess
+import sys
 from pathlib import Path
 
 import numpy as np
@@ -431,3 +435,40 @@ def test_pf5_weight_tile_swizzle_is_conflict_free(TS):
     if TS == 128:  # the 64-wide swizzle on this tile's stores: two-way conflicts
         old = lambda n, j: ((n * 8 + (j ^ ((n >> 1) & 7))) * 16 // 4 % 64) // 4
         assert len({old(4 * l, 0) for l in range(8)}) == 4
+
+
+def test_library_loads_without_the_native_call_path(tmp_path):
+    """The binding against torch's C++ ABI is a faster way to the same calls: without it the
+    package warns and goes through ctypes."""
+    pkg = tmp_path / "int4_hip"
+    shutil.copytree(ROOT / "itmo-final-project_amd" / "int4_hip", pkg,
+                    ignore=shutil.ignore_patterns("_int4_torch*", "libw4*", "__pycache__"))
+    code = ("import warnings; from int4_hip import _lib\n"
+            "with warnings.catch_warnings(record=True) as w:\n"
+            "    warnings.simplefilter('always'); lib = _lib.load()\n"
+            "assert _lib.ext is None and lib.w4_abi_version() == _lib.ABI_VERSION\n"
+            "assert any('_int4_torch' in str(x.message) for x in w), w\n"
+            "from int4_hip import gemm\n"
+            "assert gemm._lib is _lib\n")
+    env = {**os.environ, "PYTHONPATH": str(tmp_path)}
+    env.pop("INT4_HIP_LIB", None)
+    r = subprocess.run([sys.executable, "-c", code], cwd=tmp_path, env=env, capture_output=True, text=True, timeout=120)
+    assert r.returncode == 0, r.stderr
+
+
+def test_native_call_path_of_another_torch_is_not_used(lib, monkeypatch):
+    assert _lib.ext is not None and _lib.ext.torch_version == torch.__version__
+    monkeypatch.setattr(torch, "__version__", "0.0")
+    with pytest.warns(RuntimeWarning, match="built for torch"):
+        assert _lib._load_ext(lib) is None
+
+
+@pytest.mark.parametrize("missing", ["torch", "g++"])
+def test_build_needs_no_torch_for_the_library(missing, monkeypatch, tmp_path):
+    import build_lib
+    monkeypatch.setattr(build_lib, "EXT_LIB", tmp_path / "_int4_torch.so")
+    if missing == "torch":
+        monkeypatch.setitem(sys.modules, "torch", None)
+    else:
+        monkeypatch.setattr(build_lib.shutil, "which", lambda name: None)
+    assert build_lib.build_ext() is None and not list(tmp_path.iterdir())
