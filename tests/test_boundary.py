@@ -5,6 +5,7 @@ import ctypes
 import os
 import re
 import shutil
+import struct
 import subprocess
 import sys
 from pathlib import Path
@@ -472,3 +473,12 @@ def test_build_needs_no_torch_for_the_library(missing, monkeypatch, tmp_path):
     else:
         monkeypatch.setattr(build_lib.shutil, "which", lambda name: None)
     assert build_lib.build_ext() is None and not list(tmp_path.iterdir())
+
+
+def test_native_call_path_brings_no_thread_local_storage():
+    """A thread-local segment in it would slow every torch call of the process (see build_lib.py)."""
+    elf = (_lib.LIB_PATH.parent / "_int4_torch.so").read_bytes()
+    assert elf[:5] == b"\x7fELF\x02"  # 64-bit
+    off, = struct.unpack_from("<Q", elf, 32)
+    size, n = struct.unpack_from("<HH", elf, 54)
+    assert 7 not in [struct.unpack_from("<I", elf, off + i * size)[0] for i in range(n)]  # PT_TLS
