@@ -187,7 +187,7 @@ __global__ __launch_bounds__(kAttnThreads) void attn_decode_kernel(AttnDecodeArg
 
   for (int p0 = c0; p0 < c1; p0 += 64) {
     const int p = p0 + lane;
-    if (p0 + 64 > pos) {  // uniform: the block of the position (values past it: any finite one)
+    if (p0 + 64 > pos) {  // uniform: the block of the position
 #pragma unroll
       for (int i = 0; i < DW; i += 4) {
         const f32x4 kn = *reinterpret_cast<const f32x4*>(&k_s[wv * DW + i]);
@@ -196,9 +196,18 @@ __global__ __launch_bounds__(kAttnThreads) void attn_decode_kernel(AttnDecodeArg
       }
 #pragma unroll
       for (int e = 0; e < VE; ++e) {
+        // Rows past the position get its value too, whose weight is 0 there: one
+        // select a row.  An infinity or NaN must not meet those weights; it is put
+        // into its row alone (rare, uniform).
         const float vn = v_s[lane * VE + e];
+        const bool odd = !(__builtin_fabsf(vn) < __builtin_inff());
+        const float fill = odd ? 0.f : vn;
 #pragma unroll
-        for (int i = 0; i < PW; ++i) vr[i][e] = p0 + wv * PW + i >= pos ? vn : vr[i][e];
+        for (int i = 0; i < PW; ++i) vr[i][e] = p0 + wv * PW + i >= pos ? fill : vr[i][e];
+        if (__ballot(odd) != 0) {
+#pragma unroll
+          for (int i = 0; i < PW; ++i) vr[i][e] = p0 + wv * PW + i == pos ? vn : vr[i][e];
+        }
       }
     }
     float s[GP];
@@ -479,13 +488,13 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D == 64 ? 2
     }
   }
 
-  // the head's keys and values (below 2 GiB each, the host checks)
+  // the head's keys, and its values up to the prompt's end (below 2 GiB each, the host checks)
+  const int L = a.pos0 + a.T;
   const int64_t head = (int64_t)kvh * D * a.max_len;
   const __amdgpu_buffer_rsrc_t rk =
       __builtin_amdgcn_make_buffer_rsrc((void*)(a.kc + head), (short)0, D * a.max_len * 4, 0x00020000);
   const __amdgpu_buffer_rsrc_t rv =
-      __builtin_amdgcn_make_buffer_rsrc((void*)(a.vc + head), (short)0, D * a.max_len * 4, 0x00020000);
-  const int L = a.pos0 + a.T;
+      __builtin_amdgcn_make_buffer_rsrc((void*)(a.vc + head), (short)0, D * L * 4, 0x00020000);
   const int blocks = (min(a.pos0 + tb + (two_heads ? 15 : 31), L - 1) >> 6) + 1;
   float m[2], l[2];
   f32x4 o[2][NT];
@@ -520,13 +529,14 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D == 64 ? 2
     }
     __builtin_amdgcn_sched_barrier(0);
   };
-  // values of a block, r in {2 h, 2 h + 1}; rows past the prompt hold nothing yet:
-  // a valid row, whose weight is 0
+  // values of a block, r in {2 h, 2 h + 1}; rows past the prompt hold nothing yet and
+  // lie past the resource's range, which reads zeros (a row of the prompt in their
+  // place would add 0 x infinity where it holds one)
   f32x4 vv[2][8][VH];
   auto load_v = [&](int p0, int h) {
 #pragma unroll
     for (int x = 0; x < 8; ++x) {
-      const uint32_t vo = (uint32_t)(min(p0 + 16 * j + 8 * h + x, L - 1) * D + 4 * i) * 4u;
+      const uint32_t vo = (uint32_t)((p0 + 16 * j + 8 * h + x) * D + 4 * i) * 4u;
 #pragma unroll
       for (int hh = 0; hh < VH; ++hh)
         vv[h][x][hh] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rv, vo, 256u * (uint32_t)hh, 0));

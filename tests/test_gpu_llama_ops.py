@@ -159,6 +159,44 @@ def test_attention_decode_infinities_and_nan():
     assert torch.equal(got[3], torch.zeros(d, dtype=torch.bfloat16))
 
 
+@pytest.mark.parametrize("pos", [0, 5, 64, 99])
+@pytest.mark.parametrize("bad", [float("inf"), float("-inf"), float("nan")])
+def test_attention_decode_takes_an_infinite_new_value(bad, pos):
+    """An infinity in the value being written weighs what its position weighs, as in torch's
+    product, and nothing else of the block it shares with empty positions."""
+    nh, nkv, d, L = 4, 2, 64, 100
+    q, k, v = (randn((1, n * d), seed=i) for i, n in enumerate((nh, nkv, nkv)))
+    v[0, 3] = bad
+    kc, vc = randn((nkv, d, L), 5, dtype=torch.float32), randn((nkv, L, d), 6, dtype=torch.float32)
+    cos, sin = (t[pos:pos + 1].contiguous() for t in _tables(L, d))
+    args = [t.to(DEV) for t in (q, k, v, cos, sin, kc, vc)]
+    got = llama_ops.attention_decode(*args, torch.tensor([pos], device=DEV), nh, nkv, d).cpu()
+    kc[:, :, pos], vc[:, pos] = _rope(k.float().view(1, nkv, d), cos, sin)[0], v.float().view(nkv, d)
+    want = _attention(_rope(q.float().view(1, nh, d), cos, sin), kc, vc, pos)
+    assert torch.equal(got.isfinite(), want.isfinite()) and (~want.isfinite()).sum() == nh // nkv
+    torch.testing.assert_close(got[~want.isfinite()].double(), want[~want.isfinite()], equal_nan=True)
+    _check_out(got.nan_to_num(0, 0, 0), want.nan_to_num(0, 0, 0), torch.bfloat16)
+
+
+@pytest.mark.parametrize("T", [1, 33, 64, 100])
+@pytest.mark.parametrize("d", [64, 128])
+def test_attention_prefill_takes_an_infinite_last_value(T, d):
+    """The last token's row with an infinity in its own value; positions past the prompt in
+    its block do not see it."""
+    nh, nkv, L = 4, 2, 130
+    q, k, v = (randn((T, n * d), seed=i) for i, n in enumerate((nh, nkv, nkv)))
+    v[-1, 3] = float("inf")
+    kc, vc = torch.zeros((nkv, d, L)), torch.zeros((nkv, L, d))
+    cos, sin = (t[:T].contiguous() for t in _tables(L, d))
+    args = [t.to(DEV) for t in (q, k, v, cos, sin, kc, vc)]
+    got = llama_ops.attention_prefill(*args, 0, nh, nkv, d).cpu()[-1:]
+    kc[:, :, :T] = _rope(k.float().view(T, nkv, d), cos, sin).permute(1, 2, 0)
+    vc[:, :T] = v.float().view(T, nkv, d).transpose(0, 1)
+    want = _attention(_rope(q.float().view(T, nh, d), cos, sin), kc, vc, 0)[-1:]
+    assert torch.equal(got == math.inf, want == math.inf) and (want == math.inf).sum() == nh // nkv
+    _check_out(got.nan_to_num(7, 7, 7), want.nan_to_num(7, 7, 7), torch.bfloat16)
+
+
 # rows of one vector up to the widest (16384), widths that leave threads idle
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("rows,n", [(1, 8), (1, 2048), (3, 2056), (7, 4096), (2, 8200), (500, 512), (1, 16384)])
