@@ -654,6 +654,15 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D == 64 ? 2
 constexpr int kNormThreads = 256;
 constexpr int kNormMaxVecs = 8;  // 16-byte vectors per thread: rows of up to 16384
 
+// The same words, which the compiler takes for others if ON.  It computes what
+// follows a conditional load inside the condition and keeps values that two passes
+// unpack, so that all of a row's fp16 conversions live at once.
+template <bool ON>
+__device__ __forceinline__ u32x4 opaque(u32x4 v) {
+  if constexpr (ON) asm volatile("" : "+v"(v[0]), "+v"(v[1]), "+v"(v[2]), "+v"(v[3]));
+  return v;
+}
+
 // y = x / sqrt(mean(x^2) + eps) * weight, rows of n values, fp32 inside and one
 // rounding; with a delta the row is first x + delta, rounded to the dtype (the
 // residual stream) and written to sum.  One workgroup per row, the row held in
@@ -666,36 +675,44 @@ __global__ __launch_bounds__(kNormThreads) void rmsnorm_kernel(const uint16_t* _
                                                                const uint16_t* __restrict__ delta,
                                                                const uint16_t* __restrict__ weight, int n, float eps,
                                                                uint16_t* __restrict__ sum, uint16_t* __restrict__ y) {
+  // fp16 rows above 4096: 8 vectors with a delta took 502 registers and 772 bytes of
+  // scratch a lane, 111 registers so (2048 x 16384: 393 -> 43 us, without a delta 51 ->
+  // 23).  Narrower rows fit either way and are 2-3 % faster converted under the
+  // condition; bf16 unpacks by shifts, which the compiler repeats by itself.
+  constexpr bool OQ = DT == W4_DTYPE_FP16 && VPT >= 4;
   __shared__ float part[kNormThreads / 64];
-  const int tid = threadIdx.x, vecs = n / 8;
+  const uint32_t tid = threadIdx.x, vecs = (uint32_t)n / 8;
   const int64_t row = (int64_t)blockIdx.x * n;
+  x += row, y += row;
+  if constexpr (ADD) delta += row, sum += row;
   u32x4 xr[VPT], dr[VPT], wr[VPT];
 #pragma unroll
   for (int i = 0; i < VPT; ++i) {
-    const int v = tid + i * kNormThreads;
+    const uint32_t v = tid + i * kNormThreads;
     xr[i] = dr[i] = wr[i] = u32x4{0u, 0u, 0u, 0u};
     if (v < vecs) {
-      xr[i] = *reinterpret_cast<const u32x4*>(x + row + v * 8);
-      if constexpr (ADD) dr[i] = *reinterpret_cast<const u32x4*>(delta + row + v * 8);
+      xr[i] = *reinterpret_cast<const u32x4*>(x + v * 8);
+      if constexpr (ADD) dr[i] = *reinterpret_cast<const u32x4*>(delta + v * 8);
       wr[i] = *reinterpret_cast<const u32x4*>(weight + v * 8);
     }
   }
-  float xv[VPT][8], sq = 0.f;
+  float sq = 0.f;
 #pragma unroll
   for (int i = 0; i < VPT; ++i) {
-    unpack8<DT>(xr[i], xv[i]);
+    float xv[8];
+    unpack8<DT>(opaque<OQ>(xr[i]), xv);
     if constexpr (ADD) {
       float dv[8];
-      unpack8<DT>(dr[i], dv);
+      unpack8<DT>(opaque<OQ>(dr[i]), dv);
 #pragma unroll
-      for (int j = 0; j < 8; ++j) xv[i][j] += dv[j];
-      const u32x4 s = pack8<DT>(xv[i]);
-      const int v = tid + i * kNormThreads;
-      if (v < vecs) *reinterpret_cast<u32x4*>(sum + row + v * 8) = s;
-      unpack8<DT>(s, xv[i]);
+      for (int j = 0; j < 8; ++j) xv[j] += dv[j];
+      xr[i] = pack8<DT>(xv);
+      const uint32_t v = tid + i * kNormThreads;
+      if (v < vecs) *reinterpret_cast<u32x4*>(sum + v * 8) = xr[i];
+      unpack8<DT>(xr[i], xv);
     }
 #pragma unroll
-    for (int j = 0; j < 8; ++j) sq = __builtin_fmaf(xv[i][j], xv[i][j], sq);
+    for (int j = 0; j < 8; ++j) sq = __builtin_fmaf(xv[j], xv[j], sq);
   }
   sq = wave_sum(sq);
   if ((tid & 63) == 0) part[tid >> 6] = sq;
@@ -703,12 +720,13 @@ __global__ __launch_bounds__(kNormThreads) void rmsnorm_kernel(const uint16_t* _
   const float r = 1.0f / sqrtf(((part[0] + part[1]) + (part[2] + part[3])) / (float)n + eps);
 #pragma unroll
   for (int i = 0; i < VPT; ++i) {
-    const int v = tid + i * kNormThreads;
-    float wv[8], o[8];
-    unpack8<DT>(wr[i], wv);
+    const uint32_t v = tid + i * kNormThreads;
+    float xv[8], wv[8], o[8];
+    unpack8<DT>(opaque<OQ>(xr[i]), xv);
+    unpack8<DT>(opaque<OQ>(wr[i]), wv);
 #pragma unroll
-    for (int j = 0; j < 8; ++j) o[j] = xv[i][j] * r * wv[j];
-    if (v < vecs) *reinterpret_cast<u32x4*>(y + row + v * 8) = pack8<DT>(o);
+    for (int j = 0; j < 8; ++j) o[j] = xv[j] * r * wv[j];
+    if (v < vecs) *reinterpret_cast<u32x4*>(y + v * 8) = pack8<DT>(o);
   }
 }
 

@@ -482,3 +482,18 @@ def test_native_call_path_brings_no_thread_local_storage():
     off, = struct.unpack_from("<Q", elf, 32)
     size, n = struct.unpack_from("<HH", elf, 54)
     assert 7 not in [struct.unpack_from("<I", elf, off + i * size)[0] for i in range(n)]  # PT_TLS
+
+
+def test_kernels_of_the_decoder_layer_use_no_scratch():
+    """Rows and tiles that these kernels hold in registers are held in registers (the code
+    object's own metadata)."""
+    msgpack = pytest.importorskip("msgpack")
+    lib, at, seen = _lib.LIB_PATH.read_bytes(), 0, []
+    while (at := lib.find(b"AMDGPU\0\0", at)) >= 0:
+        namesz, size, kind = struct.unpack_from("<III", lib, at - 12)
+        at += 8
+        if (namesz, kind) == (7, 32):  # an NT_AMDGPU_METADATA note
+            seen += msgpack.unpackb(lib[at:at + size])["amdhsa.kernels"]
+    ours = [k for k in seen if re.search(r"attn_|rope_cache|rmsnorm|norm_head|silu_mul|dec_kernel_pro", k[".name"])]
+    assert len(ours) > 60
+    assert [k[".name"] for k in ours if k[".private_segment_fixed_size"]] == []
