@@ -757,6 +757,10 @@ template <int DT, int NC>
 __global__ __launch_bounds__(256) void norm_head_kernel(NormHeadArgs a) {
   // rows a wave takes at a time: twice as many measured 1-4 % slower (fewer waves fit)
   constexpr int R = head_rows(NC);
+  // fp16 rows above 2048: with every conversion of the norm's operands alive at once,
+  // rows above 3584 took 296 registers, one wave per SIMD (8000 x 4096: 24.0 us, now
+  // 14.2; 32000 x 4096 48.6, now 40.6; 128256 x 3072 117.5, now 117.3).
+  constexpr bool OQ = DT == W4_DTYPE_FP16 && NC >= 5;
   const int tid = threadIdx.x, lane = tid & 63;
   const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int waves = (int)gridDim.x * 4;
@@ -790,10 +794,10 @@ __global__ __launch_bounds__(256) void norm_head_kernel(NormHeadArgs a) {
   float x[NC][8], sq = 0.f;
 #pragma unroll
   for (int c = 0; c < NC; ++c) {
-    unpack8<DT>(xr[c], x[c]);
+    unpack8<DT>(opaque<OQ>(xr[c]), x[c]);
     if (a.delta) {
       float d[8];
-      unpack8<DT>(dr[c], d);
+      unpack8<DT>(opaque<OQ>(dr[c]), d);
 #pragma unroll
       for (int j = 0; j < 8; ++j) x[c][j] += d[j];
       unpack8<DT>(pack8<DT>(x[c]), x[c]);
@@ -809,7 +813,7 @@ __global__ __launch_bounds__(256) void norm_head_kernel(NormHeadArgs a) {
 #pragma unroll
   for (int c = 0; c < NC; ++c) {
     float g[8];
-    unpack8<DT>(nr[c], g);
+    unpack8<DT>(opaque<OQ>(nr[c]), g);
 #pragma unroll
     for (int j = 0; j < 8; ++j) x[c][j] = x[c][j] * rms * g[j];
     unpack8<DT>(pack8<DT>(x[c]), x[c]);

@@ -484,9 +484,9 @@ def test_native_call_path_brings_no_thread_local_storage():
     assert 7 not in [struct.unpack_from("<I", elf, off + i * size)[0] for i in range(n)]  # PT_TLS
 
 
-def test_kernels_of_the_decoder_layer_use_no_scratch():
-    """Rows and tiles that these kernels hold in registers are held in registers (the code
-    object's own metadata)."""
+@pytest.fixture(scope="module")
+def kernels():
+    """The code objects' own metadata of every kernel of the library."""
     msgpack = pytest.importorskip("msgpack")
     lib, at, seen = _lib.LIB_PATH.read_bytes(), 0, []
     while (at := lib.find(b"AMDGPU\0\0", at)) >= 0:
@@ -494,6 +494,17 @@ def test_kernels_of_the_decoder_layer_use_no_scratch():
         at += 8
         if (namesz, kind) == (7, 32):  # an NT_AMDGPU_METADATA note
             seen += msgpack.unpackb(lib[at:at + size])["amdhsa.kernels"]
-    ours = [k for k in seen if re.search(r"attn_|rope_cache|rmsnorm|norm_head|silu_mul|dec_kernel_pro", k[".name"])]
+    return seen
+
+
+def test_kernels_of_the_decoder_layer_use_no_scratch(kernels):
+    """Rows and tiles that these kernels hold in registers are held in registers."""
+    ours = [k for k in kernels if re.search(r"attn_|rope_cache|rmsnorm|norm_head|silu_mul|dec_kernel_pro", k[".name"])]
     assert len(ours) > 60
     assert [k[".name"] for k in ours if k[".private_segment_fixed_size"]] == []
+
+
+def test_head_kernels_run_two_waves_per_simd(kernels):
+    """At most 256 of a lane's 512 registers, at every width and dtype."""
+    heads = [k for k in kernels if "norm_head" in k[".name"]]
+    assert len(heads) == 16 and [k[".name"] for k in heads if k[".vgpr_count"] > 256] == []
