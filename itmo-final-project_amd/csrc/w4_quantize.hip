@@ -338,7 +338,9 @@ __device__ __forceinline__ void quantize_small_group_tiles(const QuantArgs& qa, 
         // a word near a rounding boundary, or a group whose statistics are:
         // infinite, NaN or underflowing scale, zero point near one
         if (near || bad) {
-          if constexpr (!GIVEN) st = group_stats(mx, mn);
+          if constexpr (!GIVEN) {
+            if (bad) st = group_stats(mx, mn);  // (a chain of divisions that a near word need not wait for)
+          }
           word = quantize_pack8(v, st);
         }
         tile[ts][seg][row] = word;
