@@ -253,8 +253,15 @@ __device__ __forceinline__ void quantize_small_group_tiles(const QuantArgs& qa, 
   const int t = blk * TPB + ts;
   const bool active = t < (int)tiles_total;
   const int groups = (int)((uint32_t)K / (uint32_t)G);
-  const int tn = active ? t / groups : 0;
-  const int g = active ? t - tn * groups : 0;
+  // Tiles in order along K, so that the workgroups running at one time read whole
+  // rows.  Groups of 8 and 16 write as many bytes of scales and zero points as of
+  // codes, 128 at a time, and from 2^24 weights on are faster along N, where those
+  // meet in lines (8192 x 8192: 84.9 against 89.4 us at 8, 58.3 against 64.4 at 16;
+  // 4096 x 2048: 11.8 against 11.5 and 9.4 against 9.0; G = 32, 8192 x 8192: 53.3
+  // against 48.1).
+  const bool along_n = G <= 16 && !GIVEN && N * K >= (int64_t)1 << 24;
+  const int tn = !active ? 0 : along_n ? t % (int)tiles_n : t / groups;
+  const int g = !active ? 0 : along_n ? t / (int)tiles_n : t - tn * groups;
   const int64_t n0 = (int64_t)tn * QROWS;
   const int seg = lane % L;
   const int rsub = lane / L;

@@ -286,3 +286,17 @@ def test_dequantize_tile_edges(N, K, g, dt):
     ref = int4_hip.dequantize_int4_ref(*(torch.from_numpy(a) for a in (qw, s, z)), tdt)
     view = torch.int32 if dt == "fp32" else torch.int16
     assert torch.equal(out.view(view), ref.view(view))
+
+
+# tiles in order along N (groups of 8 and 16, 2^24 weights and more) and, just below,
+# along K; a ragged last tile, zero, NaN and infinite groups in both
+@pytest.mark.parametrize("N,K", [(8200, 2048), (8130, 2048)])
+@pytest.mark.parametrize("g", [8, 16, 32])
+def test_quantize_tile_orders(N, K, g):
+    w = randn((N, K), seed=N + g, sigma=0.02).to(DEV)
+    w[3], w[N - 1, :64], w[70, 5], w[71, K - 1] = 0, 0, float("nan"), float("inf")
+    want = int4_hip.quantize_int4_ref(w.cpu(), g)
+    for got in (int4_hip.quantize_int4(w, g), int4_hip.quantize_int4_grouped([w, w[:40]], g)[0]):
+        assert torch.equal(got[0].cpu(), want[0])
+        for a, b in zip(got[1:], want[1:]):
+            assert torch.equal(a.cpu().nan_to_num(-7.0), b.nan_to_num(-7.0))
