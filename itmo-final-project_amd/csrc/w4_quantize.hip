@@ -501,7 +501,15 @@ __global__ __launch_bounds__(QSWAVES * 64) void quantize_pack_kernel(QuantGroupe
 // what a large copy reaches).  16-bit rows are stored non-temporal (9.7 us
 // cached); fp32 lanes store two 16-byte halves 32 bytes apart, where partial
 // lines made that slower (26 against 16.5 us).
-template <int ODT>
+//
+// NT: the codes are loaded non-temporal, for fp32 output of whole 128-byte lines
+// (N % 32 == 0).  Its writes are eight times the codes and fill the Infinity
+// Cache, which the codes then leave to them (inputs not in the cache: 8192 x 2048
+// 16.0 against 17.2 us, 12032 x 4096 46.1 against 48.4).  16-bit output leaves
+// room for them (8192 x 4096: 15.1 us, non-temporal 17.4; again on the same input
+// 14.7 against 17.9), and lines that two tiles share are fetched twice without the
+// cache (12001 x 4096: 22.6 against 27.4, fp32 48.3 against 49.2).
+template <int ODT, bool NT>
 __global__ __launch_bounds__(512) void dequantize_kernel(const int32_t* __restrict__ qw,
                                                          const uint16_t* __restrict__ sc,
                                                          const uint16_t* __restrict__ ze,
@@ -520,7 +528,9 @@ __global__ __launch_bounds__(512) void dequantize_kernel(const int32_t* __restri
 #pragma unroll
   for (int i = 0; i < 8; ++i) {
     const int kk = i * 8 + wv;
-    w[i] = (kk < rows && n < N) ? (uint32_t)__builtin_nontemporal_load(&qw[(k80 + kk) * N + n]) : 0u;
+    const int32_t* at = &qw[(k80 + kk) * N + n];
+    w[i] = 0u;
+    if (kk < rows && n < N) w[i] = (uint32_t)(NT ? __builtin_nontemporal_load(at) : *at);
   }
   // groups first .. first + groups - 1 (a group size below 512 divides the tile's 512 k)
   const int64_t first = (k80 * 8) >> gshift;
@@ -761,15 +771,19 @@ extern "C" int w4_dequantize(const int32_t* qweight, const uint16_t* scales, con
   const dim3 grid((unsigned)((N + 63) / 64), (unsigned)((K8 + 63) / 64));
   const int gshift = ilog2(G);
   hipStream_t st = static_cast<hipStream_t>(stream);
+  const auto launch = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, grid, dim3(512), 0, st, qweight, scales, zeros, N, K8, gshift, out);
+  };
   switch (out_dtype) {
     case W4_DTYPE_BF16:
-      hipLaunchKernelGGL((w4::dequantize_kernel<W4_DTYPE_BF16>), grid, dim3(512), 0, st, qweight, scales, zeros, N, K8, gshift, out);
+      launch(w4::dequantize_kernel<W4_DTYPE_BF16, false>);
       break;
     case W4_DTYPE_FP16:
-      hipLaunchKernelGGL((w4::dequantize_kernel<W4_DTYPE_FP16>), grid, dim3(512), 0, st, qweight, scales, zeros, N, K8, gshift, out);
+      launch(w4::dequantize_kernel<W4_DTYPE_FP16, false>);
       break;
     case W4_DTYPE_FP32:
-      hipLaunchKernelGGL((w4::dequantize_kernel<W4_DTYPE_FP32>), grid, dim3(512), 0, st, qweight, scales, zeros, N, K8, gshift, out);
+      if (N % 32 == 0) launch(w4::dequantize_kernel<W4_DTYPE_FP32, true>);
+      else launch(w4::dequantize_kernel<W4_DTYPE_FP32, false>);
       break;
     default:
       return fail(W4_ERR_INVALID, "w4_dequantize: bad out dtype %d", out_dtype);
