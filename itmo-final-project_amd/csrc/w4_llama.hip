@@ -141,13 +141,11 @@ __global__ __launch_bounds__(kAttnThreads) void attn_decode_kernel(AttnDecodeArg
   load_v(c0);
   __builtin_amdgcn_sched_barrier(0);
 
-  if (pos64 < 0 || pos64 >= a.max_len) {  // no such place in the cache: a defined output, nothing else
-    if (c == 0)
-      for (int i = tid; i < g * D; i += kAttnThreads)
-        a.out[(int64_t)h0 * D + i] = float_to_act_bits<DT>(__builtin_nanf(""));
-    return;
-  }
-  const int pos = (int)pos64;
+  // A position the cache does not hold: nothing is written to it, and a NaN query gives
+  // a NaN output (at position 0; a branch of its own cost 0.1 us at D = 128).
+  const bool in_cache = (uint64_t)pos64 < (uint64_t)a.max_len;
+  const int pos = in_cache ? (int)pos64 : 0;
+  const float qscale = in_cache ? a.qscale : __builtin_nanf("");
   const int active = pos / a.chunk + 1;
   if (c >= active) return;
   const int c1 = min(c0 + a.chunk, pos + 1);
@@ -155,8 +153,8 @@ __global__ __launch_bounds__(kAttnThreads) void attn_decode_kernel(AttnDecodeArg
   if (tid < GP * (D / 2)) {
     float r1, r2;
     rope_pair(act_bits_to_float(q1, DT), act_bits_to_float(q2, DT), rc, rs, &r1, &r2);
-    q_s[qh][qd] = qh < g ? r1 * a.qscale : 0.f;
-    q_s[qh][qd + D / 2] = qh < g ? r2 * a.qscale : 0.f;
+    q_s[qh][qd] = qh < g ? r1 * qscale : 0.f;
+    q_s[qh][qd + D / 2] = qh < g ? r2 * qscale : 0.f;
   }
   if (c == active - 1) {
     if (tid < D / 2) {
@@ -164,14 +162,14 @@ __global__ __launch_bounds__(kAttnThreads) void attn_decode_kernel(AttnDecodeArg
       rope_pair(act_bits_to_float(k1, DT), act_bits_to_float(k2, DT), rc, rs, &r1, &r2);
       k_s[tid] = r1;
       k_s[tid + D / 2] = r2;
-      if (z == 0) {
+      if (z == 0 && in_cache) {
         a.kc[((int64_t)kvh * D + tid) * a.max_len + pos] = r1;
         a.kc[((int64_t)kvh * D + tid + D / 2) * a.max_len + pos] = r2;
       }
     } else if (tid >= 128 && tid < 128 + D) {
       const float v = act_bits_to_float(v1, DT);
       v_s[tid - 128] = v;
-      if (z == 0) a.vc[((int64_t)kvh * a.max_len + pos) * D + tid - 128] = v;
+      if (z == 0 && in_cache) a.vc[((int64_t)kvh * a.max_len + pos) * D + tid - 128] = v;
     }
   }
   __syncthreads();
@@ -194,20 +192,25 @@ __global__ __launch_bounds__(kAttnThreads) void attn_decode_kernel(AttnDecodeArg
 #pragma unroll
         for (int e = 0; e < 4; ++e) kr[i + e] = p == pos ? kn[e] : kr[i + e];
       }
+      // Rows past the position get its value too, whose weight is 0 there: one select
+      // a row.  An infinity or NaN must not meet those weights; it is put into its row
+      // alone (rare, uniform).
+      float vn[VE];
+      bool odd = false;
 #pragma unroll
       for (int e = 0; e < VE; ++e) {
-        // Rows past the position get its value too, whose weight is 0 there: one
-        // select a row.  An infinity or NaN must not meet those weights; it is put
-        // into its row alone (rare, uniform).
-        const float vn = v_s[lane * VE + e];
-        const bool odd = !(__builtin_fabsf(vn) < __builtin_inff());
-        const float fill = odd ? 0.f : vn;
+        vn[e] = v_s[lane * VE + e];
+        const bool finite = __builtin_fabsf(vn[e]) < __builtin_inff();
+        const float fill = finite ? vn[e] : 0.f;
+        odd = odd || !finite;
 #pragma unroll
         for (int i = 0; i < PW; ++i) vr[i][e] = p0 + wv * PW + i >= pos ? fill : vr[i][e];
-        if (__ballot(odd) != 0) {
+      }
+      if (__builtin_expect(__ballot(odd) != 0, 0)) {
 #pragma unroll
-          for (int i = 0; i < PW; ++i) vr[i][e] = p0 + wv * PW + i == pos ? vn : vr[i][e];
-        }
+        for (int i = 0; i < PW; ++i)
+#pragma unroll
+          for (int e = 0; e < VE; ++e) vr[i][e] = p0 + wv * PW + i == pos ? vn[e] : vr[i][e];
       }
     }
     float s[GP];
