@@ -65,7 +65,7 @@ class RMSNorm(nn.Module):
     def forward(self, x: torch.Tensor) -> torch.Tensor:
         # one fused kernel; fp32 statistics (the weight is applied before the
         # final rounding, where the Hugging Face layer rounds first)
-        if self.eps is not None and llama_ops.rms_norm_ok(x, self.weight):
+        if llama_ops.rms_norm_ok(x, self.weight) and self.eps is not None:
             return llama_ops.rms_norm(x, self.weight, self.eps)
         return F.rms_norm(x, (x.shape[-1],), self.weight, self.eps)
 
@@ -87,7 +87,7 @@ def _plain_norm(module: nn.Module) -> bool:
 def _add_norm(x: torch.Tensor, delta: torch.Tensor, norm: nn.Module) -> tuple:
     """(x + delta, norm(x + delta)), in one launch where ``norm`` is a plain RMSNorm
     that nothing hooks into."""
-    if _plain_norm(norm) and llama_ops.rms_norm_ok(x, norm.weight, delta):
+    if x.dtype in llama_ops.DTYPES and _plain_norm(norm) and llama_ops.rms_norm_ok(x, norm.weight, delta):
         return llama_ops.rms_norm(x, norm.weight, norm.eps, delta)
     x = x + delta
     return x, norm(x)

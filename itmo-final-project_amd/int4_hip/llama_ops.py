@@ -17,7 +17,8 @@ from torch.compiler import is_compiling as _is_compiling
 from . import _lib
 from .gemm import _check_weight, _with_workspace
 
-_XDT = {torch.bfloat16: _lib.DTYPE_BF16, torch.float16: _lib.DTYPE_FP16}
+# dtypes of the activations the kernels take, with their codes
+DTYPES = {torch.bfloat16: _lib.DTYPE_BF16, torch.float16: _lib.DTYPE_FP16}
 _PLAIN = (torch.Tensor, nn.Parameter)
 
 
@@ -76,9 +77,11 @@ def attention_decode_ok(x, kc, vc, cos, sin, pos, nh: int, nkv: int, d: int, qkv
     """Whether ``attention_decode`` takes a step with activations like ``x``
     ([1, hidden]), the caches ``kc`` [.., nkv, d, L], ``vc`` [.., nkv, L, d] and, where
     they are known, the projections ``qkv``."""
+    if x.dtype not in DTYPES:  # (first: models of other types pay for no more)
+        return False
     L = kc.shape[-1]
     return (kc.shape[-3:] == (nkv, d, L) and vc.shape == (*kc.shape[:-3], nkv, L, d)
-            and x.shape[0] == 1 and x.dtype in _XDT
+            and x.shape[0] == 1
             and kc.dtype == vc.dtype == cos.dtype == sin.dtype == torch.float32 and pos.dtype == torch.int64
             and pos.numel() == 1 and cos.shape == sin.shape == (1, d // 2)
             and kc.is_contiguous() and vc.is_contiguous() and cos.is_contiguous() and sin.is_contiguous()
@@ -96,7 +99,7 @@ def attention_decode(q, k, v, cos, sin, kc, vc, pos, nh: int, nkv: int, d: int) 
     out = torch.empty((1, nh * d), dtype=q.dtype, device=dev)
     lib = _lib.load()
     rc = _on(dev, lambda st: _with_workspace(dev, st, _attn_ws_bytes(nh, nkv, d, max_len), lambda ws, nb:
-             lib.w4_attention_decode(q.data_ptr(), k.data_ptr(), v.data_ptr(), _XDT[q.dtype], nh, nkv, d,
+             lib.w4_attention_decode(q.data_ptr(), k.data_ptr(), v.data_ptr(), DTYPES[q.dtype], nh, nkv, d,
                                      cos.data_ptr(), sin.data_ptr(), kc.data_ptr(), vc.data_ptr(), max_len,
                                      pos.data_ptr(), out.data_ptr(), ws, nb, st)))
     if rc:
@@ -107,10 +110,12 @@ def attention_decode(q, k, v, cos, sin, kc, vc, pos, nh: int, nkv: int, d: int) 
 def attention_prefill_ok(x, kc, vc, cos, sin, pos0, nh: int, nkv: int, d: int, qkv=()) -> bool:
     """Whether ``attention_prefill`` takes the tokens of ``x`` [T, hidden] at positions
     pos0.. of the caches ``kc`` [nkv, d, L], ``vc`` [nkv, L, d], and their projections ``qkv``."""
+    if x.dtype not in DTYPES:
+        return False
     T, L = x.shape[0], kc.shape[-1]
     return (x.dim() == 2 and T >= 1 and d in (64, 128) and nh % nkv == 0 and type(pos0) is int
             and 0 <= pos0 <= L - T and L < 1 << 22 and T <= 65535 * 16 and nkv <= 65535
-            and x.dtype in _XDT and kc.dtype == vc.dtype == cos.dtype == sin.dtype == torch.float32
+            and kc.dtype == vc.dtype == cos.dtype == sin.dtype == torch.float32
             and kc.shape == (nkv, d, L) and vc.shape == (nkv, L, d) and cos.shape == sin.shape == (T, d // 2)
             and kc.is_contiguous() and cos.is_contiguous() and sin.is_contiguous()
             and (not qkv or _qkv_fit(x, qkv, nh, nkv, d)) and fusable(x, kc, vc, cos, sin, *qkv) and _dense(vc))
@@ -125,7 +130,7 @@ def attention_prefill(q, k, v, cos, sin, kc, vc, pos0: int, nh: int, nkv: int, d
     out = torch.empty_like(q)
     lib = _lib.load()
     rc = _on(dev, lambda st: lib.w4_attention_prefill(
-        q.data_ptr(), k.data_ptr(), v.data_ptr(), _XDT[q.dtype], T, nh, nkv, d, cos.data_ptr(), sin.data_ptr(),
+        q.data_ptr(), k.data_ptr(), v.data_ptr(), DTYPES[q.dtype], T, nh, nkv, d, cos.data_ptr(), sin.data_ptr(),
         kc.data_ptr(), vc.data_ptr(), kc.shape[-1], pos0, out.data_ptr(), st))
     if rc:
         _lib.check(rc, "w4_attention_prefill")
@@ -138,9 +143,11 @@ MAX_GRID = (2**32 - 1) // 256   # workgroups of 256 threads in a launch: a row, 
 
 def rms_norm_ok(x, weight, delta=None) -> bool:
     """Whether ``rms_norm`` takes ``x`` [..., n] (and a residual ``delta`` like it)."""
+    if x.dtype not in DTYPES:
+        return False
     n = x.shape[-1] if x.dim() else 0
     ts = (x, weight) if delta is None else (x, weight, delta)
-    return (x.dtype in _XDT and 0 < n <= MAX_NORM and n % 8 == 0 and weight.shape == (n,)
+    return (0 < n <= MAX_NORM and n % 8 == 0 and weight.shape == (n,)
             and x.numel() <= MAX_GRID * n
             and all(t.dtype == x.dtype for t in ts) and (delta is None or delta.shape == x.shape)
             and fusable(*ts) and _dense(*ts))
@@ -153,15 +160,15 @@ def rms_norm(x, weight, eps: float, delta=None):
     s = None if delta is None else torch.empty_like(x)
     lib = _lib.load()
     rc = _on(x.device, lambda st: lib.w4_rmsnorm(
-        x.data_ptr(), None if delta is None else delta.data_ptr(), weight.data_ptr(), _XDT[x.dtype], x.numel() // n, n,
-        eps, None if s is None else s.data_ptr(), y.data_ptr(), st))
+        x.data_ptr(), None if delta is None else delta.data_ptr(), weight.data_ptr(), DTYPES[x.dtype], x.numel() // n,
+        n, eps, None if s is None else s.data_ptr(), y.data_ptr(), st))
     if rc:
         _lib.check(rc, "w4_rmsnorm")
     return y if delta is None else (s, y)
 
 
 def silu_mul_ok(gate, up) -> bool:
-    return (gate.dtype in _XDT and up.dtype == gate.dtype and up.shape == gate.shape and gate.numel() % 8 == 0
+    return (gate.dtype in DTYPES and up.dtype == gate.dtype and up.shape == gate.shape and gate.numel() % 8 == 0
             and gate.numel() <= MAX_GRID * 2048 and fusable(gate, up) and _dense(gate, up))
 
 
@@ -169,7 +176,7 @@ def silu_mul(gate, up) -> torch.Tensor:
     """silu(gate) * up in one pass, one rounding."""
     y = torch.empty_like(gate)
     lib = _lib.load()
-    rc = _on(gate.device, lambda st: lib.w4_silu_mul(gate.data_ptr(), up.data_ptr(), _XDT[gate.dtype], gate.numel(),
+    rc = _on(gate.device, lambda st: lib.w4_silu_mul(gate.data_ptr(), up.data_ptr(), DTYPES[gate.dtype], gate.numel(),
                                                      y.data_ptr(), st))
     if rc:
         _lib.check(rc, "w4_silu_mul")
@@ -207,7 +214,7 @@ def norm_linears(x, delta, weight, eps: float, weights):
     lib, dev = _lib.load(), x.device
     nbytes = lib.w4a16_grouped_workspace_bytes(probs, len(weights), 1)
     rc = _on(dev, lambda st: _with_workspace(dev, st, nbytes, lambda ws, nb: lib.w4a16_decode_norm(
-        probs, len(weights), _XDT[x.dtype], None if delta is None else delta.data_ptr(), weight.data_ptr(), eps,
+        probs, len(weights), DTYPES[x.dtype], None if delta is None else delta.data_ptr(), weight.data_ptr(), eps,
         None if delta is None else total.data_ptr(), ws, nb, st)))
     if rc == _lib.ERR_UNSUPPORTED:
         return None
@@ -227,7 +234,7 @@ def silu_linear(gate, up, weight):
     lib, dev = _lib.load(), gate.device
     nbytes = lib.w4a16_grouped_workspace_bytes(probs, 1, 1)
     rc = _on(dev, lambda st: _with_workspace(dev, st, nbytes, lambda ws, nb: lib.w4a16_decode_silu(
-        probs, _XDT[gate.dtype], up.data_ptr(), ws, nb, st)))
+        probs, DTYPES[gate.dtype], up.data_ptr(), ws, nb, st)))
     if rc == _lib.ERR_UNSUPPORTED:
         return None
     if rc:
@@ -247,7 +254,7 @@ def norm_head(x, delta, weight, eps: float, head):
     lib = _lib.load()
     rc = _on(x.device, lambda st: lib.w4_norm_head(
         x.data_ptr(), None if delta is None else delta.data_ptr(), weight.data_ptr(), eps, head.data_ptr(),
-        _XDT[x.dtype], N, K, y.data_ptr(), st))
+        DTYPES[x.dtype], N, K, y.data_ptr(), st))
     if rc:
         _lib.check(rc, "w4_norm_head")
     return y
