@@ -47,6 +47,30 @@ __device__ __forceinline__ uint16_t float_to_act_bits(float v) {
   return __builtin_bit_cast(uint16_t, (S)v);
 }
 
+// Eight consecutive 16-bit values as floats, and back.
+template <int DT>
+__device__ __forceinline__ void unpack8(const u32x4 r, float v[8]) {
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    v[2 * j] = act_bits_to_float((uint16_t)(r[j] & 0xFFFFu), DT);
+    v[2 * j + 1] = act_bits_to_float((uint16_t)(r[j] >> 16), DT);
+  }
+}
+template <int DT>
+__device__ __forceinline__ u32x4 pack8(const float v[8]) {
+  u32x4 r;
+#pragma unroll
+  for (int j = 0; j < 4; ++j)
+    r[j] = (uint32_t)float_to_act_bits<DT>(v[2 * j]) | ((uint32_t)float_to_act_bits<DT>(v[2 * j + 1]) << 16);
+  return r;
+}
+
+// The value of another lane of the row of 16, chosen by a DPP control word.
+template <int CTRL>
+__device__ __forceinline__ uint32_t dpp_mov(uint32_t v) {
+  return (uint32_t)__builtin_amdgcn_mov_dpp((int)v, CTRL, 0xF, 0xF, true);
+}
+
 // Per (group, column) constants of the exact dequantization.
 //
 // A nibble q is placed in the mantissa of an fp16 whose exponent is fixed:

@@ -204,29 +204,6 @@ __device__ __forceinline__ u32x4 dec_perm_x(u32x4 v) {
   return r;
 }
 
-// Eight consecutive 16-bit values as floats, and back.
-template <int DT>
-__device__ __forceinline__ void dec_unpack8(const u32x4 r, float v[8]) {
-#pragma unroll
-  for (int j = 0; j < 4; ++j) {
-    v[2 * j] = act_bits_to_float((uint16_t)(r[j] & 0xFFFFu), DT);
-    v[2 * j + 1] = act_bits_to_float((uint16_t)(r[j] >> 16), DT);
-  }
-}
-template <int DT>
-__device__ __forceinline__ u32x4 dec_pack8(const float v[8]) {
-  u32x4 r;
-#pragma unroll
-  for (int j = 0; j < 4; ++j)
-    r[j] = (uint32_t)float_to_act_bits<DT>(v[2 * j]) | ((uint32_t)float_to_act_bits<DT>(v[2 * j + 1]) << 16);
-  return r;
-}
-
-template <int CTRL>
-__device__ __forceinline__ uint32_t dec_dpp(uint32_t v) {
-  return (uint32_t)__builtin_amdgcn_mov_dpp((int)v, CTRL, 0xF, 0xF, true);
-}
-
 template <int VEC>
 struct DecW;
 template <>
@@ -793,23 +770,23 @@ __device__ __forceinline__ void dec_tile_one(const DecArgs& a, int tile, uint8_t
   float unscale = 1.0f;
   auto pro_apply = [&](const u32x4 xv, const u32x4 av, const u32x4 pw) {
     float x[8], b[8];
-    dec_unpack8<DT>(xv, x);
-    dec_unpack8<DT>(av, b);
+    unpack8<DT>(xv, x);
+    unpack8<DT>(av, b);
     if constexpr (PRO == kProNorm) {
 #pragma unroll
       for (int j = 0; j < 8; ++j) x[j] += b[j];
-      dec_unpack8<DT>(dec_pack8<DT>(x), x);
-      dec_unpack8<DT>(pw, b);
+      unpack8<DT>(pack8<DT>(x), x);
+      unpack8<DT>(pw, b);
 #pragma unroll
       for (int j = 0; j < 8; ++j) x[j] *= b[j];
       if constexpr (DT == W4_DTYPE_FP16) {
         uint32_t top = 0;
 #pragma unroll
         for (int j = 0; j < 8; ++j) top = max(top, __builtin_bit_cast(uint32_t, x[j]) & 0x7FFFFFFFu);
-        top = max(top, dec_dpp<0xB1>(top));
-        top = max(top, dec_dpp<0x4E>(top));
-        top = max(top, dec_dpp<0x141>(top));
-        top = max(top, dec_dpp<0x140>(top));
+        top = max(top, dpp_mov<0xB1>(top));
+        top = max(top, dpp_mov<0x4E>(top));
+        top = max(top, dpp_mov<0x141>(top));
+        top = max(top, dpp_mov<0x140>(top));
         const uint32_t all = max(max(__builtin_amdgcn_readlane(top, 0), __builtin_amdgcn_readlane(top, 16)),
                                  max(__builtin_amdgcn_readlane(top, 32), __builtin_amdgcn_readlane(top, 48)));
         const uint32_t e = min(max(all >> 23, 20u), 240u);  // a zero, infinite or NaN slice: any scale
@@ -822,7 +799,7 @@ __device__ __forceinline__ void dec_tile_one(const DecArgs& a, int tile, uint8_t
 #pragma unroll
       for (int j = 0; j < 8; ++j) x[j] = x[j] / (1.0f + __expf(-x[j])) * b[j];
     }
-    return dec_pack8<DT>(x);
+    return pack8<DT>(x);
   };
 
   // stage the round's activations (permuted), scales and zeros
@@ -1089,12 +1066,12 @@ __device__ __forceinline__ void dec_tile_one(const DecArgs& a, int tile, uint8_t
       float sq = 0.f;
       if (sums) {
         float v[8], d[8];
-        dec_unpack8<DT>(sx, v);
-        dec_unpack8<DT>(sa, d);
+        unpack8<DT>(sx, v);
+        unpack8<DT>(sa, d);
 #pragma unroll
         for (int j = 0; j < 8; ++j) v[j] += d[j];
-        const u32x4 sum = dec_pack8<DT>(v);
-        dec_unpack8<DT>(sum, v);
+        const u32x4 sum = pack8<DT>(v);
+        unpack8<DT>(sum, v);
 #pragma unroll
         for (int j = 0; j < 8; ++j) sq = __builtin_fmaf(v[j], v[j], sq);
 #pragma unroll
@@ -1342,9 +1319,10 @@ int sixteen_ksplit(int64_t K, int G, int deeper, int64_t part) {
 // as a whole past the end of its run, so a round that crossed into the next
 // part would add that part's first steps a second time.
 // Each narrowing level (a launch with few workgroups: a lone linear) halves
-// the parts again while they stay whole rounds and groups, so a lone down_proj
-// runs 256 workgroups of 32 KB instead of 64 of 128 KB.
-// The pairing words ((ks - 1) per column) live in the workspace's counter area.
+// the parts again while they stay whole rounds and groups and the pairing words
+// ((ks - 1) of 8 bytes per column) fit the workspace's counter area: a lone
+// down_proj runs 128 workgroups of 64 KB (four parts: 49152 bytes) instead of 64
+// of 128 KB (5.7 against 6.6 us); eight parts would need 114688.
 int one_ksplit(int64_t K, int G, int level, int64_t N) {
   if (K <= 4096 || G > 4096) return 1;
   int ks = 2;

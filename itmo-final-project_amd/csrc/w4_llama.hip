@@ -46,7 +46,7 @@ __device__ __forceinline__ void rope_pair(float x1, float x2, float c, float s, 
 // shuffle through LDS per step is ten times the latency).
 template <int CTRL>
 __device__ __forceinline__ float lane_perm(float v) {
-  return __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, v), CTRL, 0xF, 0xF, true));
+  return __builtin_bit_cast(float, dpp_mov<CTRL>(__builtin_bit_cast(uint32_t, v)));
 }
 __device__ __forceinline__ float lane_read(float v, int lane) {
   return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), lane));
@@ -349,24 +349,6 @@ __global__ __launch_bounds__(kAttnThreads) void attn_decode_kernel(AttnDecodeArg
     }
     a.out[(int64_t)h0 * D + i] = float_to_act_bits<DT>(t / l_s[h]);
   }
-}
-
-// Eight consecutive 16-bit values as floats, and back.
-template <int DT>
-__device__ __forceinline__ void unpack8(const u32x4 r, float v[8]) {
-#pragma unroll
-  for (int j = 0; j < 4; ++j) {
-    v[2 * j] = act_bits_to_float((uint16_t)(r[j] & 0xFFFFu), DT);
-    v[2 * j + 1] = act_bits_to_float((uint16_t)(r[j] >> 16), DT);
-  }
-}
-template <int DT>
-__device__ __forceinline__ u32x4 pack8(const float v[8]) {
-  u32x4 r;
-#pragma unroll
-  for (int j = 0; j < 4; ++j)
-    r[j] = (uint32_t)float_to_act_bits<DT>(v[2 * j]) | ((uint32_t)float_to_act_bits<DT>(v[2 * j + 1]) << 16);
-  return r;
 }
 
 // ---------------------------------------------------------------- prompt

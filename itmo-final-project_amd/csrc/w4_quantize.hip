@@ -25,11 +25,6 @@ __device__ __forceinline__ float clamp_nan(float x, float lo, float hi) {
 __device__ __forceinline__ float fmax_p(float a, float b) { return __builtin_elementwise_maximum(a, b); }
 __device__ __forceinline__ float fmin_p(float a, float b) { return __builtin_elementwise_minimum(a, b); }
 
-template <int CTRL>
-__device__ __forceinline__ float dpp_mov(float v) {
-  return __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, v), CTRL, 0xF, 0xF, true));
-}
-
 // One DPP step of a maximum and a minimum (values without NaN).  Written in
 // assembly: the compiler puts a quieting v_max_f32 x, x before each, and the
 // NaN-propagating forms have no DPP encoding, so a step took four or six
@@ -171,16 +166,6 @@ __device__ __forceinline__ uint32_t quantize_pack8_fast(const float v[8], QStats
   return word;
 }
 
-// The eight activation-dtype weights of one 16-byte row segment, as floats.
-template <int DT>
-__device__ __forceinline__ void unpack_row8(const u32x4 r, float v[8]) {
-#pragma unroll
-  for (int j = 0; j < 4; ++j) {
-    v[2 * j] = act_bits_to_float((uint16_t)(r[j] & 0xFFFFu), DT);
-    v[2 * j + 1] = act_bits_to_float((uint16_t)(r[j] >> 16), DT);
-  }
-}
-
 // Stored fp16 patterns.  A NaN zero point is written as 0xFE00, the x86
 // "default NaN" that the reference's CPU path produces for -0/0 and for
 // negated NaN inputs; a NaN scale (NaN weights) as 0x7E00.
@@ -314,7 +299,7 @@ __device__ __forceinline__ void quantize_small_group_tiles(const QuantArgs& qa, 
       for (int i = 0; i < B; ++i) {
         const int row = sub * RW + (b0 + i) * RPI + rsub;
         float v[8];
-        unpack_row8<DT>(raw[i], v);
+        unpack8<DT>(raw[i], v);
         float rcp;
         bool bad, near;
         QStats st;
@@ -438,7 +423,7 @@ __device__ __forceinline__ void quantize_stats_rows(const QuantArgs& qa, int blk
 #pragma unroll
       for (int u = 0; u < 4; ++u) {
         float v[8];
-        unpack_row8<DT>(raw[u], v);
+        unpack8<DT>(raw[u], v);
         if (first) mx = mn = v[0];
         first = false;
 #pragma unroll
@@ -665,7 +650,8 @@ extern "C" int w4_quantize(const void* w, int w_dtype, int64_t N, int64_t K, int
   if (N == 0) return W4_OK;
   if (!w || !qweight || !scales || !zeros) return fail(W4_ERR_INVALID, "w4_quantize: null pointer");
   // (the tiles of the kernel that runs, and the rows of its statistics pass)
-  if (((N + 63) / 64) * (K / (G > 512 ? w4::QPACK : G)) >= (int64_t)1 << 31 || (G > 512 && N * (K / G) >= (int64_t)1 << 31))
+  if (((N + 63) / 64) * (K / (G > 512 ? w4::QPACK : G)) >= (int64_t)1 << 31 ||
+      (G > 512 && N * (K / G) >= (int64_t)1 << 31))
     return fail(W4_ERR_UNSUPPORTED, "w4_quantize: %lld x %lld weight has too many tiles", (long long)N,
                 (long long)K);
   const uint16_t* wp = static_cast<const uint16_t*>(w);
