@@ -146,3 +146,12 @@ def test_norm_and_activation_kernels_leave_launches_hip_refuses(monkeypatch):
     assert not llama_ops.rms_norm_ok(meta(1 << 12, 1 << 12, 8), meta(8), meta(1 << 12, 1 << 12, 8))
     for n, ok in (((1 << 24) - 1, True), (1 << 24, False)):
         assert llama_ops.silu_mul_ok(meta(n, 2048), meta(n, 2048)) == ok
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_norm_and_mlp_can_be_traced_symbolically(dtype):
+    """The host rules decide on what a symbolic tracer's stand-in cannot answer for: they
+    leave it to torch's operations first."""
+    m, x = _model().to(dtype), torch.randn(3, 64).to(dtype)
+    for mod in (m.model.norm, m.model.layers[0].mlp):
+        assert torch.equal(torch.fx.symbolic_trace(mod)(x), mod(x))
