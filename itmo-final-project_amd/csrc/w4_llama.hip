@@ -81,10 +81,17 @@ __device__ __forceinline__ float wave_sum(float v) {
 // The chunk that holds the position writes the new key and value to the cache
 // and uses them from LDS.  A decode step of the 1B model (16 layers, position
 // 575, fp16): 1559 us with the torch operations, 848 us with the first form of
-// this kernel alone.  There a layer's launch takes 6.4 us; 8.7 us with the keys
+// this kernel alone.  There a layer's launch takes 6.2 us; 8.7 us with the keys
 // loaded after the position and the query, the outputs to join after their
 // weights, a branch per element for the new key and value, and reductions by
 // LDS shuffles.
+//
+// What that costs on long caches: a workgroup past the position has loaded its
+// first block for nothing (32 / 8 heads of 64, position 100: 5.6 us in a cache of
+// 648, 6.3 in one of 4096), and the chunks follow the cache, so that a position of
+// 1500 is 24 chunks in a cache of 4096 (8.9 us), three in one of 32768 (16.7) and
+// one, block after block, in one of 131072 (37; a layer with torch's operations
+// took 470 us there, with this kernel 94).
 template <int DT, int D, int GP>
 __global__ __launch_bounds__(kAttnThreads) void attn_decode_kernel(AttnDecodeArgs a) {
   constexpr int DW = D / kAttnWaves;   // head elements per wave (keys)
@@ -303,7 +310,9 @@ __global__ __launch_bounds__(kAttnThreads) void attn_decode_kernel(AttnDecodeArg
   if (arrived != (unsigned)(active - 1)) return;
   if (tid == 0) __hip_atomic_store(a.cnt + slice, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   const float* const all = a.part + slice * a.chunks * stride;
-  // the first chunks' outputs travel with the maxima and sums
+  // The first chunks' outputs travel with the maxima and sums.  Twelve: ten chunks
+  // (cache 648) 6.19 us a launch, 6.45 with four ahead, 6.51 with eight, 6.29 with
+  // sixteen; two chunks 5.56, 5.46 with four.
   constexpr int AHEAD = 12;
   auto part_at = [&](int cc, int i) {
     return __hip_atomic_load(all + min(cc, active - 1) * stride + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -428,9 +437,12 @@ __global__ __launch_bounds__(256) void rope_cache_kernel(AttnPrefillArgs a) {
 // by V rows 16j + 4r + c.  What bounds it: the matrix cores' fp32 rate (157
 // TFLOP/s) and the latency that stays visible: half of a block's values travel
 // under its softmax, the rest and half of the next block's keys under its second
-// product (all of it would not fit the registers of two waves per SIMD).  Four layers of the 1B model and its head on 500 tokens: 1764 us
-// with torch's batched fp32 products, masks and copies; this kernel takes 21 us
-// of a layer there (29 us with each load next to its use).
+// product (all of it would not fit the registers of two waves per SIMD).  Four
+// layers of the 1B model and its head on 500 tokens: 1764 us with torch's batched
+// fp32 products, masks and copies; this kernel takes 21.7 us of a layer there (29 us
+// with each load next to its use) and the cache kernel 5.1.  Head size 128 takes all
+// 512 registers, one wave per SIMD, without scratch (an attention module of 16 / 4
+// heads on 500 tokens 75 us, 194 with torch's operations; 4096 tokens 786 and 3079).
 template <int DT, int D>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D == 64 ? 2 : 1))) void attn_prefill_kernel(
     AttnPrefillArgs a) {
@@ -1075,8 +1087,11 @@ template <int DT>
 void launch_norm_head(const w4::NormHeadArgs& a, hipStream_t st) {
   const int nc = (a.K + 511) / 512, rows = 4 * w4::head_rows(nc);
   // Eight workgroups per CU, each going through its rows; four above 2048 values,
-  // where each pays more for the norm (32000 x 3072, fp16: 31.8 against 33.7 us;
-  // 128256 x 2048: 82 against 80).
+  // where each pays more for the norm: up to about 32000 rows they are faster
+  // (16000 x 4096 22.6 against 26.1 us, 12000 x 2560 12.5 against 13.2), above that
+  // slower or equal (50257 x 2560 42.1 against 39.0, 128256 x 3072 117.7 against
+  // 114.4).  At 2048 values the line is less clear (fp16, eight against four:
+  // 16000 rows 14.5 and 12.7, 128256 rows 80.2 and 82.1).
   const int64_t wgs = ((int64_t)a.N + rows - 1) / rows;
   const int64_t most = nc <= 4 ? 2048 : 1024;
   const dim3 grid((unsigned)(wgs < most ? wgs : most)), block(256);

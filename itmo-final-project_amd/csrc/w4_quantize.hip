@@ -1,9 +1,11 @@
 // Group-wise asymmetric RTN int4 quantize/pack and the exact dequantize, for
 // gfx950.  Semantics follow the reference's torch implementation
 // (int4_triton/quantize.py:102-135) bit for bit; the kernel structure is this
-// library's own: one wave per (group, 64-column strip), min/max by wave
-// shuffles, nibble packing in registers and an LDS transpose so that every
-// qweight row segment is written as one coalesced 256-byte store.
+// library's own: up to eight waves per (group, 64-column) tile, a lane per packed
+// word, extremes by DPP steps across the lanes of a group, packing through the
+// reciprocal with the rare doubtful words redone exactly, and an LDS transpose so
+// that every qweight row segment is written as one coalesced 256-byte store.
+// Groups above 512 take a statistics pass and a packing pass.
 #include <hip/hip_runtime.h>
 
 #include <climits>
@@ -186,11 +188,10 @@ constexpr int quantize_waves_per_tile(int G) { return G / 8 < QSWAVES ? G / 8 : 
 
 // Single-pass kernel for G <= 512: lanes_per_row = G/8 lanes each own one
 // packed word of a row; 64/lanes_per_row rows are processed per iteration.
-// Bound by HBM (154 MB for the block of 1B-model weights at G = 128: 34.5 us =
-// 4.5 TB/s, a large copy reaches 5.1; 37.5 us before the statistics lost their
-// branches, the packing its per-element boundary tests, and the tiles' order
-// went along K, so that the workgroups running at one time read whole rows
-// instead of one column of every row: 35.5 us in the old order).
+// Bound by HBM (154 MB for the block of 1B-model weights at G = 128: 33.0 us =
+// 4.7 TB/s, a large copy reaches 5.2; 37.5 us before the statistics lost their
+// branches, the packing its per-element boundary tests and the tiles their order
+// along N).
 // One weight of a quantize launch (w4_quantize_grouped puts several in one).
 struct QuantArgs {
   const uint16_t* w;
@@ -384,7 +385,7 @@ __global__ __launch_bounds__(QSWAVES * 64) void quantize_small_group_grouped_ker
 // second read comes mostly from the Infinity Cache.  The one-kernel form they
 // replace (a wave looping over 64 rows, twice) had N / 64 x K / G waves, 32 for
 // a per-channel 2048 x 8192 weight: the block's seven weights per channel took
-// 3122 us, these 51 us.
+// 2703 us, these 57 us.
 constexpr int QPACK = 128;  // k per tile of the packing pass
 
 // Statistics: `wpr` waves (a power of two, chosen so that few rows still spread

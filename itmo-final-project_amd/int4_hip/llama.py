@@ -21,9 +21,14 @@ Attention is computed in fp32 from contiguous operands: the KV cache is fp32
 and keeps K transposed ([kv_heads, head_dim, positions]), so no bf16 batched
 product with a transposed operand is issued.
 
-With Int4Linear projections, q/k/v (into one buffer when decoding) and
-gate/up each go through one grouped W4A16 call (``w4a16_matmul_grouped``), so
-a layer makes 4 W4A16 launches instead of 7.
+With Int4Linear projections, q/k/v and gate/up each go through one grouped W4A16
+call (``w4a16_matmul_grouped``), so a layer makes 4 W4A16 launches instead of 7.
+On the GPU, in bf16 and fp16, the operations between them are fused kernels
+(``llama_ops``): a decode step of a layer of plain modules is five launches, the
+norms and the gated activation computed inside the linears that read them; a
+prompt's layer is eight.  What those kernels do not take (hooks, replaced modules,
+autograd, tracing, other dtypes or shapes) runs as torch operations, which define
+the results.
 """
 from __future__ import annotations
 
