@@ -88,7 +88,8 @@ def build_ext() -> Path | None:
     # the slow path of every other thread-local access: torch.empty on the GPU took
     # 1.69 us instead of 1.37, every torch call of the process in proportion.
     cmd = [gxx, "-O2", "-DNDEBUG", "-std=c++17", "-fPIC", "-shared", "-D__HIP_PLATFORM_AMD__=1",
-           "-DUSE_ROCM=1", f'-DW4_TORCH_VERSION="{torch.__version__}"', f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+           "-DUSE_ROCM=1", f'-DW4_TORCH_VERSION="{torch.__version__}"',
+           f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
            "-I", str(root / "include"), "-I", str(root / "include" / "torch" / "csrc" / "api" / "include"),
            "-I", str(Path(os.environ.get("ROCM_PATH", "/opt/rocm")) / "include"),
            "-I", sysconfig.get_paths()["include"], "-I", str(ROOT / "include"), str(EXT_SRC), "-o", str(tmp),
