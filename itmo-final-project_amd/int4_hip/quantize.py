@@ -151,8 +151,9 @@ def quantize_int4_ref(w: torch.Tensor, group_size: int = 128):
     Counterpart of int4_triton/quantize.py:102-117.  The extremes are taken
     with ``amax``/``amin`` (a NaN anywhere in a group makes its scale, zero
     and codes follow IEEE NaN arithmetic), the code of every weight is found
-    in fp32 and the eight codes of a word are OR-ed into place, so a code
-    >= 8 in nibble 7 sets the int32 sign bit.
+    in fp32 and the eight codes of a word are added in place as int32, so a code
+    >= 8 in nibble 7 sets the sign bit and an INT32_MIN code in nibble 0 (a NaN)
+    wraps with it.
     """
     N, K = w.shape
     G = _resolve_group(K, group_size)
@@ -176,7 +177,7 @@ def quantize_int4_ref(w: torch.Tensor, group_size: int = 128):
     codes = codes.to(torch.int32).reshape(N, K // 8, 8)
     words = codes[..., 0].clone()
     for i in range(1, 8):
-        words.bitwise_or_(codes[..., i] << _NIBBLE_SHIFTS[i])
+        words.add_(codes[..., i] << _NIBBLE_SHIFTS[i])
     return (words.transpose(0, 1).contiguous(), step.transpose(0, 1).contiguous(),
             zp.to(torch.float16).transpose(0, 1).contiguous())
 

@@ -108,3 +108,14 @@ def test_quantize_name_is_callable_and_a_module():
     assert int4_hip.quantize.unpack_int4_ref is int4_hip.unpack_int4_ref
     with pytest.raises(AssertionError):  # same checks as quantize_int4 (CPU tensor)
         int4_hip.quantize(torch.zeros(8, 64, dtype=torch.bfloat16), 32)
+
+
+@pytest.mark.parametrize("last", [0, 1, 2])
+def test_nan_code_beside_a_large_last_code(last):
+    """A scale that fp16 rounds to 0 makes a zero weight's code NaN (INT32_MIN in the word, which
+    only nibble 0 keeps); the word's sum wraps past a code >= 8 in nibble 7."""
+    from oracle import w4a16_oracle as O
+    tiny = 2.0 ** -24
+    w = torch.tensor([[0, 1, 1, -1, 0, 0, 2, last]], dtype=torch.float32).mul(tiny).half()
+    got, want = Q.quantize_int4_ref(w, 8), O.quantize_int4(_bits16(w), "fp16", 8)
+    assert want[1][0, 0] == 0 and np.array_equal(got[0].numpy(), want[0])
